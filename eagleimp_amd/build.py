@@ -52,17 +52,20 @@ HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-Wextra", "-ffp-contract=o
 
 
 def build_engine():
+    from concurrent.futures import ThreadPoolExecutor
     hip = _hipcc()
-    objs = []
-    for src in ("eimp_kernels.hip", "eimp_engine.cpp"):
+    cmds, objs = [], []
+    for src in ("eimp_pbwt.hip", "eimp_kernels.hip", "eimp_engine.cpp", "eimp_phase.cpp",
+                "eimp_qref.cpp"):
         obj = os.path.join(CSRC, "_" + os.path.splitext(src)[0] + ".o")
-        _run([hip, f"--offload-arch={ARCH}", *HIP_FLAGS, "-x", "hip", "-c",
-              os.path.join(CSRC, src), "-o", obj])
+        if src in ("eimp_phase.cpp", "eimp_qref.cpp"):
+            cc = ["g++", *HOST_FLAGS]
+        else:
+            cc = [hip, f"--offload-arch={ARCH}", *HIP_FLAGS, "-x", "hip"]
+        cmds.append([*cc, "-c", os.path.join(CSRC, src), "-o", obj])
         objs.append(obj)
-    for src in ("eimp_phase.cpp", "eimp_qref.cpp"):
-        obj = os.path.join(CSRC, "_" + os.path.splitext(src)[0] + ".o")
-        _run(["g++", *HOST_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj])
-        objs.append(obj)
+    with ThreadPoolExecutor(len(cmds)) as pool:  # one compiler per source
+        list(pool.map(_run, cmds))
     tmp = LIB + ".tmp"
     _run([hip, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-pthread", "-o", tmp, *objs])
     os.replace(tmp, LIB)

@@ -18,56 +18,8 @@
 #include <vector>
 
 #include "../../include/eimp.h"
-#include "eimp_internal.h"
+#include "eimp_launch.h"
 
-namespace eimp {
-hipError_t launch_site_to_hap(const PanelDev &P, uint64_t *hap, hipStream_t s);
-hipError_t launch_panel_mono(const PanelDev &P, uint64_t *pand, uint64_t *por, hipStream_t s);
-hipError_t launch_distance(const PanelDev &P, const TgtDev *tg, const uint32_t *tlist,
-                           uint32_t nsel, hipStream_t s);
-hipError_t launch_select(const PanelDev &P, const TgtDev *tg, uint32_t n, hipStream_t s);
-hipError_t launch_monos(const PanelDev &P, const TgtDev *tg, const uint32_t *tlist, uint32_t n,
-                        uint32_t max_ww, hipStream_t s);
-hipError_t launch_splits(const PanelDev &P, const TgtDev *tg, uint32_t n, hipStream_t s);
-hipError_t launch_bits_to_list(const TgtDev *tg, uint32_t n, uint32_t nbits_bh, int which,
-                               hipStream_t s);
-hipError_t launch_cref(const PanelDev &P, const TgtDev *tg, const CrefItem *items, uint32_t nitems,
-                       uint32_t maxK, bool ident, hipStream_t s);
-uint32_t cref_max_k();
-hipError_t launch_digest_count0(const TgtDev *tg, uint32_t n, hipStream_t s);
-hipError_t launch_cref_rows(const TgtDev *tg, uint32_t t, uint32_t Mp, uint64_t *rows, uint32_t rw,
-                            hipStream_t s);
-hipError_t launch_digest_rows(const TgtDev *tg, const uint32_t *d_n, uint32_t nmax, uint64_t *dig,
-                              hipStream_t s);
-size_t pbwt_big_lds_bytes(uint32_t K);
-uint32_t pbwt_big_max_k();
-hipError_t launch_pbwt_big(const BigItem *items, uint32_t nitems, uint32_t maxK, hipStream_t s);
-int pbwt_variant_count();
-int pbwt_variant_threads(int v);
-int pbwt_variant_cpw(int v);
-uint32_t pbwt_variant_maxk(int v);
-size_t pbwt_lds_bytes(int v, uint32_t Kpad);
-hipError_t pbwt_prepare(int v, size_t lds);
-hipError_t launch_pbwt(int v, const TgtDev *tg, const PbwtItem *items, uint32_t nitems, size_t lds,
-                       hipStream_t s);
-hipError_t launch_prep_dev(int cls, const PanelDev &P, const TgtDev *tg, const uint32_t *d_n,
-                           uint32_t nmax, uint32_t max_ww, hipStream_t s);
-hipError_t launch_plan(TgtDev *tg, BatchDev *B, const PlanArgs &A, hipStream_t s);
-hipError_t launch_digest_count0_dev(const TgtDev *tg, const uint32_t *d_n, uint32_t nmax,
-                                    hipStream_t s);
-size_t cref_lds_bytes(const PanelDev &P, uint32_t maxK);
-hipError_t cref_persist_prepare(const PanelDev &P, uint32_t maxK, int *occ);
-bool cref_ident_ok(const PanelDev &P);
-hipError_t launch_panel_pbwt(const PanelDev &P, uint64_t m0, uint32_t nsites, uint16_t *blocks,
-                             uint32_t *rows, int32_t *c0out, int32_t *absperm, hipStream_t s);
-uint32_t panel_pbwt_max_k();
-hipError_t launch_cref_persist(const PanelDev &P, const TgtDev *tg, BatchDev *B,
-                               const uint32_t *blockpref, const uint32_t *blockpref_id,
-                               uint32_t maxK, const uint32_t *grid, hipStream_t s);
-hipError_t pbwt_persist_prepare(int v, size_t lds, int *occ);
-hipError_t launch_pbwt_persist(int v, const TgtDev *tg, BatchDev *B, const PbwtItem *items,
-                               uint32_t grid, size_t lds, hipStream_t s);
-}  // namespace eimp
 
 using namespace eimp;
 
@@ -77,9 +29,13 @@ using namespace eimp;
 // code the name is only a stand-in: the device address of the current
 // device's copy comes from hipGetSymbolAddress (scratch_for_device) and only
 // that address is passed to kernels and copies.
+// kScratchBytes is what a batch's buffers may take; the PBWT's own tables come
+// from the extra part behind it: 26 bytes per block and direction, and a block
+// has at least 128 bytes of condensed reference in the first part.
 static constexpr size_t kScratchBytes = 64ull << 20;
+static constexpr size_t kScratchExtra = 28ull << 20;
 static constexpr size_t kNoAllocMaxTargets = 256;
-static __device__ __align__(256) uint64_t scratch[kScratchBytes / 8];
+static __device__ __align__(256) uint64_t scratch[(kScratchBytes + kScratchExtra) / 8];
 
 namespace {
 
@@ -108,6 +64,15 @@ inline uint32_t batch_layout(uint32_t flags) {
     return (flags & EIMP_BATCH_COMPACT) ? LAYOUT_COMPACT
          : (flags & EIMP_BATCH_RAW)     ? LAYOUT_RAW
                                         : LAYOUT_GPU;
+}
+// The chain shape for a largest Kpad: the smallest that holds it (the shapes are
+// in order); -1 when none does.
+int auto_pbwt_variant(uint32_t Kpad) {
+    int best = -1;
+    for (int v = 0; v < pbwt_variant_count(); v++)
+        if (pbwt_variant_maxk(v) >= Kpad && (best < 0 || pbwt_variant_maxk(v) < pbwt_variant_maxk(best)))
+            best = v;
+    return best;
 }
 inline uint64_t round_up(uint64_t n, uint64_t m) { return (n + m - 1) / m * m; }
 
@@ -185,8 +150,8 @@ struct eimp_engine {
     // batch pools
     DevBuf d_tg, d_gt, d_nerr, d_bh, d_bhflags, d_mono, d_splitsites, d_splits, d_cMdiffs,
         d_stats, d_cref, d_count0, d_out, d_digest, d_tlist, d_citems, d_pitems, d_tmp,
-        d_crows, d_ord, d_big;  // large-K PBWT: row-major cref, orders, items
-    DevBuf p_blocks, p_rows, p_c0, p_abs;  // panel PBWT
+        d_hdr, d_rowpref, d_rowlist, d_crows, d_ord, d_big;  // PBWT tables; large-K PBWT: row-major cref, orders, items
+    DevBuf p_blocks, p_rows, p_c0, p_abs, p_tg, p_items, p_list, p_hdr, p_starts;  // panel PBWT
     HostBuf h_stage;
     std::vector<TgtDev> h_tg;
     std::vector<uint32_t> h_stats;
@@ -204,6 +169,7 @@ struct eimp_engine {
     uint64_t panel_gen = 0;  // bumped whenever panel buffers change (stream contexts check it)
     int pbwt_prepared_variant = -1;
     size_t pbwt_prepared_lds = 0;
+    uint32_t ncu = 0;  // compute units
 
     hipEvent_t get_event() {
         if (!event_pool.empty()) {
@@ -247,8 +213,9 @@ struct eimp_engine {
     void release_pools() {
         DevBuf *bufs[] = {&d_tg, &d_gt, &d_nerr, &d_bh, &d_bhflags, &d_mono, &d_splitsites,
                           &d_splits, &d_cMdiffs, &d_stats, &d_cref, &d_count0, &d_out,
-                          &d_digest, &d_tlist, &d_citems, &d_pitems, &d_tmp, &d_crows, &d_ord, &d_big,
-                          &p_blocks, &p_rows, &p_c0, &p_abs};
+                          &d_digest, &d_tlist, &d_citems, &d_pitems, &d_tmp, &d_hdr, &d_rowpref, &d_rowlist, &d_crows,
+                          &d_ord, &d_big,
+                          &p_blocks, &p_rows, &p_c0, &p_abs, &p_tg, &p_items, &p_list, &p_hdr, &p_starts};
         for (auto *b : bufs) b->release();
         h_stage.release();
     }
@@ -269,19 +236,7 @@ struct eimp_engine {
                 return fail(EIMP_ERR_UNSUPPORTED, "PBWT variant too small for K");
             return pbwt_variant;
         }
-        // fewest chunks per wave among workgroups of up to 512 threads (measured
-        // best on MI355X at K = 10,000), 1024-thread workgroups only when needed
-        int best = -1;
-        for (int pass = 0; pass < 2 && best < 0; pass++) {
-            for (int v = 0; v < pbwt_variant_count(); v++) {
-                if (pbwt_variant_maxk(v) < Kmax_pad) continue;
-                if (pass == 0 && pbwt_variant_threads(v) > 512) continue;
-                if (best < 0 || pbwt_variant_cpw(v) < pbwt_variant_cpw(best) ||
-                    (pbwt_variant_cpw(v) == pbwt_variant_cpw(best) &&
-                     pbwt_variant_threads(v) < pbwt_variant_threads(best)))
-                    best = v;
-            }
-        }
+        const int best = auto_pbwt_variant(Kmax_pad);
         if (best < 0) return fail(EIMP_ERR_UNSUPPORTED, "K beyond the PBWT kernels' LDS capacity");
         return best;
     }
@@ -326,7 +281,8 @@ int ensure_pmono(eimp_engine *e) {
 // (eimp_engine_run_batch_noalloc).
 enum MemSlot : int {
     MS_TG, MS_NERR, MS_BH, MS_BHF, MS_MONO, MS_SS, MS_SPL, MS_CMD, MS_STATS, MS_TLIST,
-    MS_CREF, MS_DIG, MS_CITEMS, MS_PITEMS, MS_CROWS, MS_ORD, MS_BIG
+    MS_CREF, MS_DIG, MS_CITEMS, MS_PITEMS, MS_CROWS, MS_ORD, MS_BIG,
+    MS_HDR, MS_RPREF, MS_RLIST  // tables of the PBWT
 };
 struct BatchMem {
     virtual ~BatchMem() = default;
@@ -356,6 +312,9 @@ struct PoolMem final : BatchMem {
         case MS_CREF: return e->d_cref;
         case MS_DIG: return e->d_digest;
         case MS_CITEMS: return e->d_citems;
+        case MS_HDR: return e->d_hdr;
+        case MS_RPREF: return e->d_rowpref;
+        case MS_RLIST: return e->d_rowlist;
         case MS_CROWS: return e->d_crows;
         case MS_ORD: return e->d_ord;
         case MS_BIG: return e->d_big;
@@ -391,14 +350,21 @@ struct PoolMem final : BatchMem {
 // are the caller's (rows[t]: 2*Mp*RS uint32, count0[t]: Mp int32, Mp <= max_Mp).
 struct ScratchMem final : BatchMem {
     char *base;
-    size_t used = 0;
+    size_t used = 0, used_extra = 0;
     uint32_t *const *rows;
     int32_t *const *c0;
     size_t max_Mp;
     ScratchMem(uint64_t *scr, uint32_t *const *rows_, int32_t *const *c0_, size_t max_Mp_)
         : base(reinterpret_cast<char *>(scr)), rows(rows_), c0(c0_), max_Mp(max_Mp_) {}
-    int get(MemSlot, size_t bytes, const char *what, void **p) override {
+    int get(MemSlot s, size_t bytes, const char *what, void **p) override {
         const size_t b = round_up(std::max<size_t>(bytes, 1), 256);
+        if (s >= MS_HDR) {
+            if (used_extra + b > kScratchExtra)
+                return fail(EIMP_ERR_UNSUPPORTED, std::string("no-allocation scratch full (at ") + what + ")");
+            *p = base + kScratchBytes + used_extra;
+            used_extra += b;
+            return EIMP_OK;
+        }
         if (used + b > kScratchBytes)
             return fail(EIMP_ERR_UNSUPPORTED, std::string("batch needs more than the ") +
                                                   std::to_string(kScratchBytes >> 20) +
@@ -446,7 +412,10 @@ int scratch_for_device(int dev, uint64_t **out) {
 int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem &mem) {
     std::vector<TgtDev> &tg = e->h_tg;
     uint64_t cref_bytes = 0, crows_bytes = 0, ord_bytes = 0;
-    std::vector<uint64_t> cref_off(n), crows_off(n, 0), ord_off(n, 0);
+    std::vector<uint64_t> cref_off(n), crows_off(n, 0), ord_off(n, 0), hdr_off(n, 0);
+    // list counters (zero), then PBWT blocks before target t
+    std::vector<uint32_t> rowpref(kRowsCounters + n + 1, 0);
+    uint64_t hdr_elems = 0;
     uint32_t Kmax_pad = 0, Kmax = 0, Kbig = 0;
     std::vector<CrefItem> citems, citems_id;  // general / identity targets
     std::vector<PbwtItem> pitems;
@@ -485,7 +454,11 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
             Kmax_pad = std::max(Kmax_pad, T.Kpad);
             pitems.push_back(PbwtItem{t, 0});
             pitems.push_back(PbwtItem{t, 1});
+            hdr_off[t] = hdr_elems;
+            hdr_elems += 2 * nblk;
         }
+        rowpref[kRowsCounters + t + 1] =
+            rowpref[kRowsCounters + t] + (T.Kpad > lds_cap ? 0u : pbwt_blocks(T.Mp));
     }
     // the subset cref kernel reads the haplotype-major panel (the drop-in's
     // initialize uploads only the site-major one: transposed here, once)
@@ -505,7 +478,7 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
         if (lds > 160 * 1024)
             return fail(EIMP_ERR_UNSUPPORTED, "K beyond the PBWT kernel's slots or 160 KiB of LDS");
         if (e->pbwt_prepared_variant != v || e->pbwt_prepared_lds < lds) {
-            HIPCHK(pbwt_prepare(v, lds));
+            HIPCHK(pbwt_prepare(v, lds, nullptr));
             e->pbwt_prepared_variant = v;
             e->pbwt_prepared_lds = lds;
         }
@@ -517,13 +490,17 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
         return tg[a.t].Mp > tg[b.t].Mp;
     });
     void *p_cref = nullptr, *p_dig = nullptr, *p_ci = nullptr, *p_pi = nullptr, *p_tg = nullptr;
-    void *p_crows = nullptr, *p_ord = nullptr, *p_big = nullptr;
+    void *p_crows = nullptr, *p_ord = nullptr, *p_big = nullptr, *p_hdr = nullptr, *p_rp = nullptr,
+         *p_rl = nullptr;
     CHK(mem.get(MS_CREF, cref_bytes, "cref", &p_cref));
     CHK(mem.get(MS_DIG, (size_t)n * 16, "digest", &p_dig));
     const size_t nci = citems.size();
     citems.insert(citems.end(), citems_id.begin(), citems_id.end());
     CHK(mem.get(MS_CITEMS, std::max<size_t>(citems.size(), 1) * sizeof(CrefItem), "cref items", &p_ci));
     CHK(mem.get(MS_PITEMS, std::max<size_t>(pitems.size(), 1) * sizeof(PbwtItem), "pbwt items", &p_pi));
+    CHK(mem.get(MS_HDR, hdr_elems * 2, "block headers", &p_hdr));
+    CHK(mem.get(MS_RPREF, rowpref.size() * 4, "row prefix", &p_rp));
+    CHK(mem.get(MS_RLIST, 2ull * rowpref.back() * sizeof(RowItem), "row items", &p_rl));
     if (!big.empty()) {
         CHK(mem.get(MS_CROWS, crows_bytes, "large-K cref rows", &p_crows));
         CHK(mem.get(MS_ORD, ord_bytes, "large-K orders", &p_ord));
@@ -538,6 +515,7 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
     for (uint32_t t = 0; t < n; t++) {
         TgtDev &T = tg[t];
         T.cref = reinterpret_cast<uint16_t *>(static_cast<char *>(p_cref) + cref_off[t]);
+        T.hdr = static_cast<uint16_t *>(p_hdr) + hdr_off[t];
         T.digest = digest ? d_dig + 2 * t : nullptr;
     }
     std::vector<BigItem> bitems;
@@ -570,9 +548,11 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
     if (!citems.empty())
         HIPCHK(hipMemcpyAsync(d_ci, citems.data(), citems.size() * sizeof(CrefItem),
                               hipMemcpyHostToDevice, e->stream));
-    if (!pitems.empty())
+    if (!pitems.empty()) {
         HIPCHK(hipMemcpyAsync(d_pi, pitems.data(), pitems.size() * sizeof(PbwtItem),
                               hipMemcpyHostToDevice, e->stream));
+        HIPCHK(hipMemcpyAsync(p_rp, rowpref.data(), rowpref.size() * 4, hipMemcpyHostToDevice, e->stream));
+    }
     if (!bitems.empty())
         HIPCHK(hipMemcpyAsync(p_big, bitems.data(), bitems.size() * sizeof(BigItem),
                               hipMemcpyHostToDevice, e->stream));
@@ -587,8 +567,13 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
     }
     e->tend(ti);
     ti = e->tbegin(EIMP_KCLASS_PBWT);
-    if (!pitems.empty())
-        HIPCHK(launch_pbwt(v, d_tg, d_pi, (uint32_t)pitems.size(), lds, e->stream));
+    if (!pitems.empty()) {
+        HIPCHK(launch_order(v, d_tg, d_pi, (uint32_t)pitems.size(), nullptr, nullptr, nullptr, lds,
+                            e->stream));
+        uint32_t *rp = static_cast<uint32_t *>(p_rp);
+        HIPCHK(launch_rows(d_tg, nullptr, n, rp + kRowsCounters, static_cast<RowItem *>(p_rl), rp,
+                           Kmax_pad, rowpref.back(), e->ncu, e->stream));
+    }
     if (!bitems.empty())
         HIPCHK(launch_pbwt_big(static_cast<const BigItem *>(p_big), (uint32_t)bitems.size(), Kbig,
                                e->stream));
@@ -873,7 +858,7 @@ struct eimp_stream {
     double kms[EIMP_NKCLASS] = {};
     // device buffers; d_in = header (256 B) | TgtDev[nmax] | genotypes
     DevBuf d_in, d_nerr, d_bh, d_bhflags, d_mono, d_splitsites, d_splits, d_cMdiffs, d_stats,
-        d_digest, d_blockpref, d_pitems, d_tmp;
+        d_digest, d_blockpref, d_pitems, d_hdr, d_rowpref, d_rowlist, d_tmp;
     std::shared_ptr<StreamPool> pool;  // the output pool, maybe shared with other contexts
     uint64_t tab_off = 0, gt_off = 0, gt_cap_words = 0;
     HostBuf h_in, h_out;  // h_out = stats | digests | TgtDev table
@@ -929,6 +914,7 @@ int stream_launch_build(eimp_stream *s) {
     A.blockpref_id = s->d_blockpref.as<uint32_t>() + s->nmax + 1;
     A.ident_ok = cref_ident_ok(e->pd) ? 1u : 0u;
     A.pitems = s->d_pitems.as<PbwtItem>();
+    A.rowpref = s->d_rowpref.as<uint32_t>();
     A.layout = batch_layout(s->flags);
     A.digest = (s->flags & EIMP_BATCH_DIGEST) ? 1u : 0u;
     // timed contexts record an event before each kernel class (the planner
@@ -942,8 +928,12 @@ int stream_launch_build(eimp_stream *s) {
     HIPCHK(launch_cref_persist(e->pd, s->d_tg(), s->d_batch(), A.blockpref, A.blockpref_id, s->Kmax,
                                s->cref_grid, s->stream));
     CHK(mark(EIMP_KCLASS_PBWT));
-    HIPCHK(launch_pbwt_persist(s->pbwt_v, s->d_tg(), s->d_batch(), s->d_pitems.as<PbwtItem>(),
-                               s->pbwt_grid, s->pbwt_lds, s->stream));
+    const uint32_t Kpad = (uint32_t)round_up(s->Kmax, 64);
+    HIPCHK(launch_order(s->pbwt_v, s->d_tg(), s->d_pitems.as<PbwtItem>(), s->pbwt_grid,
+                        &s->d_batch()->npbwt, &s->d_batch()->pbwt_ctr, nullptr, s->pbwt_lds, s->stream));
+    HIPCHK(launch_rows(s->d_tg(), d_n, 0, A.rowpref + kRowsCounters, s->d_rowlist.as<RowItem>(),
+                       A.rowpref, Kpad, (uint64_t)s->nmax * pbwt_blocks(2 * s->Wmax + 1), e->ncu,
+                       s->stream));
     if (A.digest) HIPCHK(launch_digest_count0_dev(s->d_tg(), d_n, s->nmax, s->stream));
     CHK(mark(EIMP_KCLASS_COPY));
     return EIMP_OK;
@@ -972,7 +962,7 @@ void stream_release(eimp_stream *s) {
     if (s->build_done) (void)hipEventDestroy(s->build_done);
     DevBuf *bufs[] = {&s->d_in, &s->d_nerr, &s->d_bh, &s->d_bhflags, &s->d_mono, &s->d_splitsites,
                       &s->d_splits, &s->d_cMdiffs, &s->d_stats, &s->d_digest, &s->d_blockpref,
-                      &s->d_pitems, &s->d_tmp};
+                      &s->d_pitems, &s->d_hdr, &s->d_rowpref, &s->d_rowlist, &s->d_tmp};
     for (auto *b : bufs) b->release();
     s->h_in.release();
     s->h_out.release();
@@ -1030,6 +1020,11 @@ int stream_setup(eimp_stream *s, size_t pool_bytes, const std::shared_ptr<Stream
     CHK(s->d_digest.ensure(nmax * 16, "digests"));
     CHK(s->d_blockpref.ensure(2 * (nmax + 1) * 4, "block prefix"));
     CHK(s->d_pitems.ensure(2 * nmax * sizeof(PbwtItem), "pbwt items"));
+    // up to 2 W + 1 rows per direction: block headers of both directions
+    const uint64_t hdr_n = pbwt_blocks(2 * s->Wmax + 1);
+    CHK(s->d_hdr.ensure(nmax * hdr_n * 2, "block headers"));
+    CHK(s->d_rowpref.ensure((kRowsCounters + nmax + 1) * 4, "row prefix"));
+    CHK(s->d_rowlist.ensure(2 * nmax * hdr_n * sizeof(RowItem), "row items"));
     if (pool) {
         s->pool = pool;
     } else {
@@ -1050,10 +1045,10 @@ int stream_setup(eimp_stream *s, size_t pool_bytes, const std::shared_ptr<Stream
         return fail(EIMP_ERR_UNSUPPORTED, "K beyond the PBWT kernel's slots or 160 KiB of LDS");
     s->pbwt_v = v;
     s->pbwt_lds = lds;
-    int ncu = 0, occ_c[2] = {0, 0}, occ_p = 0;
-    HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, e->dev));
+    const int ncu = (int)e->ncu;
+    int occ_c[2] = {0, 0}, occ_p = 0;
     HIPCHK(cref_persist_prepare(e->pd, s->Kmax, occ_c));
-    HIPCHK(pbwt_persist_prepare(v, lds, &occ_p));
+    HIPCHK(pbwt_prepare(v, lds, &occ_p));
     s->cref_grid[0] = (uint32_t)(std::max(ncu, 1) * std::max(occ_c[0], 1));
     // identity targets need K == N_ad
     const bool ident_possible = cref_ident_ok(e->pd) && s->Kmax == e->Nad && e->Ncorr == e->Nad;
@@ -1072,6 +1067,7 @@ int stream_setup(eimp_stream *s, size_t pool_bytes, const std::shared_ptr<Stream
         T.splits = s->d_splits.as<uint64_t>() + t * Ww;
         T.cMdiffs = s->d_cMdiffs.as<float>() + t * round_up(s->Wmax + 1, 64);
         T.stats = s->d_stats.as<uint32_t>() + 4 * t;
+        T.hdr = s->d_hdr.as<uint16_t>() + t * hdr_n;
     }
     if (!(s->flags & (EIMP_STREAM_NO_GRAPH | EIMP_STREAM_TIMED))) {
         CHK(stream_capture(s, stream_launch_prep, &s->graph_prep, &s->exec_prep));
@@ -1155,6 +1151,9 @@ int eimp_engine_create(int device_index, eimp_engine **engine) {
         delete e;
         return fail(EIMP_ERR_HIP, "stream creation failed");
     }
+    int ncu = 0;
+    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device_index);
+    e->ncu = (uint32_t)std::max(ncu, 1);
     // this device's copy of the no-allocation scratch (device current)
     const int rc = scratch_for_device(device_index, &e->scratch);
     if (rc != EIMP_OK) {
@@ -1410,9 +1409,10 @@ int eimp_engine_ref_pbwt(eimp_engine *e, size_t m0, size_t nsites, uint32_t *row
         return fail(EIMP_ERR_INVALID, "site range outside the panel");
     if (nsites >= (1u << 31)) return fail(EIMP_ERR_UNSUPPORTED, "too many sites");
     const uint64_t N = e->Nad, Kpad = round_up(N, 64);
-    // panels up to one workgroup's LDS run the LDS-resident kernel; wider ones
+    // panels up to one workgroup's LDS run the LDS-resident kernels; wider ones
     // the large-K kernel (order in global memory)
-    const bool big = Kpad > panel_pbwt_max_k();
+    const int v = auto_pbwt_variant((uint32_t)Kpad);
+    const bool big = v < 0;
     if (big && (N > pbwt_big_max_k() || pbwt_big_lds_bytes((uint32_t)N) > 160 * 1024))
         return fail(EIMP_ERR_UNSUPPORTED, "panel wider than " + std::to_string(pbwt_big_max_k()) +
                                               " haplotypes");
@@ -1422,6 +1422,28 @@ int eimp_engine_ref_pbwt(eimp_engine *e, size_t m0, size_t nsites, uint32_t *row
     CHK(e->p_rows.ensure(nsites * RS * 4, "panel PBWT rows"));
     CHK(e->p_c0.ensure(nsites * 4, "panel PBWT count0"));
     if (absperm) CHK(e->p_abs.ensure((nsites + 1) * N * 4, "panel PBWT permutations"));
+    if (!big) {
+        // one forward chain over the site blocks: a target record, its chain
+        // item and the rows' work items (the forward half only)
+        CHK(e->p_tg.ensure(sizeof(TgtDev), "panel PBWT record"));
+        CHK(e->p_items.ensure(sizeof(PbwtItem) + (kRowsCounters + 2) * 4, "panel PBWT items"));
+        CHK(e->p_list.ensure(2 * nblk * sizeof(RowItem), "panel PBWT row items"));
+        CHK(e->p_hdr.ensure(nblk * 4, "panel PBWT block headers"));
+        if (absperm) CHK(e->p_starts.ensure(nblk * Kpad * 2, "panel PBWT block orders"));
+        TgtDev T{};
+        T.K = (uint32_t)N;
+        T.Kpad = (uint32_t)Kpad;
+        T.Mp = (uint32_t)nsites;
+        T.RS = (uint32_t)RS;
+        T.cref = e->p_blocks.as<uint16_t>();
+        T.out = e->p_rows.as<uint32_t>();
+        T.count0 = e->p_c0.as<int32_t>();
+        T.hdr = e->p_hdr.as<uint16_t>();
+        uint32_t items[2 + kRowsCounters + 2] = {};
+        items[2 + kRowsCounters + 1] = (uint32_t)nblk;
+        HIPCHK(hipMemcpyAsync(e->p_tg.p, &T, sizeof(T), hipMemcpyHostToDevice, e->stream));
+        HIPCHK(hipMemcpyAsync(e->p_items.p, items, sizeof(items), hipMemcpyHostToDevice, e->stream));
+    }
     if (big) {
         CHK(e->d_ord.ensure(2 * Kpad * 4, "panel PBWT orders"));
         CHK(e->d_big.ensure(sizeof(BigItem), "panel PBWT item"));
@@ -1442,9 +1464,21 @@ int eimp_engine_ref_pbwt(eimp_engine *e, size_t m0, size_t nsites, uint32_t *row
     if (a) (void)hipEventRecord(a, e->stream);
     if (big)
         HIPCHK(launch_pbwt_big(e->d_big.as<BigItem>(), 1, (uint32_t)N, e->stream));
-    else
-        HIPCHK(launch_panel_pbwt(e->pd, m0, (uint32_t)nsites, e->p_blocks.as<uint16_t>(), e->p_rows.as<uint32_t>(),
-                                 e->p_c0.as<int32_t>(), absperm ? e->p_abs.as<int32_t>() : nullptr, e->stream));
+    else {
+        const size_t lds = pbwt_lds_bytes(v, (uint32_t)Kpad);
+        HIPCHK(pbwt_prepare(v, lds, nullptr));
+        HIPCHK(launch_site_blocks(e->pd, m0, (uint32_t)nsites, e->p_blocks.as<uint16_t>(), e->stream));
+        uint16_t *starts = absperm ? e->p_starts.as<uint16_t>() : nullptr;
+        HIPCHK(launch_order(v, e->p_tg.as<TgtDev>(), e->p_items.as<PbwtItem>(), 1, nullptr, nullptr, starts,
+                            lds, e->stream));
+        uint32_t *rp = e->p_items.as<uint32_t>() + 2;
+        if (absperm)
+            HIPCHK(launch_dense(v, e->p_tg.as<TgtDev>(), (uint32_t)nblk, starts, e->p_abs.as<int32_t>(), lds,
+                                e->stream));
+        else
+            HIPCHK(launch_rows(e->p_tg.as<TgtDev>(), nullptr, 1, rp + kRowsCounters,
+                               e->p_list.as<RowItem>(), rp, (uint32_t)Kpad, nblk, e->ncu, e->stream));
+    }
     if (b) (void)hipEventRecord(b, e->stream);
     HIPCHK(hipStreamSynchronize(e->stream));
     if (device_ms) {

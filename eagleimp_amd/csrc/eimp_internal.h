@@ -65,6 +65,7 @@ struct TgtDev {
     uint16_t *cref;        // nblk x Kpad, transposed 16-row blocks
     int32_t *count0;       // Mp
     uint32_t *out;         // 2 x Mp x RS uint32 (forward rows, then backward rows)
+    uint16_t *hdr;         // 2 x nblk: runs listed in a block's rows (forward, then backward blocks)
     uint64_t *digest;      // [0] pbwt words, [1] count0
     uint32_t Mp;
     uint32_t Kpad;         // K rounded up to 64
@@ -98,6 +99,16 @@ struct CrefItem {
     uint32_t t, b0, b1, pad;
 };
 
+// 16-row blocks of a target's PBWT, both directions
+__host__ __device__ inline uint32_t pbwt_blocks(uint32_t Mp) { return 2 * ((Mp + 15) / 16); }
+
+// k_rows work item: block q of chain 2 t + direction, its runs; and the words
+// that count the lists of items
+struct RowItem {
+    uint32_t chain, q, runs;
+};
+constexpr uint32_t kRowsCounters = 4;
+
 // PBWT work item: target t, direction (0 fwd, 1 bck)
 struct PbwtItem {
     uint32_t t, dir;
@@ -126,6 +137,7 @@ struct PlanArgs {
     uint32_t *blockpref;     // nmax + 1 prefix sums of cref blocks (gather targets)
     uint32_t *blockpref_id;  // nmax + 1 prefix sums of cref blocks (identity targets)
     PbwtItem *pitems;        // 2 * nmax
+    uint32_t *rowpref;       // kRowsCounters, then nmax + 1 prefix sums of pbwt_blocks
     uint32_t layout;         // LAYOUT_*
     uint32_t digest;
     uint32_t ident_ok;       // identity targets take the transpose kernel

@@ -16,90 +16,13 @@
 //   k_bits_to_list   bitmap -> ascending index list (drop-in inputs)
 //   k_cref           condensed reference in 16-row transposed blocks
 //                    (Target::condensedReferenceT, src/Target.cpp:953-1059)
-//   k_pbwt           compressed forward / backward PBWT
-//                    (PBWT::buildComprPBWT, src/PBWT.cpp:207-285)
 #include <map>
 #include <mutex>
-#include <type_traits>
 
-#include "eimp_internal.h"
+#include "eimp_device.h"
+#include "eimp_launch.h"
 
 namespace eimp {
-
-// ---------------------------------------------------------------------------
-// wave helpers
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
-
-// Pointers read out of device structs are generic, so accesses through them
-// compile to FLAT instructions, which count in the LDS counter as well: the
-// next s_waitcnt for an LDS result then also waits for a FLAT store to be
-// acknowledged by memory.  Inside loops that mix LDS traffic with global
-// stores the pointers are cast to the global address space first.
-template <class T>
-using gptr_t = __attribute__((address_space(1))) T *;
-template <class T>
-__device__ __forceinline__ gptr_t<T> gmem(T *p) {
-    return (gptr_t<T>)p;
-}
-// Arrays that no kernel running at the same time writes, read at wave-uniform
-// addresses through the constant address space: scalar loads.
-template <class T>
-using cptr_t = const __attribute__((address_space(4))) T *;
-template <class T>
-__device__ __forceinline__ cptr_t<T> cmem(const T *p) {
-    return (cptr_t<T>)p;
-}
-// LDS (address space 3) pointers: 32-bit byte addresses
-template <class T>
-using lds_ptr_t = __attribute__((address_space(3))) T *;
-// compile-time loop: f(std::integral_constant<int, I>) for I in [B, E)
-template <int B, int E, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-    if constexpr (B < E) {
-        f(std::integral_constant<int, B>{});
-        static_for<B + 1, E>(f);
-    }
-}
-
-// clang vector types: assignable through global-address-space pointers
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ uint32_t mbcnt(uint64_t m) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
-__device__ __forceinline__ uint64_t lanemask_lt() {
-    uint32_t l = lane_id();
-    return l == 0 ? 0ull : (~0ull >> (64 - l));
-}
-
-__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
-__device__ __forceinline__ uint64_t wave_sum64(uint64_t v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
-__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor(v, o));
-    return v;
-}
-// inclusive scan over the wave
-__device__ __forceinline__ uint32_t wave_scan_incl(uint32_t v) {
-    uint32_t l = lane_id();
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        uint32_t u = __shfl_up(v, o);
-        if (l >= (uint32_t)o) v += u;
-    }
-    return v;
-}
 
 // bits [bitoff, bitoff+64) of a bit row with `words` readable words
 __device__ __forceinline__ uint64_t funnel(const uint64_t *__restrict__ row, uint64_t bitoff,
@@ -908,557 +831,6 @@ __global__ __launch_bounds__(CREF_NT) void k_cref_ident(PanelDev P, const TgtDev
     for (uint32_t b = it.b0; b < it.b1; b++) cref_block_ident<GPT>(P, tg[it.t], b, srow);
 }
 
-// ---------------------------------------------------------------------------
-// a9: compressed PBWT.  One workgroup per (target, direction).
-//
-// The K positions of the current order are cut into chunks of 64; wave w
-// holds chunks [w*NS, w*NS+NS) (NS slots, chosen per target so that all waves
-// are busy), one position per lane, as a 32-bit payload: hap index << 16 |
-// the 16 bits of the current cref block for that haplotype.  Positions
-// K..Kpad-1 (and whole padding chunks) carry all-ones row bits: under the
-// stable partition (zeros first) they never move, and they give the
-// 1-padding of the last word.  A step:
-//   pass 1  ballot of the row bit per slot: the slot's two data words go to
-//           output lane c; the wave's zero count (scalar) to LDS
-//   (barrier) zeros before the wave's first chunk and in the row (count0)
-//           from the NW wave counts, in scalar registers
-//   pass 2  per slot: the ones before the chunk are a scalar running sum, so
-//           mbcnt of the ballot plus that base gives a one's destination and
-//           a lane constant minus it a zero's; payloads scattered into LDS
-//           (two contiguous runs per chunk); output lanes store their data /
-//           cumulative-zero pairs
-//   (barrier)
-//   pass 3  read back the payloads of my positions.
-// A row whose K bits are all equal keeps the order: pass 2, the second
-// barrier and pass 3 are skipped (the wave counts alternate between two LDS
-// halves, so the next step's counts never overwrite ones still being read).
-// At each 16-row block boundary the next block's uint16 values are staged in
-// LDS and gathered by hap index.
-// ---------------------------------------------------------------------------
-// v_writelane_b32 through the LLVM intrinsic (no clang builtin in this
-// toolchain); the compiler sees it, so it inserts the wait states a VALU-written
-// SGPR operand needs.
-extern "C" __device__ uint32_t eimp_llvm_writelane(uint32_t val, uint32_t lane, uint32_t old)
-    __asm("llvm.amdgcn.writelane");
-
-// writes a wave-uniform value into lane L of a VGPR
-template <int L>
-__device__ __forceinline__ uint32_t writelane(uint32_t old, uint32_t val) {
-    return eimp_llvm_writelane(val, (uint32_t)L, old);
-}
-
-
-// Exclusive prefix sum of v over lanes 0..N-1 (other lanes: garbage), by DPP
-// row shifts and row broadcasts (no LDS).
-template <int N>
-__device__ __forceinline__ uint32_t lane_scan_excl(uint32_t v) {
-    uint32_t x = v;
-    // within rows of 16 lanes: lane i += lane i-1, i-2, i-4, i-8 (zero past the row start)
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, true);
-    if constexpr (N > 2) x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, true);
-    if constexpr (N > 4) x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, true);
-    if constexpr (N > 8) x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, true);
-    // across rows: lane 15 of each row into rows 1 and 3, then lane 31 into rows 2 and 3
-    if constexpr (N > 16) x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xA, 0xF, false);
-    if constexpr (N > 32) x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xC, 0xF, false);
-    return x - v;
-}
-
-// LDS bytes before the PBWT payloads: 32 (NS - 1) words, the largest amount a
-// slot's store address sits below its destination (pbwt_steps, pass 2).
-__host__ __device__ constexpr uint32_t pbwt_pay_bias(int ns) { return 128u * (uint32_t)(ns - 1); }
-
-// NS = slots per wave for this target.  Wave w owns chunks [w*NS, w*NS+NS);
-// chunks >= Kpad/64 are padding (all-ones bits, never moving), so every slot
-// is processed unconditionally.
-// ABS (panel PBWT for imputation): also writes the order after every step to
-// absperm (row step+1; row 0 = identity) and the step's count0 to c0out.
-// WS: how each wave sums the NW wave zero counts after the first barrier --
-// 0: NW LDS broadcasts read into scalars (short latency; best when the
-// workgroups sharing a CU are at different points, as with targets of mixed
-// K and windows), 1: one LDS read per lane and a DPP lane scan (fewer
-// instructions and scalar registers; best for uniform targets).  The
-// autotuner picks between the variants built with each.
-//
-// The kernels that call this use dynamic LDS only (the host checks that they
-// have no static LDS), so LDS byte addresses are plain offsets from 0: pay[]
-// starts at byte pbwt_pay_bias(NS), which keeps pass 2's store addresses
-// (before their immediate offsets) non-negative.
-template <int NT, int NS, bool ABS = false, int WS = 0>
-__device__ __forceinline__ void pbwt_steps(const TgtDev &T, const bool rev, uint32_t *smem,
-                                           int32_t *__restrict__ absperm = nullptr,
-                                           int32_t *__restrict__ c0out = nullptr) {
-    constexpr int NW = NT / 64;
-    constexpr uint32_t NPOS = NS * NW * 64;
-    static_assert(NS <= 64, "one output lane per slot");
-    const uint32_t K = T.K, Mp = T.Mp, Kpad = T.Kpad, RS = T.RS;
-    const uint32_t nch = Kpad / 64;
-    const uint32_t npairs = (K + 31) / 32;
-    const uint32_t KW = 2 * npairs;
-    // NPOS payloads at LDS bytes [PBIAS, PBIAS + 4*NPOS): the partition's
-    // stores address them as 4 sel + 128 c (pass 2), sel >= 0
-    constexpr uint32_t PBIAS = pbwt_pay_bias(NS);
-    uint32_t *pay = smem + PBIAS / 4;
-    // Kpad + 2 uint16: the next cref block by haplotype (and all ones at id
-    // Kpad), staged at block boundaries (when no payloads are in flight) from
-    // LDS byte 0
-    uint16_t *stage = (uint16_t *)smem;
-    // 2 x NW: zeros of each wave's chunks, by step parity (a step that moves
-    // nothing has no second barrier, so the next step writes the other half)
-    uint32_t *wzero2 = pay + NPOS;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = lane_id();
-    const uint32_t ch0 = wave * NS;                // first chunk of this wave
-    // pass 2's per-lane constant (bytes): 4 (64 ch0 + ln + 64 (NS - 1))
-    const uint32_t vbase4 = 4u * (ch0 * 64u + ln + 64u * (NS - 1));
-    const gptr_t<const uint16_t> cref = gmem((const uint16_t *)T.cref);
-    // wave-uniform flags as scalars: their branches stay scalar branches
-    const bool dig = __builtin_amdgcn_readfirstlane(T.digest != nullptr ? 1u : 0u) != 0;
-
-    uint32_t p[NS];
-    {
-        const uint32_t b0 = (rev ? Mp - 1 : 0) >> 4;
-#pragma unroll
-        for (int c = 0; c < NS; c++) {
-            const uint32_t pos = (ch0 + (uint32_t)c) * 64 + ln;
-            // the cref kernel writes all-ones for K <= k < Kpad; positions of
-            // padding chunks (>= Kpad) all carry id Kpad, whose staged value
-            // is all ones
-            const uint32_t v = pos < Kpad ? (uint32_t)cref[(uint64_t)b0 * Kpad + pos] : 0xFFFFu;
-            p[c] = ((pos < Kpad ? pos : Kpad) << 16) | v;
-        }
-    }
-    if constexpr (ABS) {
-        if (absperm) {
-#pragma unroll
-            for (int c = 0; c < NS; c++) {
-                const uint32_t pos = (ch0 + (uint32_t)c) * 64 + ln;
-                if (pos < K) absperm[pos] = (int32_t)pos;
-            }
-        }
-    }
-    const gptr_t<uint32_t> outbase = gmem(T.out) + (rev ? (uint64_t)Mp * RS : 0ull);
-    const uint64_t gbase = rev ? (uint64_t)Mp * KW : 0ull;
-    uint64_t dsum = 0;
-    const bool raw = (__builtin_amdgcn_readfirstlane(T.flags) & TF_RAW) != 0;
-    const uint32_t och = ch0 + ln;         // chunk stored by this lane
-    const bool ostore = ln < (uint32_t)NS && och < nch;
-    // the raw layout has one word pair per chunk, the others two
-    const bool second = !raw && 2 * och + 1 < npairs;
-    // digest of this lane's words: g = gbase + step*KW + 4*och (+0..3), key
-    // g * kDigKey, rotation -g (alignbit uses 5 bits)
-    const uint32_t g0 = (uint32_t)gbase + 4u * och;
-
-    {
-        // The padding words of every row of this direction, stored once: after
-        // the logical pairs (words >= 2*npairs) zero, or in the raw layout
-        // all ones after the data words (positions >= K are all ones).
-        const uint32_t pw0 = raw ? 2 * nch : 2 * npairs;  // even, as RS
-        const uint32_t fw = raw ? ~0u : 0u;
-        for (uint32_t rr = threadIdx.x; rr < Mp; rr += NT) {
-            const gptr_t<u32x2> prow = (gptr_t<u32x2>)(outbase + (uint64_t)rr * RS);
-            for (uint32_t w = pw0 / 2; w < RS / 2; w++) prow[w] = u32x2{fw, fw};
-        }
-    }
-    // this lane's byte offset of its chunk's words within a row (opaque
-    // 32-bit value added to the scalar row address: stores take the
-    // scalar-base form, no 64-bit vector address per step)
-    uint32_t obyte;
-    asm("" : "=v"(obyte) : "0"((raw ? 8u : 16u) * och));
-    const uint32_t rs_bytes = RS * 4u;
-    uint64_t rowaddr = (uint64_t)(size_t)outbase;
-    // row bit of the current row within its 16-row block: forward rows go up
-    // from bit 0, backward rows down from bit 15 (shifts as data, so the step
-    // has no direction branch)
-    uint32_t jbit = 1u << ((rev ? Mp - 1 : 0) & 15);
-    const uint32_t jl = rev ? 0u : 1u, jr = rev ? 1u : 0u;
-    // first step whose row begins a new 16-row block
-    uint32_t nextb = rev ? ((Mp - 1) & 15) + 1 : 16u;
-    // forward pass: count0 of the current 16-row block, lane (step & 15)
-    uint32_t c0acc = 0;
-    // PF: the next block boundary's cref block (Kpad uint16 = Kpad/2 words,
-    // at most NPF per thread since Kpad <= NS * NT) is loaded into registers
-    // one block ahead, so staging it waits for no global load.  Only the
-    // 1024-thread shapes (one workgroup per CU, 128 VGPRs a wave) have the
-    // registers; the others load at the boundary.
-    constexpr bool PF = NT >= 1024;
-    constexpr int NPF = PF ? (NS + 1) / 2 : 1;
-    uint32_t pf[NPF];
-    auto block_src = [&](uint32_t st) {
-        const uint32_t r = rev ? Mp - 1 - st : st;
-        return (gptr_t<const uint32_t>)(cref + (uint64_t)(r >> 4) * Kpad);
-    };
-    auto prefetch = [&](uint32_t st) {
-        const gptr_t<const uint32_t> src = block_src(st);
-#pragma unroll
-        for (int i = 0; i < NPF; i++) {
-            const uint32_t q = threadIdx.x + (uint32_t)i * NT;
-            pf[i] = q < Kpad / 2 ? src[q] : 0u;
-        }
-    };
-    if constexpr (PF) {
-        if (nextb < Mp) prefetch(nextb);
-    }
-    for (uint32_t step = 0; step < Mp; ++step) {
-        if (step == nextb) {
-            nextb += 16;
-            jbit = rev ? 0x8000u : 1u;
-            if (!rev && wave == 0 && ln < 16u) {  // the previous block's count0
-                if constexpr (ABS) gmem(c0out)[step - 16 + ln] = (int32_t)c0acc;
-                else gmem(T.count0)[step - 16 + ln] = (int32_t)c0acc;
-            }
-            uint32_t *st32 = (uint32_t *)stage;
-            __syncthreads();  // every wave has read back its payloads
-            if constexpr (PF) {
-#pragma unroll
-                for (int i = 0; i < NPF; i++) {
-                    const uint32_t q = threadIdx.x + (uint32_t)i * NT;
-                    if (q < Kpad / 2) st32[q] = pf[i];
-                }
-                if (nextb < Mp) prefetch(nextb);
-            } else {
-                const gptr_t<const uint32_t> src = block_src(step);
-                for (uint32_t q = threadIdx.x; q < Kpad / 2; q += NT) st32[q] = src[q];
-            }
-            if (threadIdx.x == 0) st32[Kpad / 2] = ~0u;  // id Kpad: the padding chunks
-            __syncthreads();
-#pragma unroll
-            for (int c = 0; c < NS; c++)
-                p[c] = (p[c] & 0xFFFF0000u) | (uint32_t)stage[p[c] >> 16];
-        }
-        // pass 1: slot c's ballot words go to lane c.  Lanes >= NS of
-        // olo/ohi are never read: no initial value (asm).
-        uint32_t olo, ohi;
-        asm volatile("" : "=v"(olo), "=v"(ohi));
-        uint64_t mk[NS];  // the ballots stay in scalar registers for pass 2
-        static_for<0, NS>([&](auto ci) {
-            constexpr int c = decltype(ci)::value;
-            const uint64_t m = __ballot((p[c] & jbit) != 0u);
-            mk[c] = m;
-            olo = writelane<c>(olo, (uint32_t)m);
-            ohi = writelane<c>(ohi, (uint32_t)(m >> 32));
-        });
-        // zeros of lane c's chunk, their exclusive scan over the wave's chunks
-        // (lanes >= NS: don't care) and the wave's total, written to LDS by
-        // every lane (one address, one value)
-        const uint32_t zl = 64u - (uint32_t)__popc(olo) - (uint32_t)__popc(ohi);
-        const uint32_t zex = lane_scan_excl<NS>(zl);
-        uint32_t *wzero = wzero2 + (step & 1u) * (uint32_t)NW;
-        wzero[wave] = (uint32_t)__builtin_amdgcn_readlane((int)(zex + zl), NS - 1);
-        __syncthreads();
-        // zeros before my first chunk, and in the whole row (count0)
-        uint32_t run = 0, cnt0 = 0;
-        if constexpr (WS == 0) {
-#pragma unroll
-            for (int w2 = 0; w2 < NW; w2++) {
-                const uint32_t v = __builtin_amdgcn_readfirstlane(wzero[w2]);
-                cnt0 += v;
-                run += (uint32_t)w2 < wave ? v : 0u;
-            }
-        } else {
-            // lane w reads wave w's count (NW is a power of two)
-            const uint32_t wv = wzero[ln & (NW - 1)];
-            const uint32_t wex = lane_scan_excl<NW>(wv);
-            run = (uint32_t)__builtin_amdgcn_readlane((int)wex, (int)wave);
-            cnt0 = (uint32_t)__builtin_amdgcn_readlane((int)(wex + wv), NW - 1);
-        }
-        // count0 of the row (its zeros among the K chosen haplotypes: the
-        // padding positions are all ones) into lane (step & 15); the forward
-        // pass stores each block's 16 at the next block boundary
-        c0acc = eimp_llvm_writelane(cnt0, step & 15u, c0acc);
-        // lane c: zeros before chunk ch0 + c (lanes >= NS: don't care)
-        const uint32_t zbv = run + zex;
-        // A row whose K bits are all equal (about a fifth of the rows on
-        // these panels) leaves the order as it is: no partition, no second
-        // barrier, no read-back.  cnt0 is the same in every wave, so the whole
-        // workgroup takes the same branch.
-        if (cnt0 != 0u && cnt0 != K) {
-            // pass 2: stable partition, zeros first.  For slot c let ob_c / run_c
-            // be the destinations of the row's first one / zero at or after the
-            // chunk (ob_c = cnt0 + ones before it, run_c = zeros before it, so
-            // ob_c + run_c = cnt0 + 64 (ch0 + c)) and t the ones below me in the
-            // chunk: a one goes to ob_c + t, a zero to run_c + ln - t.  With
-            //   x = ob_c + t + 32 (NS - 1 - c)
-            // dest + 32 (NS - 1 - c) is x for a one and V - x for a zero, with
-            // V = cnt0 + 64 ch0 + ln + 64 (NS - 1) the same for every slot, so
-            //   PBIAS + 4 dest = 4 sel + 128 c,  sel = bit ? x : V - x >= 0,
-            // and 128 c is the store's immediate offset (pay[] starts at byte
-            // PBIAS = 128 (NS - 1)).  In bytes: 4x = 4t + 4a_c with
-            // a_c = ob_c + 32 (NS - 1 - c) (one v_lshl_add with the scalar
-            // 4a_c), 4(V - x) = 4V - 4x; a_c is a scalar running sum
-            // (a_{c+1} = a_c + ones_c - 32), so a slot costs
-            // five vector instructions and its store.  No branch on the
-            // chunk's contents: a test for all-equal chunks costs more (scalar
-            // compare and taken branches) than the vector instructions it
-            // would skip.
-            {
-                uint32_t a4 = (cnt0 + ch0 * 64u - run + 32u * (NS - 1)) * 4u;
-                const uint32_t V4 = vbase4 + cnt0 * 4u;
-                static_for<0, NS>([&](auto ci) {
-                    constexpr int c = decltype(ci)::value;
-                    const uint64_t m = mk[c];
-                    const uint32_t x4 = mbcnt(m) * 4u + a4;
-                    const uint32_t sel4 = __builtin_amdgcn_inverse_ballot_w64(m) ? x4 : V4 - x4;
-                    *(lds_ptr_t<uint32_t>)(size_t)(sel4 + 128u * (uint32_t)c) = p[c];
-                    a4 += (uint32_t)__popcll(m) * 4u - 128u;
-                    // opaque scalar: keeps the running sum in bytes (left to
-                    // itself the compiler factors the 4 out, one more vector op)
-                    asm volatile("" : "+s"(a4));
-                });
-            }
-            __syncthreads();
-#pragma unroll
-            for (int c = 0; c < NS; c++) p[c] = pay[(ch0 + (uint32_t)c) * 64 + ln];
-        }
-        if constexpr (ABS) {
-            if (absperm) {
-                const gptr_t<int32_t> ap = gmem(absperm) + (uint64_t)(step + 1) * K;
-#pragma unroll
-                for (int c = 0; c < NS; c++) {
-                    const uint32_t pos = (ch0 + (uint32_t)c) * 64 + ln;
-                    if (pos < K) ap[pos] = (int32_t)(p[c] >> 16);
-                }
-            }
-        }
-        // the row: chunk ch holds pairs 2ch and 2ch+1 (raw layout: words 2ch, 2ch+1)
-        const uint32_t o1 = zbv + 32u - (uint32_t)__popc(olo);
-        const uint32_t o3 = o1 + 32u - (uint32_t)__popc(ohi);
-        // the logical words only: the padding was filled before the loop
-        if (ostore) {
-            const gptr_t<char> rowb = (gptr_t<char>)(size_t)rowaddr;
-            *(gptr_t<u32x2>)(rowb + obyte) = u32x2{olo, raw ? ohi : o1};
-            if (second) *(gptr_t<u32x2>)(rowb + obyte + 8u) = u32x2{ohi, o3};
-        }
-        if (dig && ostore) {
-            // rotl(v ^ key, g mod 32) == rotr by -g: one v_alignbit each
-            const uint32_t g = g0 + step * KW;
-            const uint32_t dkey = g * kDigKey, dneg = 0u - g;
-            dsum += __builtin_amdgcn_alignbit(olo ^ dkey, olo ^ dkey, dneg);
-            const uint32_t x1 = o1 ^ (dkey + kDigKey);
-            dsum += __builtin_amdgcn_alignbit(x1, x1, dneg - 1u);
-            if (2 * och + 1 < npairs) {
-                const uint32_t x2 = ohi ^ (dkey + 2u * kDigKey), x3 = o3 ^ (dkey + 3u * kDigKey);
-                dsum += __builtin_amdgcn_alignbit(x2, x2, dneg - 2u);
-                dsum += __builtin_amdgcn_alignbit(x3, x3, dneg - 3u);
-            }
-        }
-        rowaddr += rs_bytes;
-        jbit = (jbit << jl) >> jr;
-    }
-    // the forward pass's last (partial) block of count0
-    if (!rev && wave == 0 && Mp > 0) {
-        const uint32_t b0 = (Mp - 1) & ~15u;
-        if (ln < Mp - b0) {
-            if constexpr (ABS) gmem(c0out)[b0 + ln] = (int32_t)c0acc;
-            else gmem(T.count0)[b0 + ln] = (int32_t)c0acc;
-        }
-    }
-    if (dig) {
-        dsum = wave_sum64(dsum);
-        if (ln == 0) atomicAdd((unsigned long long *)&T.digest[0], (unsigned long long)dsum);
-    }
-}
-
-// slot counts instantiated; a target uses the smallest one >= ceil(chunks / waves)
-constexpr int kSlotCounts[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 14, 16, 20, 24, 28, 32};
-constexpr int kNumSlotCounts = sizeof(kSlotCounts) / sizeof(kSlotCounts[0]);
-
-__host__ __device__ inline int pbwt_slots_for(uint32_t Kpad, int nt) {
-    const uint32_t need = (Kpad / 64 + nt / 64 - 1) / (nt / 64);
-    for (int i = 0; i < kNumSlotCounts; i++)
-        if ((uint32_t)kSlotCounts[i] >= need) return kSlotCounts[i];
-    return -1;
-}
-
-template <int NT, int CPW, int WS>
-__device__ __forceinline__ void pbwt_target(const TgtDev &T, const bool rev, uint32_t *smem) {
-    const int ns = pbwt_slots_for(T.Kpad, NT);
-    static_for<0, kNumSlotCounts>([&](auto ii) {
-        constexpr int NSv = kSlotCounts[decltype(ii)::value];
-        if constexpr (NSv <= CPW) {
-            if (ns == NSv) pbwt_steps<NT, NSv, false, WS>(T, rev, smem);
-        }
-    });
-}
-
-// Waves per SIMD that one workgroup's LDS allows at the variant's capacity
-// (at most 6, above which the larger variants would spill registers): the
-// register budget is capped so that VGPRs do not lower the occupancy (512 x 20:
-// three workgroups per CU need at most 85 VGPRs).
-constexpr int pbwt_waves_hint(int NT, int CPW) {
-    const int lds = (int)pbwt_pay_bias(CPW) + CPW * NT * 4 + 2 * (NT / 64) * 4;
-    const int w = (163840 / lds) * (NT / 256);
-    return w < 1 ? 1 : (w > 6 ? 6 : w);
-}
-
-template <int NT, int CPW, int WS>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(pbwt_waves_hint(NT, CPW))))
-void k_pbwt(const TgtDev *__restrict__ tg, const PbwtItem *__restrict__ items) {
-    extern __shared__ uint32_t smem[];
-    const PbwtItem it = items[blockIdx.x];
-    pbwt_target<NT, CPW, WS>(tg[it.t], it.dir != 0, smem);
-}
-
-// ---------------------------------------------------------------------------
-// Compressed PBWT for K beyond the LDS-resident kernels (src/PBWT.cpp:207-285,
-// the same rows): the order lives in global memory (two arrays of Kpad
-// haplotype indexes, swapped every step; L2-resident at these sizes) and only
-// the current row's K bits are staged in LDS.  One workgroup of BIG_NT
-// threads per item; wave w takes chunks w, w + NW, ... of 64 positions.  A
-// step: stage row r; pass 1 counts the zeros of every chunk (ballots) into
-// LDS; a block scan turns them into zeros-before-chunk; pass 2 recomputes
-// each chunk's ballot, scatters every index to its place under the stable
-// partition (zeros first) and writes the chunk's (data, cumulative zeros)
-// pairs.  Positions K..Kpad-1 hold index K and read as ones (1-padding).
-// ---------------------------------------------------------------------------
-constexpr int BIG_NT = 1024;
-constexpr uint32_t kBigMaxK = 1u << 19;  // LDS: K/8 bytes of row + K/16 of chunk counts
-
-
-__device__ __forceinline__ uint32_t big_bit(const uint32_t *rowb, uint32_t idx, uint32_t K) {
-    return idx < K ? (rowb[idx >> 5] >> (idx & 31)) & 1u : 1u;
-}
-
-__global__ __launch_bounds__(BIG_NT) void k_pbwt_big(const BigItem *__restrict__ items) {
-    extern __shared__ uint32_t smem[];
-    constexpr uint32_t NW = BIG_NT / 64;
-    const BigItem I = items[blockIdx.x];
-    const uint32_t K = I.K, Mp = I.Mp, RS = I.RS;
-    const uint32_t Kpad = (K + 63) / 64 * 64, nch = Kpad / 64;
-    const uint32_t nw32 = (K + 31) / 32, npairs = nw32, KW = 2 * npairs;
-    uint32_t *rowb = smem;               // nw32 words: the current row
-    uint32_t *cz = smem + (nw32 + 1) / 2 * 2;  // nch: zeros per chunk, then zeros before it
-    __shared__ uint32_t s_part[NW + 1];
-    const uint32_t tid = threadIdx.x, wave = tid >> 6, ln = lane_id();
-    gptr_t<uint32_t> ordA = gmem(I.ord0), ordB = gmem(I.ord1);
-    for (uint32_t q = tid; q < Kpad; q += BIG_NT) {
-        ordA[q] = q < K ? q : K;
-        if (I.absperm && q < K) gmem(I.absperm)[q] = (int32_t)q;
-    }
-    {
-        // the padding words of every row, stored once (as pbwt_steps)
-        const uint32_t pw0 = I.raw ? 2 * nch : 2 * npairs;
-        const uint32_t fw = I.raw ? ~0u : 0u;
-        for (uint32_t rr = tid; rr < Mp; rr += BIG_NT) {
-            gptr_t<uint32_t> prow = gmem(I.out) + (uint64_t)rr * RS;
-            for (uint32_t w = pw0; w < RS; w++) prow[w] = fw;
-        }
-    }
-    uint64_t dsum = 0;
-    __syncthreads();
-    for (uint32_t step = 0; step < Mp; step++) {
-        const uint32_t r = I.rev ? Mp - 1 - step : step;
-        const gptr_t<const uint32_t> src = (gptr_t<const uint32_t>)(I.rows + (uint64_t)r * I.rstride);
-        for (uint32_t q = tid; q < nw32; q += BIG_NT) rowb[q] = src[q];
-        __syncthreads();
-        // pass 1: zeros of every chunk
-        for (uint32_t ch = wave; ch < nch; ch += NW) {
-            const uint32_t idx = ordA[ch * 64 + ln];
-            const uint64_t m = __ballot(big_bit(rowb, idx, K));
-            if (ln == 0) cz[ch] = 64u - (uint32_t)__popcll(m);
-        }
-        __syncthreads();
-        // exclusive scan of cz over the chunks: thread tid owns a contiguous run
-        const uint32_t per = (nch + BIG_NT - 1) / BIG_NT;
-        const uint32_t c0 = min(nch, tid * per), c1 = min(nch, c0 + per);
-        uint32_t mine = 0;
-        for (uint32_t c = c0; c < c1; c++) mine += cz[c];
-        const uint32_t incl = wave_scan_incl(mine);
-        if (ln == 63) s_part[wave] = incl;
-        __syncthreads();
-        uint32_t before = 0, total = 0;
-        for (uint32_t w = 0; w < NW; w++) {
-            const uint32_t v = s_part[w];
-            total += v;
-            before += w < wave ? v : 0u;
-        }
-        uint32_t run = before + incl - mine;
-        for (uint32_t c = c0; c < c1; c++) {
-            const uint32_t z = cz[c];
-            cz[c] = run;
-            run += z;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            if (I.count0) gmem(I.count0)[r] = (int32_t)total;
-        }
-        // pass 2: scatter the order, write the row's pairs
-        const gptr_t<uint32_t> row = gmem(I.out) + (uint64_t)step * RS;
-        for (uint32_t ch = wave; ch < nch; ch += NW) {
-            const uint32_t pos = ch * 64 + ln;
-            const uint32_t idx = ordA[pos];
-            const uint32_t b = big_bit(rowb, idx, K);
-            const uint64_t m = __ballot(b);
-            const uint32_t zb = __builtin_amdgcn_readfirstlane(cz[ch]);
-            const uint32_t t = mbcnt(m);  // ones below me in the chunk
-            const uint32_t dest = b ? total + (ch * 64u - zb) + t : zb + (ln - t);
-            ordB[dest] = idx;
-            if (I.absperm && dest < K) gmem(I.absperm)[(uint64_t)(step + 1) * K + dest] = (int32_t)idx;
-            const uint32_t lo = (uint32_t)m, hi = (uint32_t)(m >> 32);
-            const uint32_t o1 = zb + 32u - (uint32_t)__popc(lo);
-            const uint32_t o3 = zb + 64u - (uint32_t)__popcll(m);
-            const bool second = 2 * ch + 1 < npairs;
-            if (ln == 0) {
-                if (I.raw) {
-                    row[2 * ch] = lo;
-                    row[2 * ch + 1] = hi;
-                } else {
-                    row[4 * ch] = lo;
-                    row[4 * ch + 1] = o1;
-                    if (second) {
-                        row[4 * ch + 2] = hi;
-                        row[4 * ch + 3] = o3;
-                    }
-                }
-                if (I.digest) {
-                    const uint64_t g = I.gbase + (uint64_t)step * KW + 4ull * ch;
-                    dsum += (uint64_t)dig_word(g, lo) + dig_word(g + 1, o1);
-                    if (second) dsum += (uint64_t)dig_word(g + 2, hi) + dig_word(g + 3, o3);
-                }
-            }
-        }
-        __syncthreads();  // the new order is complete (and cz free) before the next step
-        const gptr_t<uint32_t> tmp = ordA;
-        ordA = ordB;
-        ordB = tmp;
-    }
-    if (I.digest && ln == 0) atomicAdd((unsigned long long *)I.digest, (unsigned long long)dsum);
-}
-
-static hipError_t raise_lds_limit(const void *fn, size_t lds);
-
-size_t pbwt_big_lds_bytes(uint32_t K) {
-    const uint32_t nw32 = (K + 31) / 32, nch = (K + 63) / 64;
-    return (size_t)((nw32 + 1) / 2 * 2 + nch) * 4;
-}
-uint32_t pbwt_big_max_k() { return kBigMaxK; }
-
-hipError_t launch_pbwt_big(const BigItem *items, uint32_t nitems, uint32_t maxK, hipStream_t s) {
-    if (!nitems) return hipSuccess;
-    const size_t lds = pbwt_big_lds_bytes(maxK);
-    hipError_t e = raise_lds_limit((const void *)k_pbwt_big, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_pbwt_big, dim3(nitems), dim3(BIG_NT), lds, s, items);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// Panel PBWT for imputation (PBWT(refT, true), src/PBWT.cpp:53-71,131-153):
-// one workgroup, forward only, K = all panel haplotypes, the absolute order
-// after every site and count0 per site written out.
-// ---------------------------------------------------------------------------
-template <int NT, int CPW>
-__global__ __launch_bounds__(NT) void k_panel_pbwt(TgtDev T, int32_t *__restrict__ absperm,
-                                                  int32_t *__restrict__ c0out) {
-    extern __shared__ uint32_t smem[];
-    const int ns = pbwt_slots_for(T.Kpad, NT);
-    static_for<0, kNumSlotCounts>([&](auto ii) {
-        constexpr int NSv = kSlotCounts[decltype(ii)::value];
-        if constexpr (NSv <= CPW) {
-            if (ns == NSv) pbwt_steps<NT, NSv, true, 1>(T, false, smem, absperm, c0out);
-        }
-    });
-}
-
 // Site rows [m0, m0 + nsites) of the panel as 16-row blocks, one uint16 per
 // haplotype (bit j = site m0 + 16b + j), haplotypes N..Kpad-1 all ones.
 // grid (nblk, ceil(nw/256)), block 256: a thread transposes one 64-haplotype word.
@@ -1621,8 +993,12 @@ __global__ __launch_bounds__(PLAN_NT) void k_plan(TgtDev *__restrict__ tg, Batch
             A.blockpref_id[t] = (uint32_t)bpi;
         }
     }
-    uint64_t nfit;
+    uint64_t nfit, nrow;
     (void)block_excl_scan64(fit ? 1u : 0u, s_w, nfit);
+    const uint64_t rp = block_excl_scan64(fit ? pbwt_blocks(Mp) : 0u, s_w, nrow);
+    if (t < kRowsCounters) A.rowpref[t] = 0;
+    if (valid) A.rowpref[kRowsCounters + t] = (uint32_t)rp;
+    if (t == 0) A.rowpref[kRowsCounters + n] = (uint32_t)nrow;
     if (t == 0) {
         if (!rrg) A.blockpref[n] = (uint32_t)nb_tot;
         if (!rri) A.blockpref_id[n] = (uint32_t)nb_id;
@@ -1738,32 +1114,6 @@ __global__ __launch_bounds__(CREF_NT, 4) void k_cref_persist_ident(PanelDev P,
     }
 }
 
-// PBWT items from the queue
-template <int NT, int CPW, int WS>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(pbwt_waves_hint(NT, CPW))))
-void k_pbwt_persist(const TgtDev *__restrict__ tg,
-                                                    BatchDev *__restrict__ B,
-                                                    const PbwtItem *__restrict__ items) {
-    // dynamic LDS only, so the payloads start at LDS address 0; the next item's
-    // index passes through smem[0], which no item uses between two items
-    extern __shared__ uint32_t smem[];
-    // highest wave priority for instruction issue: the PBWT chains bound the
-    // launch, and other contexts' kernels may share these CUs (measured:
-    // 1.3% off the launch at 200k x 500k)
-    __builtin_amdgcn_s_setprio(3);
-    const uint32_t np = B->npbwt;
-    for (;;) {
-        if (threadIdx.x == 0) smem[0] = atomicAdd(&B->pbwt_ctr, 1u);
-        __syncthreads();
-        const uint32_t i = __builtin_amdgcn_readfirstlane(smem[0]);
-        __syncthreads();
-        if (i >= np) break;
-        const PbwtItem it = items[i];
-        pbwt_target<NT, CPW, WS>(tg[it.t], it.dir != 0, smem);
-        __syncthreads();
-    }
-}
-
 // count0 digest (grid n, block 256)
 __global__ __launch_bounds__(256) void k_digest_count0(const TgtDev *__restrict__ tg,
                                                       const uint32_t *__restrict__ d_n) {
@@ -1827,7 +1177,7 @@ __global__ __launch_bounds__(256) void k_cref_rows(const TgtDev *__restrict__ tg
 // ---------------------------------------------------------------------------
 // The dynamic-LDS limit of a kernel is process-wide: contexts of different
 // sizes (and engines with different panels) only ever raise it.
-static hipError_t raise_lds_limit(const void *fn, size_t lds) {
+hipError_t raise_lds_limit(const void *fn, size_t lds) {
     static std::mutex mu;
     static std::map<const void *, size_t> limit;
     std::lock_guard<std::mutex> lk(mu);
@@ -1836,15 +1186,6 @@ static hipError_t raise_lds_limit(const void *fn, size_t lds) {
     hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e == hipSuccess) cur = lds;
     return e;
-}
-
-// The PBWT kernels address their payloads from LDS byte 0 (pbwt_steps):
-// they must have no static LDS ahead of the dynamic buffer.
-static hipError_t pbwt_lds_at_zero(const void *fn) {
-    hipFuncAttributes a{};
-    hipError_t e = hipFuncGetAttributes(&a, fn);
-    if (e != hipSuccess) return e;
-    return a.sharedSizeBytes == 0 ? hipSuccess : hipErrorInvalidKernelFile;
 }
 
 hipError_t launch_site_to_hap(const PanelDev &P, uint64_t *hap, hipStream_t s) {
@@ -1937,74 +1278,13 @@ hipError_t launch_cref_rows(const TgtDev *tg, uint32_t t, uint32_t Mp, uint64_t 
     return hipGetLastError();
 }
 
-// PBWT variants: (threads, chunks per wave), one-item-per-workgroup and queue kernels
-struct PbwtVariant {
-    int nt, cpw;
-    void (*fn)(const TgtDev *, const PbwtItem *);
-    void (*fn_persist)(const TgtDev *, BatchDev *, const PbwtItem *);
-};
-#define PBWT_VARIANT(NT, CPW, WS) {NT, CPW, k_pbwt<NT, CPW, WS>, k_pbwt_persist<NT, CPW, WS>}
-static const PbwtVariant kPbwtVariants[] = {
-    PBWT_VARIANT(256, 8, 0),  PBWT_VARIANT(256, 16, 0),  PBWT_VARIANT(512, 20, 0),
-    PBWT_VARIANT(512, 32, 0), PBWT_VARIANT(1024, 24, 0),
-    // the same shapes with the DPP wave-count scan (uniform targets)
-    PBWT_VARIANT(512, 20, 1), PBWT_VARIANT(1024, 24, 1),
-};
-#undef PBWT_VARIANT
-constexpr int kNumPbwtVariants = sizeof(kPbwtVariants) / sizeof(kPbwtVariants[0]);
-
-int pbwt_variant_count() { return kNumPbwtVariants; }
-int pbwt_variant_threads(int v) { return kPbwtVariants[v].nt; }
-int pbwt_variant_cpw(int v) { return kPbwtVariants[v].cpw; }
-uint32_t pbwt_variant_maxk(int v) {
-    return (uint32_t)(kPbwtVariants[v].nt / 64) * kPbwtVariants[v].cpw * 64;
-}
-size_t pbwt_lds_bytes(int v, uint32_t Kpad) {
-    const int nt = kPbwtVariants[v].nt;
-    const int ns = pbwt_slots_for(Kpad, nt);
-    if (ns < 0 || ns > kPbwtVariants[v].cpw) return ~(size_t)0;
-    const size_t npos = (size_t)ns * nt;  // NS x NW x 64
-    // bias, payloads (the cref stage shares them), wave counts
-    return pbwt_pay_bias(ns) + npos * 4 + 2 * (nt / 64) * 4;
-}
-hipError_t pbwt_prepare(int v, size_t lds) {
-    hipError_t e = pbwt_lds_at_zero((const void *)kPbwtVariants[v].fn);
-    if (e != hipSuccess) return e;
-    return raise_lds_limit((const void *)kPbwtVariants[v].fn, lds);
-}
-hipError_t launch_pbwt(int v, const TgtDev *tg, const PbwtItem *items, uint32_t nitems, size_t lds,
-                       hipStream_t s) {
-    if (!nitems) return hipSuccess;
-    hipLaunchKernelGGL(kPbwtVariants[v].fn, dim3(nitems), dim3(kPbwtVariants[v].nt), lds, s, tg,
-                       items);
-    return hipGetLastError();
-}
-
-// ---- panel PBWT for imputation: one workgroup of the 1024-thread variant
-hipError_t launch_panel_pbwt(const PanelDev &P, uint64_t m0, uint32_t nsites, uint16_t *blocks,
-                             uint32_t *rows, int32_t *c0out, int32_t *absperm, hipStream_t s) {
-    constexpr int NT = 1024, CPW = 24;
-    TgtDev T{};
-    T.K = P.N_ad;
-    T.Kpad = (P.N_ad + 63) / 64 * 64;
-    T.Mp = nsites;
-    T.RS = row_stride(T.K, LAYOUT_COMPACT);
-    T.cref = blocks;
-    T.out = rows;
-    const int ns = pbwt_slots_for(T.Kpad, NT);
-    if (ns < 0 || ns > CPW) return hipErrorInvalidValue;
+hipError_t launch_site_blocks(const PanelDev &P, uint64_t m0, uint32_t nsites, uint16_t *blocks,
+                              hipStream_t s) {
     const uint32_t nw = (P.N_ad + 63) / 64;
     hipLaunchKernelGGL(k_site_blocks, dim3((nsites + 15) / 16, (nw + 255) / 256), dim3(256), 0, s, P,
-                       m0, nsites, blocks, T.Kpad);
-    const size_t lds = pbwt_pay_bias(ns) + (size_t)ns * NT * 4 + 2 * (NT / 64) * 4;
-    hipError_t e = pbwt_lds_at_zero((const void *)k_panel_pbwt<NT, CPW>);
-    if (e != hipSuccess) return e;
-    e = raise_lds_limit((const void *)k_panel_pbwt<NT, CPW>, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_panel_pbwt<NT, CPW>), dim3(1), dim3(NT), lds, s, T, absperm, c0out);
+                       m0, nsites, blocks, (P.N_ad + 63) / 64 * 64);
     return hipGetLastError();
 }
-uint32_t panel_pbwt_max_k() { return 1024 / 64 * 24 * 64; }
 
 // ---- device-driven batch (stream contexts)
 
@@ -2082,19 +1362,4 @@ hipError_t launch_cref_persist(const PanelDev &P, const TgtDev *tg, BatchDev *B,
                            blockpref_id);
     return hipGetLastError();
 }
-hipError_t pbwt_persist_prepare(int v, size_t lds, int *occ) {
-    const void *fn = (const void *)kPbwtVariants[v].fn_persist;
-    hipError_t e = pbwt_lds_at_zero(fn);
-    if (e != hipSuccess) return e;
-    e = raise_lds_limit(fn, lds);
-    if (e != hipSuccess) return e;
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, fn, kPbwtVariants[v].nt, lds);
-}
-hipError_t launch_pbwt_persist(int v, const TgtDev *tg, BatchDev *B, const PbwtItem *items,
-                               uint32_t grid, size_t lds, hipStream_t s) {
-    hipLaunchKernelGGL(kPbwtVariants[v].fn_persist, dim3(grid), dim3(kPbwtVariants[v].nt), lds, s,
-                       tg, B, items);
-    return hipGetLastError();
-}
-
 }  // namespace eimp
