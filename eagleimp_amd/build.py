@@ -55,8 +55,9 @@ def build_engine():
     from concurrent.futures import ThreadPoolExecutor
     hip = _hipcc()
     cmds, objs = [], []
-    for src in ("eimp_pbwt.hip", "eimp_kernels.hip", "eimp_engine.cpp", "eimp_phase.cpp",
-                "eimp_qref.cpp"):
+    for src in ("eimp_order_512x32.hip", "eimp_order_1024x24.hip", "eimp_order_512x20.hip",
+                "eimp_order_256x16.hip", "eimp_order_256x8.hip", "eimp_pbwt.hip",
+                "eimp_kernels.hip", "eimp_engine.cpp", "eimp_phase.cpp", "eimp_qref.cpp"):
         obj = os.path.join(CSRC, "_" + os.path.splitext(src)[0] + ".o")
         if src in ("eimp_phase.cpp", "eimp_qref.cpp"):
             cc = ["g++", *HOST_FLAGS]

@@ -30,10 +30,14 @@ using namespace eimp;
 // device's copy comes from hipGetSymbolAddress (scratch_for_device) and only
 // that address is passed to kernels and copies.
 // kScratchBytes is what a batch's buffers may take; the PBWT's own tables come
-// from the extra part behind it: 26 bytes per block and direction, and a block
-// has at least 128 bytes of condensed reference in the first part.
+// from the extra part behind it: 26 bytes per block and direction (a block has
+// at least 128 bytes of condensed reference in the first part), the segments of
+// cut chains (at most kScratchSegs; their items are fewer bytes than they).
 static constexpr size_t kScratchBytes = 64ull << 20;
-static constexpr size_t kScratchExtra = 28ull << 20;
+static constexpr size_t kScratchSegs = 16ull << 20;
+static constexpr size_t kScratchExtra = 64ull << 20;
+// segments of cut chains where the device memory is the engine's
+static constexpr size_t kSegBytes = 64ull << 20;
 static constexpr size_t kNoAllocMaxTargets = 256;
 static __device__ __align__(256) uint64_t scratch[(kScratchBytes + kScratchExtra) / 8];
 
@@ -150,7 +154,7 @@ struct eimp_engine {
     // batch pools
     DevBuf d_tg, d_gt, d_nerr, d_bh, d_bhflags, d_mono, d_splitsites, d_splits, d_cMdiffs,
         d_stats, d_cref, d_count0, d_out, d_digest, d_tlist, d_citems, d_pitems, d_tmp,
-        d_hdr, d_rowpref, d_rowlist, d_crows, d_ord, d_big;  // PBWT tables; large-K PBWT: row-major cref, orders, items
+        d_hdr, d_rowpref, d_rowlist, d_seg, d_crows, d_ord, d_big;  // PBWT tables; large-K PBWT: row-major cref, orders, items
     DevBuf p_blocks, p_rows, p_c0, p_abs, p_tg, p_items, p_list, p_hdr, p_starts;  // panel PBWT
     HostBuf h_stage;
     std::vector<TgtDev> h_tg;
@@ -169,6 +173,7 @@ struct eimp_engine {
     uint64_t panel_gen = 0;  // bumped whenever panel buffers change (stream contexts check it)
     int pbwt_prepared_variant = -1;
     size_t pbwt_prepared_lds = 0;
+    int pbwt_prepared_occ = 1;  // resident workgroups per CU
     uint32_t ncu = 0;  // compute units
 
     hipEvent_t get_event() {
@@ -213,7 +218,7 @@ struct eimp_engine {
     void release_pools() {
         DevBuf *bufs[] = {&d_tg, &d_gt, &d_nerr, &d_bh, &d_bhflags, &d_mono, &d_splitsites,
                           &d_splits, &d_cMdiffs, &d_stats, &d_cref, &d_count0, &d_out,
-                          &d_digest, &d_tlist, &d_citems, &d_pitems, &d_tmp, &d_hdr, &d_rowpref, &d_rowlist, &d_crows,
+                          &d_digest, &d_tlist, &d_citems, &d_pitems, &d_tmp, &d_hdr, &d_rowpref, &d_rowlist, &d_seg, &d_crows,
                           &d_ord, &d_big,
                           &p_blocks, &p_rows, &p_c0, &p_abs, &p_tg, &p_items, &p_list, &p_hdr, &p_starts};
         for (auto *b : bufs) b->release();
@@ -275,14 +280,49 @@ int ensure_pmono(eimp_engine *e) {
     return e->sync();
 }
 
+// chains' worth of parallel work on the device, times 10: a further workgroup
+// on a CU adds about 0.2 of the first (384 chains of 941 blocks on 256 CUs take
+// 9.3 ms at K = 10,000, one alone 6.3)
+uint32_t seg_par(const eimp_engine *e, int occ) {
+    return e->ncu * (10u + 2u * (uint32_t)std::max(occ - 1, 0));
+}
+
+// The segments of chains of nblk blocks (cut alike in both directions; Kpad
+// each): the candidate with the least expected time (as k_plan).  Returns L.
+uint32_t choose_segments(const std::vector<uint32_t> &nblk, const std::vector<uint32_t> &Kpad, uint32_t par,
+                         uint64_t cap_words, uint32_t max_segs) {
+    uint64_t t_none = 0, t_best = 0;
+    uint32_t best = 0;
+    for (int c = kSegCands; c >= 0; c--) {
+        const uint32_t L = c < kSegCands ? 4u << c : 0u;
+        uint64_t path = 0, work = 0, words = 0, segs = 0;
+        for (size_t i = 0; i < nblk.size(); i++) {
+            uint32_t len;
+            const uint32_t S = seg_split(nblk[i], L, len);
+            path = std::max(path, seg_path(nblk[i], S, len, Kpad[i]));
+            work += seg_work(nblk[i], S, Kpad[i]);
+            words += seg_words(S, Kpad[i]);
+            segs += S > 1 ? 2 * S : 0;
+        }
+        const uint64_t t = seg_time(path, work, par);
+        if (c == kSegCands) {
+            t_none = t_best = t;
+        } else if (words <= cap_words && segs <= max_segs && t < t_best && t < t_none - t_none / 4) {
+            t_best = t;
+            best = L;
+        }
+    }
+    return best;
+}
+
 // Where one batch's device buffers come from: the engine's grow-only pools
 // (eimp_engine_run_batch, the drop-in call) or a bump allocator over the
 // file-scope scratch array with caller-provided outputs
 // (eimp_engine_run_batch_noalloc).
 enum MemSlot : int {
     MS_TG, MS_NERR, MS_BH, MS_BHF, MS_MONO, MS_SS, MS_SPL, MS_CMD, MS_STATS, MS_TLIST,
-    MS_CREF, MS_DIG, MS_CITEMS, MS_PITEMS, MS_CROWS, MS_ORD, MS_BIG,
-    MS_HDR, MS_RPREF, MS_RLIST  // tables of the PBWT
+    MS_CREF, MS_DIG, MS_CITEMS, MS_CROWS, MS_ORD, MS_BIG,
+    MS_OITEMS, MS_HDR, MS_RPREF, MS_RLIST, MS_SEG  // tables of the PBWT
 };
 struct BatchMem {
     virtual ~BatchMem() = default;
@@ -290,6 +330,8 @@ struct BatchMem {
     virtual int get(MemSlot s, size_t bytes, const char *what, void **p) = 0;
     // sets T.out and T.count0 of targets 0..n-1 (Mp and RS set)
     virtual int place_outputs(std::vector<TgtDev> &tg, uint32_t n) = 0;
+    // bytes that the segments of cut chains may take
+    virtual uint64_t seg_room() const { return kSegBytes; }
     // false: nothing may be allocated (resident panel parts must exist already)
     virtual bool may_alloc() const { return true; }
 };
@@ -312,6 +354,7 @@ struct PoolMem final : BatchMem {
         case MS_CREF: return e->d_cref;
         case MS_DIG: return e->d_digest;
         case MS_CITEMS: return e->d_citems;
+        case MS_SEG: return e->d_seg;
         case MS_HDR: return e->d_hdr;
         case MS_RPREF: return e->d_rowpref;
         case MS_RLIST: return e->d_rowlist;
@@ -358,7 +401,7 @@ struct ScratchMem final : BatchMem {
         : base(reinterpret_cast<char *>(scr)), rows(rows_), c0(c0_), max_Mp(max_Mp_) {}
     int get(MemSlot s, size_t bytes, const char *what, void **p) override {
         const size_t b = round_up(std::max<size_t>(bytes, 1), 256);
-        if (s >= MS_HDR) {
+        if (s >= MS_OITEMS) {
             if (used_extra + b > kScratchExtra)
                 return fail(EIMP_ERR_UNSUPPORTED, std::string("no-allocation scratch full (at ") + what + ")");
             *p = base + kScratchBytes + used_extra;
@@ -386,6 +429,7 @@ struct ScratchMem final : BatchMem {
         }
         return EIMP_OK;
     }
+    uint64_t seg_room() const override { return kScratchSegs; }
     bool may_alloc() const override { return false; }
 };
 
@@ -407,6 +451,20 @@ int scratch_for_device(int dev, uint64_t **out) {
     return EIMP_OK;
 }
 
+// Items of one chain (kind CHAIN_ROWS or CHAIN_STARTS) cut into S segments.
+void chain_items(uint32_t t, uint32_t dir, uint32_t nblk, uint32_t S, uint32_t len, uint32_t kind,
+                 std::vector<OrderItem> &rows, std::vector<OrderItem> &rank, std::vector<OrderItem> &comb) {
+    for (uint32_t s = 0; s < S; s++) {
+        const uint32_t q0 = s * len, q1 = std::min(nblk, q0 + len);
+        rows.push_back(OrderItem{t, dir, kind, s, q0, q1});
+        if (s + 1 < S) {
+            rank.push_back(OrderItem{t, dir, CHAIN_RANK_UP, s, q0, q1});
+            rank.push_back(OrderItem{t, dir, CHAIN_RANK_DOWN, s, q0, q1});
+        }
+    }
+    if (S > 1) comb.push_back(OrderItem{t, dir, CHAIN_COMBINE, 0, 0, S});
+}
+
 // Phase B for targets whose phase-A fields (bh, splitsites, S) are in place.
 // Sizes outputs, builds cref + PBWT in the given output layout (LAYOUT_*).
 int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem &mem) {
@@ -418,7 +476,7 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
     uint64_t hdr_elems = 0;
     uint32_t Kmax_pad = 0, Kmax = 0, Kbig = 0;
     std::vector<CrefItem> citems, citems_id;  // general / identity targets
-    std::vector<PbwtItem> pitems;
+    std::vector<uint32_t> chains;             // targets of the chain kernel
     std::vector<uint32_t> big;                // targets beyond the LDS-resident PBWT kernels
     uint32_t lds_cap = 0;
     for (int v = 0; v < pbwt_variant_count(); v++) lds_cap = std::max(lds_cap, pbwt_variant_maxk(v));
@@ -452,8 +510,7 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
             ord_bytes += 4ull * T.Kpad * 4;
         } else {
             Kmax_pad = std::max(Kmax_pad, T.Kpad);
-            pitems.push_back(PbwtItem{t, 0});
-            pitems.push_back(PbwtItem{t, 1});
+            chains.push_back(t);
             hdr_off[t] = hdr_elems;
             hdr_elems += 2 * nblk;
         }
@@ -471,33 +528,53 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
         return fail(EIMP_ERR_UNSUPPORTED, "panel too wide for the cref kernel's LDS staging");
     int v = -1;
     size_t lds = 0;
-    if (!pitems.empty()) {
+    if (!chains.empty()) {
         v = e->choose_pbwt_variant(Kmax_pad);
         if (v < 0) return v;
         lds = pbwt_lds_bytes(v, Kmax_pad);
         if (lds > 160 * 1024)
             return fail(EIMP_ERR_UNSUPPORTED, "K beyond the PBWT kernel's slots or 160 KiB of LDS");
         if (e->pbwt_prepared_variant != v || e->pbwt_prepared_lds < lds) {
-            HIPCHK(pbwt_prepare(v, lds, nullptr));
+            HIPCHK(pbwt_prepare(v, lds, &e->pbwt_prepared_occ));
             e->pbwt_prepared_variant = v;
             e->pbwt_prepared_lds = lds;
         }
     }
+    // chains longest first, cut into segments where that shortens the batch
+    std::stable_sort(chains.begin(), chains.end(), [&](uint32_t a, uint32_t b) { return tg[a].Mp > tg[b].Mp; });
+    std::vector<OrderItem> oitems, rank_items, comb_items;
+    uint64_t seg_elems = 0;
+    std::vector<uint64_t> seg_off(n, 0);
+    if (!chains.empty()) {
+        std::vector<uint32_t> nb, kp;
+        for (uint32_t t : chains) {
+            nb.push_back((tg[t].Mp + 15) / 16);
+            kp.push_back(tg[t].Kpad);
+        }
+        const uint32_t L = choose_segments(nb, kp, seg_par(e, e->pbwt_prepared_occ), mem.seg_room() / 2, ~0u);
+        for (size_t i = 0; i < chains.size(); i++) {
+            TgtDev &T = tg[chains[i]];
+            T.nseg = seg_split(nb[i], L, T.seglen);
+            seg_off[chains[i]] = seg_elems;
+            seg_elems += seg_words(T.nseg, T.Kpad);
+            for (uint32_t dir = 0; dir < 2; dir++) chain_items(chains[i], dir, nb[i], T.nseg, T.seglen, CHAIN_ROWS, oitems, rank_items, comb_items);
+        }
+    }
+    const size_t nrows_items = oitems.size(), nrank = rank_items.size();
+    oitems.insert(oitems.end(), rank_items.begin(), rank_items.end());
+    oitems.insert(oitems.end(), comb_items.begin(), comb_items.end());
     if (!big.empty() && pbwt_big_lds_bytes(Kbig) > 160 * 1024)
         return fail(EIMP_ERR_UNSUPPORTED, "K beyond the large-K PBWT kernel's LDS");
-    // longest targets first
-    std::stable_sort(pitems.begin(), pitems.end(), [&](const PbwtItem &a, const PbwtItem &b) {
-        return tg[a.t].Mp > tg[b.t].Mp;
-    });
     void *p_cref = nullptr, *p_dig = nullptr, *p_ci = nullptr, *p_pi = nullptr, *p_tg = nullptr;
     void *p_crows = nullptr, *p_ord = nullptr, *p_big = nullptr, *p_hdr = nullptr, *p_rp = nullptr,
-         *p_rl = nullptr;
+         *p_rl = nullptr, *p_seg = nullptr;
     CHK(mem.get(MS_CREF, cref_bytes, "cref", &p_cref));
     CHK(mem.get(MS_DIG, (size_t)n * 16, "digest", &p_dig));
     const size_t nci = citems.size();
     citems.insert(citems.end(), citems_id.begin(), citems_id.end());
     CHK(mem.get(MS_CITEMS, std::max<size_t>(citems.size(), 1) * sizeof(CrefItem), "cref items", &p_ci));
-    CHK(mem.get(MS_PITEMS, std::max<size_t>(pitems.size(), 1) * sizeof(PbwtItem), "pbwt items", &p_pi));
+    CHK(mem.get(MS_OITEMS, std::max<size_t>(oitems.size(), 1) * sizeof(OrderItem), "pbwt items", &p_pi));
+    CHK(mem.get(MS_SEG, seg_elems * 2, "pbwt segments", &p_seg));
     CHK(mem.get(MS_HDR, hdr_elems * 2, "block headers", &p_hdr));
     CHK(mem.get(MS_RPREF, rowpref.size() * 4, "row prefix", &p_rp));
     CHK(mem.get(MS_RLIST, 2ull * rowpref.back() * sizeof(RowItem), "row items", &p_rl));
@@ -511,11 +588,12 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
     uint64_t *d_dig = static_cast<uint64_t *>(p_dig);
     TgtDev *d_tg = static_cast<TgtDev *>(p_tg);
     CrefItem *d_ci = static_cast<CrefItem *>(p_ci);
-    PbwtItem *d_pi = static_cast<PbwtItem *>(p_pi);
+    OrderItem *d_oi = static_cast<OrderItem *>(p_pi);
     for (uint32_t t = 0; t < n; t++) {
         TgtDev &T = tg[t];
         T.cref = reinterpret_cast<uint16_t *>(static_cast<char *>(p_cref) + cref_off[t]);
         T.hdr = static_cast<uint16_t *>(p_hdr) + hdr_off[t];
+        T.seg = static_cast<uint16_t *>(p_seg) + seg_off[t];
         T.digest = digest ? d_dig + 2 * t : nullptr;
     }
     std::vector<BigItem> bitems;
@@ -548,8 +626,8 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
     if (!citems.empty())
         HIPCHK(hipMemcpyAsync(d_ci, citems.data(), citems.size() * sizeof(CrefItem),
                               hipMemcpyHostToDevice, e->stream));
-    if (!pitems.empty()) {
-        HIPCHK(hipMemcpyAsync(d_pi, pitems.data(), pitems.size() * sizeof(PbwtItem),
+    if (!oitems.empty()) {
+        HIPCHK(hipMemcpyAsync(d_oi, oitems.data(), oitems.size() * sizeof(OrderItem),
                               hipMemcpyHostToDevice, e->stream));
         HIPCHK(hipMemcpyAsync(p_rp, rowpref.data(), rowpref.size() * 4, hipMemcpyHostToDevice, e->stream));
     }
@@ -567,9 +645,14 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
     }
     e->tend(ti);
     ti = e->tbegin(EIMP_KCLASS_PBWT);
-    if (!pitems.empty()) {
-        HIPCHK(launch_order(v, d_tg, d_pi, (uint32_t)pitems.size(), nullptr, nullptr, nullptr, lds,
-                            e->stream));
+    if (!oitems.empty()) {
+        auto chains_run = [&](size_t first, size_t count, bool rows) {
+            return launch_order(v, d_tg, d_oi + first, rows, (uint32_t)count, nullptr, nullptr, nullptr, lds,
+                                e->stream);
+        };
+        HIPCHK(chains_run(nrows_items, nrank, false));
+        HIPCHK(chains_run(nrows_items + nrank, comb_items.size(), false));
+        HIPCHK(chains_run(0, nrows_items, true));
         uint32_t *rp = static_cast<uint32_t *>(p_rp);
         HIPCHK(launch_rows(d_tg, nullptr, n, rp + kRowsCounters, static_cast<RowItem *>(p_rl), rp,
                            Kmax_pad, rowpref.back(), e->ncu, e->stream));
@@ -858,14 +941,15 @@ struct eimp_stream {
     double kms[EIMP_NKCLASS] = {};
     // device buffers; d_in = header (256 B) | TgtDev[nmax] | genotypes
     DevBuf d_in, d_nerr, d_bh, d_bhflags, d_mono, d_splitsites, d_splits, d_cMdiffs, d_stats,
-        d_digest, d_blockpref, d_pitems, d_hdr, d_rowpref, d_rowlist, d_tmp;
+        d_digest, d_blockpref, d_oitems, d_seg, d_hdr, d_rowpref, d_rowlist, d_tmp;
     std::shared_ptr<StreamPool> pool;  // the output pool, maybe shared with other contexts
     uint64_t tab_off = 0, gt_off = 0, gt_cap_words = 0;
     HostBuf h_in, h_out;  // h_out = stats | digests | TgtDev table
     // launch configuration
     int pbwt_v = -1;
     size_t pbwt_lds = 0;
-    uint32_t cref_grid[2] = {0, 0}, pbwt_grid = 0;
+    uint32_t cref_grid[2] = {0, 0}, pbwt_grid = 0, seg_par = 0;
+    uint64_t seg_bytes = 0;
     hipGraph_t graph_prep = nullptr, graph_build = nullptr;
     hipGraphExec_t exec_prep = nullptr, exec_build = nullptr;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -913,7 +997,12 @@ int stream_launch_build(eimp_stream *s) {
     A.blockpref = s->d_blockpref.as<uint32_t>();
     A.blockpref_id = s->d_blockpref.as<uint32_t>() + s->nmax + 1;
     A.ident_ok = cref_ident_ok(e->pd) ? 1u : 0u;
-    A.pitems = s->d_pitems.as<PbwtItem>();
+    A.rows_items = s->d_oitems.as<OrderItem>();
+    A.rank_items = A.rows_items + 2 * s->nmax + kMaxSegments;
+    A.comb_items = A.rank_items + 2 * kMaxSegments;
+    A.seg = s->d_seg.as<uint16_t>();
+    A.seg_cap = s->seg_bytes / 2;
+    A.seg_par = s->seg_par;
     A.rowpref = s->d_rowpref.as<uint32_t>();
     A.layout = batch_layout(s->flags);
     A.digest = (s->flags & EIMP_BATCH_DIGEST) ? 1u : 0u;
@@ -929,8 +1018,13 @@ int stream_launch_build(eimp_stream *s) {
                                s->cref_grid, s->stream));
     CHK(mark(EIMP_KCLASS_PBWT));
     const uint32_t Kpad = (uint32_t)round_up(s->Kmax, 64);
-    HIPCHK(launch_order(s->pbwt_v, s->d_tg(), s->d_pitems.as<PbwtItem>(), s->pbwt_grid,
-                        &s->d_batch()->npbwt, &s->d_batch()->pbwt_ctr, nullptr, s->pbwt_lds, s->stream));
+    BatchDev *B = s->d_batch();
+    HIPCHK(launch_order(s->pbwt_v, s->d_tg(), A.rank_items, false, s->pbwt_grid, &B->nrank, &B->rank_ctr,
+                        nullptr, s->pbwt_lds, s->stream));
+    HIPCHK(launch_order(s->pbwt_v, s->d_tg(), A.comb_items, false, s->pbwt_grid, &B->ncomb, &B->comb_ctr,
+                        nullptr, s->pbwt_lds, s->stream));
+    HIPCHK(launch_order(s->pbwt_v, s->d_tg(), A.rows_items, true, s->pbwt_grid, &B->npbwt, &B->pbwt_ctr,
+                        nullptr, s->pbwt_lds, s->stream));
     HIPCHK(launch_rows(s->d_tg(), d_n, 0, A.rowpref + kRowsCounters, s->d_rowlist.as<RowItem>(),
                        A.rowpref, Kpad, (uint64_t)s->nmax * pbwt_blocks(2 * s->Wmax + 1), e->ncu,
                        s->stream));
@@ -962,7 +1056,7 @@ void stream_release(eimp_stream *s) {
     if (s->build_done) (void)hipEventDestroy(s->build_done);
     DevBuf *bufs[] = {&s->d_in, &s->d_nerr, &s->d_bh, &s->d_bhflags, &s->d_mono, &s->d_splitsites,
                       &s->d_splits, &s->d_cMdiffs, &s->d_stats, &s->d_digest, &s->d_blockpref,
-                      &s->d_pitems, &s->d_hdr, &s->d_rowpref, &s->d_rowlist, &s->d_tmp};
+                      &s->d_oitems, &s->d_seg, &s->d_hdr, &s->d_rowpref, &s->d_rowlist, &s->d_tmp};
     for (auto *b : bufs) b->release();
     s->h_in.release();
     s->h_out.release();
@@ -1019,7 +1113,7 @@ int stream_setup(eimp_stream *s, size_t pool_bytes, const std::shared_ptr<Stream
     CHK(s->d_stats.ensure(nmax * 16, "stats"));
     CHK(s->d_digest.ensure(nmax * 16, "digests"));
     CHK(s->d_blockpref.ensure(2 * (nmax + 1) * 4, "block prefix"));
-    CHK(s->d_pitems.ensure(2 * nmax * sizeof(PbwtItem), "pbwt items"));
+    CHK(s->d_oitems.ensure((4 * nmax + 3ull * kMaxSegments) * sizeof(OrderItem), "pbwt items"));
     // up to 2 W + 1 rows per direction: block headers of both directions
     const uint64_t hdr_n = pbwt_blocks(2 * s->Wmax + 1);
     CHK(s->d_hdr.ensure(nmax * hdr_n * 2, "block headers"));
@@ -1053,7 +1147,16 @@ int stream_setup(eimp_stream *s, size_t pool_bytes, const std::shared_ptr<Stream
     // identity targets need K == N_ad
     const bool ident_possible = cref_ident_ok(e->pd) && s->Kmax == e->Nad && e->Ncorr == e->Nad;
     s->cref_grid[1] = ident_possible ? (uint32_t)(std::max(ncu, 1) * std::max(occ_c[1], 1)) : 0u;
-    s->pbwt_grid = (uint32_t)std::min<uint64_t>(2 * nmax, (uint64_t)std::max(ncu, 1) * std::max(occ_p, 1));
+    // one workgroup per CU, or per chain where there are more: workgroups beyond
+    // the items take them first where they share a CU (192 targets on 768
+    // workgroups 11.8 ms, on 384 8.7 ms)
+    s->pbwt_grid = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(2 * nmax, (uint64_t)ncu),
+                                                (uint64_t)ncu * (uint64_t)std::max(occ_p, 1));
+    s->seg_par = seg_par(e, occ_p);
+    // segments of cut chains: at most sqrt(blocks) per chain
+    const uint64_t max_nblk = (2ull * s->Wmax + 1 + 15) / 16;
+    s->seg_bytes = std::min<uint64_t>(kSegBytes, nmax * seg_words(seg_isqrt((uint32_t)max_nblk) + 1, Kpad) * 2);
+    CHK(s->d_seg.ensure(s->seg_bytes, "pbwt segments"));
     // fixed per-slot pointers of the target table
     TgtDev *tab = reinterpret_cast<TgtDev *>(s->h_in.as<char>() + s->tab_off);
     for (uint64_t t = 0; t < nmax; t++) {
@@ -1422,11 +1525,12 @@ int eimp_engine_ref_pbwt(eimp_engine *e, size_t m0, size_t nsites, uint32_t *row
     CHK(e->p_rows.ensure(nsites * RS * 4, "panel PBWT rows"));
     CHK(e->p_c0.ensure(nsites * 4, "panel PBWT count0"));
     if (absperm) CHK(e->p_abs.ensure((nsites + 1) * N * 4, "panel PBWT permutations"));
+    std::vector<OrderItem> oitems, rank_items, comb_items;
+    size_t lds = 0;
     if (!big) {
         // one forward chain over the site blocks: a target record, its chain
         // item and the rows' work items (the forward half only)
         CHK(e->p_tg.ensure(sizeof(TgtDev), "panel PBWT record"));
-        CHK(e->p_items.ensure(sizeof(PbwtItem) + (kRowsCounters + 2) * 4, "panel PBWT items"));
         CHK(e->p_list.ensure(2 * nblk * sizeof(RowItem), "panel PBWT row items"));
         CHK(e->p_hdr.ensure(nblk * 4, "panel PBWT block headers"));
         if (absperm) CHK(e->p_starts.ensure(nblk * Kpad * 2, "panel PBWT block orders"));
@@ -1439,10 +1543,26 @@ int eimp_engine_ref_pbwt(eimp_engine *e, size_t m0, size_t nsites, uint32_t *row
         T.out = e->p_rows.as<uint32_t>();
         T.count0 = e->p_c0.as<int32_t>();
         T.hdr = e->p_hdr.as<uint16_t>();
-        uint32_t items[2 + kRowsCounters + 2] = {};
-        items[2 + kRowsCounters + 1] = (uint32_t)nblk;
+        lds = pbwt_lds_bytes(v, (uint32_t)Kpad);
+        int occ = 1;
+        HIPCHK(pbwt_prepare(v, lds, &occ));
+        // (the cost model counts two directions of a target: half the device)
+        const uint32_t L = choose_segments({(uint32_t)nblk}, {(uint32_t)Kpad}, 2 * seg_par(e, occ), kSegBytes / 2, ~0u);
+        T.nseg = seg_split((uint32_t)nblk, L, T.seglen);
+        chain_items(0, 0, (uint32_t)nblk, T.nseg, T.seglen, absperm ? CHAIN_STARTS : CHAIN_ROWS, oitems,
+                    rank_items, comb_items);
+        CHK(e->d_seg.ensure(std::max<uint64_t>(seg_words(T.nseg, T.Kpad) * 2, 256), "panel PBWT segments"));
+        T.seg = e->d_seg.as<uint16_t>();
+        // counters and the row prefix, then the chain items
+        std::vector<uint32_t> items(kRowsCounters + 2, 0u);
+        items[kRowsCounters + 1] = (uint32_t)nblk;
+        for (const auto *l : {&oitems, &rank_items, &comb_items}) {
+            const uint32_t *w = reinterpret_cast<const uint32_t *>(l->data());
+            items.insert(items.end(), w, w + l->size() * (sizeof(OrderItem) / 4));
+        }
+        CHK(e->p_items.ensure(items.size() * 4, "panel PBWT items"));
         HIPCHK(hipMemcpyAsync(e->p_tg.p, &T, sizeof(T), hipMemcpyHostToDevice, e->stream));
-        HIPCHK(hipMemcpyAsync(e->p_items.p, items, sizeof(items), hipMemcpyHostToDevice, e->stream));
+        HIPCHK(hipMemcpyAsync(e->p_items.p, items.data(), items.size() * 4, hipMemcpyHostToDevice, e->stream));
     }
     if (big) {
         CHK(e->d_ord.ensure(2 * Kpad * 4, "panel PBWT orders"));
@@ -1465,13 +1585,17 @@ int eimp_engine_ref_pbwt(eimp_engine *e, size_t m0, size_t nsites, uint32_t *row
     if (big)
         HIPCHK(launch_pbwt_big(e->d_big.as<BigItem>(), 1, (uint32_t)N, e->stream));
     else {
-        const size_t lds = pbwt_lds_bytes(v, (uint32_t)Kpad);
-        HIPCHK(pbwt_prepare(v, lds, nullptr));
         HIPCHK(launch_site_blocks(e->pd, m0, (uint32_t)nsites, e->p_blocks.as<uint16_t>(), e->stream));
         uint16_t *starts = absperm ? e->p_starts.as<uint16_t>() : nullptr;
-        HIPCHK(launch_order(v, e->p_tg.as<TgtDev>(), e->p_items.as<PbwtItem>(), 1, nullptr, nullptr, starts,
-                            lds, e->stream));
-        uint32_t *rp = e->p_items.as<uint32_t>() + 2;
+        const OrderItem *oi = reinterpret_cast<const OrderItem *>(e->p_items.as<uint32_t>() + kRowsCounters + 2);
+        auto chains_run = [&](size_t first, size_t count, bool rows) {
+            return launch_order(v, e->p_tg.as<TgtDev>(), oi + first, rows, (uint32_t)count, nullptr, nullptr,
+                                starts, lds, e->stream);
+        };
+        HIPCHK(chains_run(oitems.size(), rank_items.size(), false));
+        HIPCHK(chains_run(oitems.size() + rank_items.size(), comb_items.size(), false));
+        HIPCHK(chains_run(0, oitems.size(), !absperm));
+        uint32_t *rp = e->p_items.as<uint32_t>();
         if (absperm)
             HIPCHK(launch_dense(v, e->p_tg.as<TgtDev>(), (uint32_t)nblk, starts, e->p_abs.as<int32_t>(), lds,
                                 e->stream));

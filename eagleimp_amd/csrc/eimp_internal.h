@@ -65,12 +65,14 @@ struct TgtDev {
     uint16_t *cref;        // nblk x Kpad, transposed 16-row blocks
     int32_t *count0;       // Mp
     uint32_t *out;         // 2 x Mp x RS uint32 (forward rows, then backward rows)
+    uint16_t *seg;         // 2 x nseg x 3 x Kpad: segments of the chains (nseg > 1)
     uint16_t *hdr;         // 2 x nblk: runs listed in a block's rows (forward, then backward blocks)
     uint64_t *digest;      // [0] pbwt words, [1] count0
     uint32_t Mp;
     uint32_t Kpad;         // K rounded up to 64
     uint32_t RS;           // output row stride in uint32
     uint32_t S;
+    uint32_t nseg, seglen; // segments of each chain, blocks of a segment
 };
 
 // Device-side header of a batch run by a stream context (device-driven
@@ -78,7 +80,7 @@ struct TgtDev {
 struct BatchDev {
     uint32_t n;           // targets in this submission (written by the host)
     uint32_t ncref;       // cref blocks queued by k_plan: subset (gather) targets
-    uint32_t npbwt;       // PBWT items queued by k_plan
+    uint32_t npbwt;       // PBWT chain items queued by k_plan: rows
     uint32_t nfit;        // targets whose outputs fit the pools
     uint32_t cref_ctr;    // work-queue counters (zeroed by k_plan)
     uint32_t pbwt_ctr;
@@ -89,6 +91,8 @@ struct BatchDev {
     // in blockpref (item i = block i / nrr of target i % nrr)
     uint32_t rr[2];
     uint32_t nrr[2];
+    // chain items of cut chains: ranks of the segments, then their combination
+    uint32_t nrank, rank_ctr, ncomb, comb_ctr;
 };
 
 // 16-row blocks per work item of the subset cref kernel (256 splits)
@@ -109,10 +113,57 @@ struct RowItem {
 };
 constexpr uint32_t kRowsCounters = 4;
 
-// PBWT work item: target t, direction (0 fwd, 1 bck)
-struct PbwtItem {
-    uint32_t t, dir;
+// PBWT chain items (k_order): target t, direction (0 fwd, 1 bck), blocks
+// [q0, q1) in processing order, segment seg
+enum : uint32_t { CHAIN_ROWS, CHAIN_STARTS, CHAIN_RANK_UP, CHAIN_RANK_DOWN, CHAIN_COMBINE };
+struct OrderItem {
+    uint32_t t, dir, kind, seg, q0, q1;
 };
+
+// Cut of a chain of nblk blocks for segments of about L blocks (0: none).  A
+// cut chain is three times the blocks (both rank passes and the rows), so its
+// latency, 2 len + about 2 block times per segment for the combination, is
+// least near sqrt(nblk) segments and no gain below 3.
+__host__ __device__ inline uint32_t seg_isqrt(uint32_t x) {
+    uint32_t r = 0;
+    for (uint32_t b = 1u << 15; b; b >>= 1)
+        if ((uint64_t)(r | b) * (r | b) <= x) r |= b;
+    return r;
+}
+__host__ __device__ inline uint32_t seg_split(uint32_t nblk, uint32_t L, uint32_t &len) {
+    len = nblk;
+    if (!L) return 1;
+    uint32_t s = (nblk + L - 1) / L;
+    const uint32_t most = seg_isqrt(nblk);
+    if (s > most) s = most;
+    if (s < 3) return 1;
+    len = (nblk + s - 1) / s;
+    return (nblk + len - 1) / len;
+}
+// Time of a block of a chain that has its CU to itself, about 0.5 us (2.4 us
+// at K = 1,000, 4.3 at 3,000, 6.7 at 10,000), and a chain's latency and work
+// (one direction) in these units.
+__host__ __device__ inline uint64_t seg_block_cost(uint32_t Kpad) { return 4 + Kpad / 1024; }
+__host__ __device__ inline uint64_t seg_path(uint32_t nblk, uint32_t S, uint32_t len, uint32_t Kpad) {
+    return seg_block_cost(Kpad) * (S > 1 ? 2 * ((uint64_t)len + S) : nblk);
+}
+__host__ __device__ inline uint64_t seg_work(uint32_t nblk, uint32_t S, uint32_t Kpad) {
+    return seg_block_cost(Kpad) * (S > 1 ? 3 * (uint64_t)nblk + 2 * S : nblk);
+}
+// Expected time of a batch's chains for candidate L: the longest chain, or all
+// work over par / 10 chains' worth of parallel work.
+__host__ __device__ inline uint64_t seg_time(uint64_t path, uint64_t work, uint32_t par) {
+    const uint64_t w = 20 * work / par;
+    return path > w ? path : w;
+}
+// candidates: segments of 4 << c blocks, c < kSegCands, and none
+constexpr int kSegCands = 14;
+// uint16 words of a target's segments, both directions
+__host__ __device__ inline uint64_t seg_words(uint32_t S, uint32_t Kpad) {
+    return S > 1 ? 6ull * S * Kpad : 0ull;
+}
+// most segments of a batch (target, direction, segment)
+constexpr uint32_t kMaxSegments = 8192;
 
 // One item of the large-K PBWT kernel (order in global memory): one
 // direction of one target, or the panel PBWT.
@@ -136,7 +187,12 @@ struct PlanArgs {
     uint64_t *dig_base;    // 2 words per target
     uint32_t *blockpref;     // nmax + 1 prefix sums of cref blocks (gather targets)
     uint32_t *blockpref_id;  // nmax + 1 prefix sums of cref blocks (identity targets)
-    PbwtItem *pitems;        // 2 * nmax
+    OrderItem *rows_items;   // 2 * nmax + kMaxSegments
+    OrderItem *rank_items;   // 2 * kMaxSegments
+    OrderItem *comb_items;   // 2 * nmax
+    uint16_t *seg;           // seg_cap words for the segments of cut chains
+    uint64_t seg_cap;
+    uint32_t seg_par;        // chains' worth of parallel work, times 10
     uint32_t *rowpref;       // kRowsCounters, then nmax + 1 prefix sums of pbwt_blocks
     uint32_t layout;         // LAYOUT_*
     uint32_t digest;

@@ -1008,13 +1008,74 @@ __global__ __launch_bounds__(PLAN_NT) void k_plan(TgtDev *__restrict__ tg, Batch
         B->rr[1] = rri ? 1u : 0u;
         B->nrr[0] = (uint32_t)ng;
         B->nrr[1] = (uint32_t)ni;
-        B->npbwt = 2 * (uint32_t)nfit;
         B->nfit = (uint32_t)nfit;
         B->cref_ctr = 0;
         B->cref_id_ctr = 0;
         B->pbwt_ctr = 0;
     }
-    // PBWT items 2t (forward) and 2t+1 (backward), most work first:
+    // Chains: cut into segments where that shortens the batch.  Wave w works out
+    // the expected time of candidate w (the last one: no cut).
+    __shared__ uint32_t s_nb[PLAN_NT], s_kp[PLAN_NT];
+    __shared__ uint64_t s_time[kSegCands + 1];
+    __shared__ uint32_t s_L;
+    s_nb[t] = fit ? nblk : 0u;
+    s_kp[t] = Kpad;
+    __syncthreads();
+    {
+        const uint32_t w = t >> 6;
+        if (w <= (uint32_t)kSegCands) {
+            const uint32_t L = w < (uint32_t)kSegCands ? 4u << w : 0u;
+            uint64_t path = 0, work = 0, words = 0, segs = 0;
+            for (uint32_t i = t & 63; i < n; i += 64) {
+                const uint32_t nb = s_nb[i], kp = s_kp[i];
+                if (!nb) continue;
+                uint32_t len;
+                const uint32_t Sg = seg_split(nb, L, len);
+                const uint64_t p = seg_path(nb, Sg, len, kp);
+                path = p > path ? p : path;
+                work += seg_work(nb, Sg, kp);
+                words += seg_words(Sg, kp);
+                segs += Sg > 1 ? 2 * Sg : 0;
+            }
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                const uint64_t p = __shfl_xor(path, o);
+                path = p > path ? p : path;
+            }
+            work = wave_sum64(work);
+            words = wave_sum64(words);
+            segs = wave_sum64(segs);
+            if ((t & 63) == 0)
+                s_time[w] = words > A.seg_cap || segs > kMaxSegments ? ~0ull
+                                                                    : seg_time(path, work, A.seg_par);
+        }
+    }
+    __syncthreads();
+    if (t == 0) {
+        // the least expected time, the longer segments of equals; a cut must
+        // be worth a quarter (256 windowed targets: cut where a tenth was
+        // expected, 32.1 ms of chains, uncut 31.5)
+        int best = kSegCands;
+        for (int c = kSegCands - 1; c >= 0; c--)
+            if (s_time[c] < s_time[best] && s_time[c] != ~0ull &&
+                s_time[c] < s_time[kSegCands] - s_time[kSegCands] / 4)
+                best = c;
+        s_L = best < kSegCands ? 4u << best : 0u;
+    }
+    __syncthreads();
+    uint32_t seglen = nblk;
+    const uint32_t nseg = fit ? seg_split(nblk, s_L, seglen) : 1u;
+    uint64_t seg_tot;
+    const uint64_t seg_off = block_excl_scan64(fit ? seg_words(nseg, Kpad) : 0u, s_w, seg_tot);
+    if (valid) {
+        tg[t].nseg = nseg;
+        tg[t].seglen = seglen;
+        tg[t].seg = A.seg + seg_off;
+    }
+    __syncthreads();
+    s_nb[t] = nseg;  // now the segments of target t
+    s_kp[t] = seglen;
+    // PBWT chains 2t (forward) and 2t+1 (backward), most work first:
     // key = (~(Mp * Kpad) & 40 bits) << 24 | item; unused slots sort last
     const uint64_t wk = fit ? ((~((uint64_t)Mp * Kpad)) & 0xFFFFFFFFFFull) << 24 : ~0ull;
     keys[2 * t] = fit ? (wk | (2 * t)) : ~0ull;
@@ -1037,9 +1098,40 @@ __global__ __launch_bounds__(PLAN_NT) void k_plan(TgtDev *__restrict__ tg, Batch
             __syncthreads();
         }
     }
-    for (uint32_t i = t; i < 2 * (uint32_t)nfit; i += PLAN_NT) {
-        const uint32_t item = (uint32_t)(keys[i] & 0xFFFFFFu);
-        A.pitems[i] = PbwtItem{item >> 1, item & 1u};
+    // thread t writes the items of the sorted chains 2t and 2t + 1
+    uint32_t ch[2], cs[2];
+    uint64_t nr = 0, nk = 0, nc = 0;
+    for (uint32_t e = 0; e < 2; e++) {
+        const uint32_t i = 2 * t + e;
+        ch[e] = i < 2 * (uint32_t)nfit ? (uint32_t)(keys[i] & 0xFFFFFFu) : ~0u;
+        cs[e] = ch[e] != ~0u ? s_nb[ch[e] >> 1] : 0u;
+        nr += cs[e];
+        nk += cs[e] > 1 ? 2 * (cs[e] - 1) : 0;
+        nc += cs[e] > 1 ? 1 : 0;
+    }
+    uint64_t nr_tot, nk_tot, nc_tot;
+    uint64_t r0 = block_excl_scan64(nr, s_w, nr_tot), k0 = block_excl_scan64(nk, s_w, nk_tot),
+             c0 = block_excl_scan64(nc, s_w, nc_tot);
+    for (uint32_t e = 0; e < 2; e++) {
+        if (ch[e] == ~0u) continue;
+        const uint32_t tt = ch[e] >> 1, dir = ch[e] & 1u, len = s_kp[tt];
+        const uint32_t nb = (tg[tt].Mp + 15) / 16;
+        for (uint32_t s = 0; s < cs[e]; s++) {
+            const uint32_t q0 = s * len, q1 = min(nb, q0 + len);
+            A.rows_items[r0++] = OrderItem{tt, dir, CHAIN_ROWS, s, q0, q1};
+            if (s + 1 < cs[e]) {
+                A.rank_items[k0++] = OrderItem{tt, dir, CHAIN_RANK_UP, s, q0, q1};
+                A.rank_items[k0++] = OrderItem{tt, dir, CHAIN_RANK_DOWN, s, q0, q1};
+            }
+        }
+        if (cs[e] > 1) A.comb_items[c0++] = OrderItem{tt, dir, CHAIN_COMBINE, 0, 0, cs[e]};
+    }
+    if (t == 0) {
+        B->npbwt = (uint32_t)nr_tot;
+        B->nrank = (uint32_t)nk_tot;
+        B->ncomb = (uint32_t)nc_tot;
+        B->rank_ctr = 0;
+        B->comb_ctr = 0;
     }
 }
 

@@ -36,10 +36,10 @@ uint32_t pbwt_variant_maxk(int v);
 size_t pbwt_lds_bytes(int v, uint32_t Kpad);
 // occ (or null): resident workgroups per CU
 hipError_t pbwt_prepare(int v, size_t lds, int *occ);
-// chains: nitems workgroups, one item each, or with ctr taking items in turn
-// up to *d_items; starts: null, or the order at the start of every block of
-// the one chain (then no rows)
-hipError_t launch_order(int v, const TgtDev *tg, const PbwtItem *items, uint32_t nitems,
+// chain items (CHAIN_ROWS ones, or the other kinds): grid workgroups, one item
+// each, or with ctr taking items in turn up to *d_items; starts: for
+// CHAIN_STARTS items
+hipError_t launch_order(int v, const TgtDev *tg, const OrderItem *items, bool rows, uint32_t grid,
                         const uint32_t *d_items, uint32_t *ctr, uint16_t *starts, size_t lds,
                         hipStream_t s);
 // the rows of one forward chain from the starts, and the order after each

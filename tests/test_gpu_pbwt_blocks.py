@@ -61,3 +61,26 @@ def test_panel_pbwt_blocks(built, N, n):
         if absperm:
             assert np.array_equal(ap, want[2])
     eng.close()
+
+
+@pytest.mark.parametrize("N,F,flip,K", [(300, 3, 0.0, 300), (300, 3, 0.0, 77), (1500, 40, 0.001, 1300),
+                                        (2200, 30, 0.0, 2112)])
+def test_cut_chains(built, N, F, flip, K):
+    """Few long chains are cut into segments: haplotypes that a segment does
+    not tell apart (without flips whole classes are equal), padded and full K,
+    the synchronous call, a stream context and the panel's chain."""
+    M = 5000
+    panel = synth.make_panel(54, N=N, M=M, F=F, T=2, flip_rate=flip)
+    tg = synth.make_targets(panel, 54, 2, K=K, wmin=M - 300, wmax=M, miss=0.01)
+    res = _check(panel, tg, tg.K, "compact", f"cut N {N} F {F}")
+    eng = panel_engine(panel, give_hap=True)
+    st = eng.stream(2, M, K, 256 << 20)
+    st.submit(tg.gt, tg.s0, tg.W, tg.K)
+    got, nd, _ = st.wait()
+    assert nd == 0 and np.array_equal(got.dig_pbwt, res.dig_pbwt)
+    assert np.array_equal(got.dig_count0, res.dig_count0)
+    st.close()
+    rows, c0, ap, _ = eng.ref_pbwt(7, M - 40)
+    want = oracle.build_ref_pbwt(np.ascontiguousarray(panel.site[7:7 + M - 40]), N)
+    assert np.array_equal(rows, want[0]) and np.array_equal(c0, want[1]) and np.array_equal(ap, want[2])
+    eng.close()
