@@ -280,6 +280,9 @@ int ensure_pmono(eimp_engine *e) {
     return e->sync();
 }
 
+// subset cref items that fill the device: four workgroups per CU
+uint32_t cref_want(const eimp_engine *e) { return 4 * e->ncu; }
+
 // chains' worth of parallel work on the device, times 10: a further workgroup
 // on a CU adds about 0.2 of the first (384 chains of 941 blocks on 256 CUs take
 // 9.3 ms at K = 10,000, one alone 6.3)
@@ -477,6 +480,8 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
     uint32_t Kmax_pad = 0, Kmax = 0, Kbig = 0;
     std::vector<CrefItem> citems, citems_id;  // general / identity targets
     std::vector<uint32_t> chains;             // targets of the chain kernel
+    std::vector<uint32_t> subset;             // targets of the subset cref kernel
+    uint32_t n128 = 0;
     std::vector<uint32_t> big;                // targets beyond the LDS-resident PBWT kernels
     uint32_t lds_cap = 0;
     for (int v = 0; v < pbwt_variant_count(); v++) lds_cap = std::max(lds_cap, pbwt_variant_maxk(v));
@@ -492,10 +497,10 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
         const bool ident = (T.flags & TF_IDENTITY) && e->Nad <= 2ull * 256 * 64;
         if (!ident) Kmax = std::max(Kmax, T.K);
         if (ident) {
-            for (uint32_t b = 0; b < nblk; b++) citems_id.push_back(CrefItem{t, b, b + 1, 0});
+            for (uint32_t b = 0; b < nblk; b++) citems_id.push_back(CrefItem{t, b, b + 1, 0, 0});
         } else {
-            for (uint32_t b = 0; b < nblk; b += kCrefGroup)
-                citems.push_back(CrefItem{t, b, (uint32_t)std::min<uint64_t>(nblk, b + kCrefGroup), 0});
+            subset.push_back(t);
+            n128 += (uint32_t)((nblk + kCrefGroup - 1) / kCrefGroup);
         }
         if (T.Kpad > lds_cap) {
             // order in global memory: rows of K bits, two orders of Kpad per direction
@@ -516,6 +521,15 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
         }
         rowpref[kRowsCounters + t + 1] =
             rowpref[kRowsCounters + t] + (T.Kpad > lds_cap ? 0u : pbwt_blocks(T.Mp));
+    }
+    uint32_t cgrp = 1, cparts = 1;
+    cref_cut(n128, Kmax, cref_want(e), cgrp, cparts);
+    for (uint32_t t : subset) {
+        const uint32_t nblk = (tg[t].Mp + 15) / 16, passes = (tg[t].K + kCrefThreads - 1) / kCrefThreads;
+        const uint32_t per = (passes + cparts - 1) / cparts;
+        for (uint32_t b = 0; b < nblk; b += cgrp)
+            for (uint32_t p = 0; p < passes; p += per)
+                citems.push_back(CrefItem{t, b, std::min(nblk, b + cgrp), p, std::min(passes, p + per)});
     }
     // the subset cref kernel reads the haplotype-major panel (the drop-in's
     // initialize uploads only the site-major one: transposed here, once)
@@ -869,7 +883,7 @@ int run_batch_impl(eimp_engine *e, size_t n, const eimp_target *targets, float c
     HIPCHK(launch_select(e->pd, d_tg, nt, e->stream));
     e->tend(ti);
     ti = e->tbegin(EIMP_KCLASS_MONOS);
-    HIPCHK(launch_monos(e->pd, d_tg, d_mono_list, (uint32_t)mono_list.size(), max_ww, e->stream));
+    HIPCHK(launch_monos(e->pd, d_tg, d_mono_list, (uint32_t)mono_list.size(), max_ww, e->ncu, e->stream));
     e->tend(ti);
     ti = e->tbegin(EIMP_KCLASS_SPLITS);
     HIPCHK(launch_splits(e->pd, d_tg, nt, e->stream));
@@ -980,7 +994,7 @@ int stream_launch_prep(eimp_stream *s) {
     const uint32_t *d_n = &s->d_batch()->n;
     for (int cls = EIMP_KCLASS_DISTANCE; cls <= EIMP_KCLASS_SPLITS; cls++) {
         if (s->timed) HIPCHK(hipEventRecord(s->kev[cls], s->stream));
-        HIPCHK(launch_prep_dev(cls, e->pd, s->d_tg(), d_n, s->nmax, s->max_ww, s->stream));
+        HIPCHK(launch_prep_dev(cls, e->pd, s->d_tg(), d_n, s->nmax, s->max_ww, e->ncu, s->stream));
     }
     if (s->timed) HIPCHK(hipEventRecord(s->kev_prep_end, s->stream));
     return EIMP_OK;
@@ -1003,6 +1017,7 @@ int stream_launch_build(eimp_stream *s) {
     A.seg = s->d_seg.as<uint16_t>();
     A.seg_cap = s->seg_bytes / 2;
     A.seg_par = s->seg_par;
+    A.cref_want = cref_want(e);
     A.rowpref = s->d_rowpref.as<uint32_t>();
     A.layout = batch_layout(s->flags);
     A.digest = (s->flags & EIMP_BATCH_DIGEST) ? 1u : 0u;

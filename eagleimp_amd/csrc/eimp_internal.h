@@ -91,17 +91,42 @@ struct BatchDev {
     // in blockpref (item i = block i / nrr of target i % nrr)
     uint32_t rr[2];
     uint32_t nrr[2];
+    // subset cref items: blocks of a group, parts of the haplotypes, passes of a part
+    uint32_t cref_grp, cref_parts, cref_per;
     // chain items of cut chains: ranks of the segments, then their combination
     uint32_t nrank, rank_ctr, ncomb, comb_ctr;
 };
 
-// 16-row blocks per work item of the subset cref kernel (256 splits)
+// 16-row blocks per work item of the subset cref kernel in a full batch
 constexpr uint32_t kCrefGroup = 128;
+constexpr uint32_t kCrefThreads = 256;
 
-// cref work item: target t, blocks [b0, b1)
+// cref work item: target t, blocks [b0, b1), passes [p0, p1) of kCrefThreads
+// haplotypes
 struct CrefItem {
-    uint32_t t, b0, b1, pad;
+    uint32_t t, b0, b1, p0, p1;
 };
+
+// Cut of a batch's subset cref work (n128 groups of kCrefGroup blocks, up to K
+// haplotypes) into at least `want` items where it can be: first the
+// haplotypes into parts, then groups of 32 blocks.  A batch with that many
+// groups stays whole: smaller groups read more of each row's cache lines
+// twice (96 targets on the 200,000-haplotype panel: 3.5 ms whole).
+__host__ __device__ inline void cref_cut(uint32_t n128, uint32_t K, uint32_t want, uint32_t &grp,
+                                         uint32_t &parts) {
+    const uint32_t passes = (K + kCrefThreads - 1) / kCrefThreads;
+    grp = kCrefGroup;
+    parts = 1;
+    if (n128 >= want || !n128) return;
+    uint32_t groups = n128;
+    if ((uint64_t)n128 * passes < want) {
+        grp = 32;
+        groups = 4 * n128;
+    }
+    parts = (want + groups - 1) / groups;
+    if (parts > passes) parts = passes;
+    if (parts < 1) parts = 1;
+}
 
 // 16-row blocks of a target's PBWT, both directions
 __host__ __device__ inline uint32_t pbwt_blocks(uint32_t Mp) { return 2 * ((Mp + 15) / 16); }
@@ -192,6 +217,7 @@ struct PlanArgs {
     OrderItem *comb_items;   // 2 * nmax
     uint16_t *seg;           // seg_cap words for the segments of cut chains
     uint64_t seg_cap;
+    uint32_t cref_want;      // subset cref items that fill the device
     uint32_t seg_par;        // chains' worth of parallel work, times 10
     uint32_t *rowpref;       // kRowsCounters, then nmax + 1 prefix sums of pbwt_blocks
     uint32_t layout;         // LAYOUT_*

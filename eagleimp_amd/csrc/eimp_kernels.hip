@@ -16,6 +16,7 @@
 //   k_bits_to_list   bitmap -> ascending index list (drop-in inputs)
 //   k_cref           condensed reference in 16-row transposed blocks
 //                    (Target::condensedReferenceT, src/Target.cpp:953-1059)
+#include <algorithm>
 #include <map>
 #include <mutex>
 
@@ -316,15 +317,31 @@ __global__ __launch_bounds__(SEL_NT) void k_select(PanelDev P, const TgtDev *__r
         sel_before += scount;
     }
     if (tid == 0) T.stats[3] = sel_before;
+    // k_monos starts from these
+    if (!(T.flags & TF_IDENTITY)) {
+        for (uint32_t w = tid; w < (T.W + 63) / 64; w += SEL_NT) {
+            T.mand_w[w] = ~0ull;
+            T.mor_w[w] = 0ull;
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
-// a5: monos for targets that select a subset.  grid (ceil(Ww/64), n), block
-// MONO_NT: the waves split the K chosen rows, lanes cover 64 window words
-// (256 threads: they fit beside a PBWT workgroup, as the selection does).
+// a5: monos for targets that select a subset.  grid (ceil(Ww/64), n, parts),
+// block MONO_NT: the waves split the part's share of the K chosen rows, lanes
+// cover 64 window words (256 threads: they fit beside a PBWT workgroup, as the
+// selection does).  A few targets have few word groups, so their rows are cut
+// into parts (mono_parts) whose results meet in mand_w / mor_w by atomics; the
+// selection has set those to ones and zeros (4 targets of up to 30,000 sites
+// and 10,000 rows: 905 us in one part, 70 us in 16).
 // ---------------------------------------------------------------------------
 constexpr int MONO_NT = 256;
 constexpr int MONO_NW = MONO_NT / 64;
+// parts for a grid of `groups` workgroups per part
+static uint32_t mono_parts(uint64_t groups, uint32_t ncu) {
+    const uint64_t want = 4ull * ncu;
+    return groups * 2 > want ? 1u : (uint32_t)std::min<uint64_t>(32, want / std::max<uint64_t>(groups, 1));
+}
 
 __global__ __launch_bounds__(MONO_NT) void k_monos(PanelDev P, const TgtDev *__restrict__ tg,
                                                    const uint32_t *__restrict__ tlist,
@@ -333,6 +350,9 @@ __global__ __launch_bounds__(MONO_NT) void k_monos(PanelDev P, const TgtDev *__r
     if (!tlist && blockIdx.y >= *d_n) return;
     const TgtDev &T = tg[tlist ? tlist[blockIdx.y] : blockIdx.y];
     if (T.flags & TF_IDENTITY) return;
+    const uint32_t per = (T.K + gridDim.z - 1) / gridDim.z;
+    const uint32_t k0 = blockIdx.z * per, kend = min(T.K, k0 + per);
+    if (k0 >= kend || (uint64_t)blockIdx.x * 64 * 64 >= T.W) return;
     __shared__ uint64_t s_and[MONO_NW][64], s_or[MONO_NW][64];
     const uint32_t wave = threadIdx.x >> 6, l = lane_id();
     const uint64_t Ww = (T.W + 63) / 64;
@@ -341,8 +361,8 @@ __global__ __launch_bounds__(MONO_NT) void k_monos(PanelDev P, const TgtDev *__r
     uint64_t a = ~0ull, o = 0ull;
     const uint64_t bitoff = T.s0 + 64 * i;
     if (valid) {
-        uint32_t k = wave;
-        for (; k + 3 * MONO_NW < T.K; k += 4 * MONO_NW) {
+        uint32_t k = k0 + wave;
+        for (; k + 3 * MONO_NW < kend; k += 4 * MONO_NW) {
             uint64_t v0 = funnel(P.hap + (uint64_t)T.bh[k] * P.hap_stride, bitoff, P.hap_stride);
             uint64_t v1 = funnel(P.hap + (uint64_t)T.bh[k + MONO_NW] * P.hap_stride, bitoff,
                                  P.hap_stride);
@@ -353,7 +373,7 @@ __global__ __launch_bounds__(MONO_NT) void k_monos(PanelDev P, const TgtDev *__r
             a &= v0 & v1 & v2 & v3;
             o |= v0 | v1 | v2 | v3;
         }
-        for (; k < T.K; k += MONO_NW) {
+        for (; k < kend; k += MONO_NW) {
             uint64_t v = funnel(P.hap + (uint64_t)T.bh[k] * P.hap_stride, bitoff, P.hap_stride);
             a &= v;
             o |= v;
@@ -367,8 +387,13 @@ __global__ __launch_bounds__(MONO_NT) void k_monos(PanelDev P, const TgtDev *__r
             a &= s_and[w][l];
             o |= s_or[w][l];
         }
-        T.mand_w[i] = a;
-        T.mor_w[i] = o;
+        if (gridDim.z == 1) {
+            T.mand_w[i] = a;
+            T.mor_w[i] = o;
+        } else {
+            atomicAnd((unsigned long long *)&T.mand_w[i], (unsigned long long)a);
+            atomicOr((unsigned long long *)&T.mor_w[i], (unsigned long long)o);
+        }
     }
 }
 
@@ -551,12 +576,14 @@ __global__ __launch_bounds__(SEL_NT) void k_bits_to_list(const TgtDev *__restric
 //    one block, its rows built in LDS from the site-major panel (every thread
 //    streaming two words through all the block's site rows, 8 independent
 //    loads in flight) and transposed in registers;
-//  - the others: one work item = CREF_G blocks, from the haplotype-major
-//    panel, reading only the K chosen rows.
+//  - the others: one work item = a group of blocks and a range of the chosen
+//    haplotypes, from the haplotype-major panel, reading only the K chosen
+//    rows.  A batch that fills the device takes groups of 128 blocks and all
+//    haplotypes in one item (neighbouring groups share cache lines of the
+//    rows); one that does not is cut finer (cref_cut).
 // count0 (zeros per row) is written by the forward PBWT pass.
 // ---------------------------------------------------------------------------
-constexpr int CREF_NT = 256;
-constexpr uint32_t CREF_G = kCrefGroup;  // blocks per work item of the subset kernel
+constexpr int CREF_NT = (int)kCrefThreads;
 constexpr uint32_t CREF_TW = 512;  // words of the haplotype axis per tile (16 rows: 64 KB)
 
 __host__ __device__ inline uint32_t cref_tile_words(uint32_t nw) {
@@ -633,8 +660,9 @@ __device__ __forceinline__ void cref_fill(const PanelDev &P, const TgtDev &T, ui
     }
 }
 
-// Blocks [b0, b1) of a subset target from the haplotype-major panel.  Thread
-// x takes the chosen haplotypes k = x, x + CREF_NT, ... and streams each one's
+// Blocks [b0, b1) of a subset target from the haplotype-major panel, passes
+// [p0, p1) of CREF_NT haplotypes: thread x takes the chosen haplotypes k = x +
+// CREF_NT p and streams each one's
 // row over the sites of the blocks, 32 window sites per step:
 //   inc = (v & HomRef) | (~v & HomAlt)  (HomRef = is0 & ~is2, HomAlt =
 //                                        is2 & ~is0; split sites and sites
@@ -651,7 +679,7 @@ __device__ __forceinline__ void cref_fill(const PanelDev &P, const TgtDev &T, ui
 // would need all N bits of every site).  Haplotypes K..Kpad-1 get all-ones
 // values (the PBWT kernel's padding); count0 comes from the PBWT kernel.
 __device__ __forceinline__ void cref_range_hap(const PanelDev &P, const TgtDev &T, uint32_t b0,
-                                               uint32_t b1) {
+                                               uint32_t b1, uint32_t p0, uint32_t p1) {
     const uint32_t tid = threadIdx.x;
     const uint32_t K = T.K, S = T.S, Kpad = T.Kpad, W = T.W;
     const bool ident = (T.flags & TF_IDENTITY) != 0;
@@ -667,13 +695,14 @@ __device__ __forceinline__ void cref_range_hap(const PanelDev &P, const TgtDev &
     const uint32_t m0 = sa == 0 ? 0u : splitsites[sa - 1] + 1;
     const uint32_t m1 = last ? W : splitsites[sb - 1] + 1;
     const uint32_t i0 = m0 >> 5, i1 = (m1 + 31) >> 5;  // 32-site window words
-    for (uint32_t k = K + tid; k < Kpad; k += CREF_NT)
-        for (uint32_t b = b0; b < b1; b++) dst[(uint64_t)b * Kpad + k] = 0xFFFFu;
+    if (p0 == 0)
+        for (uint32_t k = K + tid; k < Kpad; k += CREF_NT)
+            for (uint32_t b = b0; b < b1; b++) dst[(uint64_t)b * Kpad + k] = 0xFFFFu;
     // window word i of a row = bits sh.. of row words q0 + i, q0 + i + 1
     const uint64_t rowlen = 2 * P.hap_stride;  // uint32 words per haplotype row
     const uint64_t q0 = T.s0 >> 5;
     const uint32_t sh = (uint32_t)T.s0 & 31;
-    for (uint32_t kb = 0; kb < K; kb += CREF_NT) {
+    for (uint32_t kb = p0 * CREF_NT; kb < min(K, p1 * CREF_NT); kb += CREF_NT) {
         const uint32_t k = kb + tid;
         const bool act = k < K;
         const uint32_t h = act ? (ident ? k : bh[k]) : 0u;
@@ -844,7 +873,7 @@ __device__ __forceinline__ void cref_block_ident(const PanelDev &P, const TgtDev
 __global__ __launch_bounds__(CREF_NT) void k_cref(PanelDev P, const TgtDev *__restrict__ tg,
                                                  const CrefItem *__restrict__ items) {
     const CrefItem it = items[blockIdx.x];
-    cref_range_hap(P, tg[it.t], it.b0, it.b1);
+    cref_range_hap(P, tg[it.t], it.b0, it.b1, it.p0, it.p1);
 }
 
 template <int GPT>
@@ -994,9 +1023,14 @@ __global__ __launch_bounds__(PLAN_NT) void k_plan(TgtDev *__restrict__ tg, Batch
     // panel rows at the same time, from the cache.
     const bool idk = fit && A.ident_ok && (tg[t].flags & TF_IDENTITY);
     const bool gk = fit && !idk;
-    // subset targets are queued in items of CREF_G blocks
-    const uint32_t ngrp = (nblk + CREF_G - 1) / CREF_G;
-    uint64_t nb_tot, nb_id, ng, ni, mxg, mxi;
+    // subset targets are queued in items of a group of blocks and a part of the
+    // haplotypes, cut alike for the batch
+    uint64_t nb128, nb_tot, nb_id, ng, ni, mxg, mxi;
+    (void)block_excl_scan64(gk ? (nblk + kCrefGroup - 1) / kCrefGroup : 0u, s_w, nb128);
+    const uint32_t Kg = (uint32_t)block_max64(gk ? K : 0u, s_w);
+    uint32_t grp, parts;
+    cref_cut((uint32_t)nb128, Kg, A.cref_want, grp, parts);
+    const uint32_t ngrp = (nblk + grp - 1) / grp;
     const uint64_t bp = block_excl_scan64(gk ? ngrp : 0u, s_w, nb_tot);
     const uint64_t bpi = block_excl_scan64(idk ? nblk : 0u, s_w, nb_id);
     const uint64_t pg = block_excl_scan64(gk ? 1u : 0u, s_w, ng);
@@ -1026,7 +1060,10 @@ __global__ __launch_bounds__(PLAN_NT) void k_plan(TgtDev *__restrict__ tg, Batch
     if (t == 0) {
         if (!rrg) A.blockpref[n] = (uint32_t)nb_tot;
         if (!rri) A.blockpref_id[n] = (uint32_t)nb_id;
-        B->ncref = (uint32_t)(rrg ? ng * mxg : nb_tot);
+        B->ncref = (uint32_t)(rrg ? ng * mxg : nb_tot) * parts;
+        B->cref_grp = grp;
+        B->cref_parts = parts;
+        B->cref_per = ((Kg + CREF_NT - 1) / CREF_NT + parts - 1) / parts;
         B->ncref_id = (uint32_t)(rri ? ni * mxi : nb_id);
         B->rr[0] = rrg ? 1u : 0u;
         B->rr[1] = rri ? 1u : 0u;
@@ -1159,18 +1196,18 @@ __global__ __launch_bounds__(PLAN_NT) void k_plan(TgtDev *__restrict__ tg, Batch
     }
 }
 
-// next cref item from a queue: queue position i (i >= nq ends), target t,
+// next cref item from a queue of nq, `parts` to an entry: position i (i >= nq ends), target t,
 // item b of t (items of `unit` 16-row blocks); b = ~0u for an empty item of a
 // block-major queue
-__device__ __forceinline__ void cref_pop(uint32_t *ctr, uint32_t nq, uint32_t n, uint32_t rr,
-                                         uint32_t nrr, const TgtDev *__restrict__ tg,
+__device__ __forceinline__ void cref_pop(uint32_t *ctr, uint32_t nq, uint32_t parts, uint32_t n,
+                                         uint32_t rr, uint32_t nrr, const TgtDev *__restrict__ tg,
                                          const uint32_t *__restrict__ pref, uint32_t unit,
                                          uint32_t &i, uint32_t &t, uint32_t &b) {
     __shared__ uint32_t s_i, s_t, s_b;
     if (threadIdx.x == 0) {
-        const uint32_t ii = atomicAdd(ctr, 1u);
+        const uint32_t at = atomicAdd(ctr, 1u), ii = at / parts;
         uint32_t tt = 0, bb = 0;
-        if (ii < nq) {
+        if (at < nq) {
             if (rr) {  // block-major: block ii / nrr of the (ii % nrr)-th listed target
                 tt = pref[ii % nrr];
                 bb = ii / nrr;
@@ -1185,7 +1222,7 @@ __device__ __forceinline__ void cref_pop(uint32_t *ctr, uint32_t nq, uint32_t n,
                 bb = ii - pref[lo];
             }
         }
-        s_i = ii;
+        s_i = at;
         s_t = tt;
         s_b = bb;
     }
@@ -1198,18 +1235,20 @@ __device__ __forceinline__ void cref_pop(uint32_t *ctr, uint32_t nq, uint32_t n,
     __syncthreads();
 }
 
-// cref items (CREF_G blocks) of subset targets from their queue
+// cref items of subset targets from their queue: entry i / parts of the queue
+// of block groups, part i % parts of the haplotypes
 __global__ __launch_bounds__(CREF_NT) void k_cref_persist(PanelDev P, const TgtDev *__restrict__ tg,
                                                          BatchDev *__restrict__ B,
                                                          const uint32_t *__restrict__ blockpref) {
     const uint32_t nq = B->ncref, n = B->n, rr = B->rr[0], nrr = B->nrr[0];
+    const uint32_t grp = B->cref_grp, parts = B->cref_parts, per = B->cref_per;
     for (;;) {
         uint32_t i, t, g;
-        cref_pop(&B->cref_ctr, nq, n, rr, nrr, tg, blockpref, CREF_G, i, t, g);
+        cref_pop(&B->cref_ctr, nq, parts, n, rr, nrr, tg, blockpref, grp, i, t, g);
         if (i >= nq) break;
         if (g != ~0u) {
-            const uint32_t nblk = (tg[t].Mp + 15) / 16;
-            cref_range_hap(P, tg[t], g * CREF_G, min(nblk, (g + 1) * CREF_G));
+            const uint32_t nblk = (tg[t].Mp + 15) / 16, part = i % parts;
+            cref_range_hap(P, tg[t], g * grp, min(nblk, (g + 1) * grp), part * per, (part + 1) * per);
         }
     }
 }
@@ -1224,7 +1263,7 @@ __global__ __launch_bounds__(CREF_NT, 4) void k_cref_persist_ident(PanelDev P,
     const uint32_t nq = B->ncref_id, n = B->n, rr = B->rr[1], nrr = B->nrr[1];
     for (;;) {
         uint32_t i, t, b;
-        cref_pop(&B->cref_id_ctr, nq, n, rr, nrr, tg, blockpref, 1u, i, t, b);
+        cref_pop(&B->cref_id_ctr, nq, 1u, n, rr, nrr, tg, blockpref, 1u, i, t, b);
         if (i >= nq) break;
         if (b != ~0u) cref_block_ident<GPT>(P, tg[t], b, srow);
     }
@@ -1326,9 +1365,10 @@ hipError_t launch_select(const PanelDev &P, const TgtDev *tg, uint32_t n, hipStr
     return hipGetLastError();
 }
 hipError_t launch_monos(const PanelDev &P, const TgtDev *tg, const uint32_t *tlist, uint32_t n,
-                        uint32_t max_ww, hipStream_t s) {
+                        uint32_t max_ww, uint32_t ncu, hipStream_t s) {
     if (!n) return hipSuccess;
-    hipLaunchKernelGGL(k_monos, dim3((max_ww + 63) / 64, n), dim3(MONO_NT), 0, s, P, tg, tlist,
+    const uint32_t gx = (max_ww + 63) / 64;
+    hipLaunchKernelGGL(k_monos, dim3(gx, n, mono_parts((uint64_t)gx * n, ncu)), dim3(MONO_NT), 0, s, P, tg, tlist,
                        (const uint32_t *)nullptr);
     return hipGetLastError();
 }
@@ -1406,7 +1446,7 @@ hipError_t launch_site_blocks(const PanelDev &P, uint64_t m0, uint32_t nsites, u
 // Prep phase over a batch of *d_n <= nmax targets, one kernel class per call
 // (0 distances, 1 top-K, 2 monos, 3 split sites); grids cover nmax targets.
 hipError_t launch_prep_dev(int cls, const PanelDev &P, const TgtDev *tg, const uint32_t *d_n,
-                           uint32_t nmax, uint32_t max_ww, hipStream_t s) {
+                           uint32_t nmax, uint32_t max_ww, uint32_t ncu, hipStream_t s) {
     switch (cls) {
     case 0:
         hipLaunchKernelGGL(k_distance, dim3((P.N_ad + 15) / 16, (nmax + DIST_G - 1) / DIST_G),
@@ -1416,7 +1456,9 @@ hipError_t launch_prep_dev(int cls, const PanelDev &P, const TgtDev *tg, const u
         hipLaunchKernelGGL(k_select, dim3(nmax), dim3(SEL_NT), 0, s, P, tg, d_n);
         break;
     case 2:
-        hipLaunchKernelGGL(k_monos, dim3((max_ww + 63) / 64, nmax), dim3(MONO_NT), 0, s, P, tg,
+        hipLaunchKernelGGL(k_monos,
+                           dim3((max_ww + 63) / 64, nmax, mono_parts((uint64_t)((max_ww + 63) / 64) * nmax, ncu)),
+                           dim3(MONO_NT), 0, s, P, tg,
                            (const uint32_t *)nullptr, d_n);
         break;
     default:

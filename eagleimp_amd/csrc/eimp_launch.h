@@ -14,7 +14,7 @@ hipError_t launch_distance(const PanelDev &P, const TgtDev *tg, const uint32_t *
                            uint32_t nsel, hipStream_t s);
 hipError_t launch_select(const PanelDev &P, const TgtDev *tg, uint32_t n, hipStream_t s);
 hipError_t launch_monos(const PanelDev &P, const TgtDev *tg, const uint32_t *tlist, uint32_t n,
-                        uint32_t max_ww, hipStream_t s);
+                        uint32_t max_ww, uint32_t ncu, hipStream_t s);
 hipError_t launch_splits(const PanelDev &P, const TgtDev *tg, uint32_t n, hipStream_t s);
 hipError_t launch_bits_to_list(const TgtDev *tg, uint32_t n, uint32_t nbits_bh, int which,
                                hipStream_t s);
@@ -52,7 +52,7 @@ hipError_t launch_rows(const TgtDev *tg, const uint32_t *d_n, uint32_t n, const 
                        RowItem *list, uint32_t *cnt, uint32_t Kpad, uint64_t blocks, uint32_t ncu,
                        hipStream_t s);
 hipError_t launch_prep_dev(int cls, const PanelDev &P, const TgtDev *tg, const uint32_t *d_n,
-                           uint32_t nmax, uint32_t max_ww, hipStream_t s);
+                           uint32_t nmax, uint32_t max_ww, uint32_t ncu, hipStream_t s);
 hipError_t launch_plan(TgtDev *tg, BatchDev *B, const PlanArgs &A, hipStream_t s);
 hipError_t launch_digest_count0_dev(const TgtDev *tg, const uint32_t *d_n, uint32_t nmax,
                                     hipStream_t s);
