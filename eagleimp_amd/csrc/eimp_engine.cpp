@@ -78,6 +78,13 @@ int auto_pbwt_variant(uint32_t Kpad) {
             best = v;
     return best;
 }
+// The shape with twice the threads of v where it moves a chain faster: K above
+// 2,048 (K = 3,001: 1.44 ms a call against 1.69; K = 1,000 gains nothing).
+int latency_variant(int v) {
+    return pbwt_variant_threads(v) == 256 && pbwt_variant_cpw(v) > 8 ? 2
+         : pbwt_variant_threads(v) == 512                            ? 4
+                                                                     : v;
+}
 inline uint64_t round_up(uint64_t n, uint64_t m) { return (n + m - 1) / m * m; }
 
 // Grow-only device buffer
@@ -171,9 +178,9 @@ struct eimp_engine {
     std::vector<hipEvent_t> event_pool;
     int pbwt_variant = -1;
     uint64_t panel_gen = 0;  // bumped whenever panel buffers change (stream contexts check it)
-    int pbwt_prepared_variant = -1;
-    size_t pbwt_prepared_lds = 0;
-    int pbwt_prepared_occ = 1;  // resident workgroups per CU
+    // chain shapes: dynamic LDS they are prepared for, resident workgroups per CU
+    std::map<int, size_t> pbwt_lds_ready;
+    std::map<int, int> pbwt_occ;
     uint32_t ncu = 0;  // compute units
 
     hipEvent_t get_event() {
@@ -234,6 +241,19 @@ struct eimp_engine {
         por.release();
         have_cM = have_hap = have_pmono = false;
     }
+    // Prepares shape v for chains of up to Kpad haplotypes; *lds: what they take.
+    int prepare_pbwt(int v, uint32_t Kpad, size_t *lds) {
+        *lds = pbwt_lds_bytes(v, Kpad);
+        if (*lds > 160 * 1024)
+            return fail(EIMP_ERR_UNSUPPORTED, "K beyond the PBWT kernel's slots or 160 KiB of LDS");
+        if (pbwt_lds_ready[v] < *lds) {
+            int occ = 1;
+            HIPCHK(pbwt_prepare(v, *lds, &occ));
+            pbwt_occ[v] = occ;
+            pbwt_lds_ready[v] = *lds;
+        }
+        return EIMP_OK;
+    }
     int choose_pbwt_variant(uint32_t Kmax_pad) {
         if (pbwt_variant >= 0) {
             if (pbwt_variant >= pbwt_variant_count()) return fail(EIMP_ERR_INVALID, "bad variant");
@@ -293,7 +313,7 @@ uint32_t seg_par(const eimp_engine *e, int occ) {
 // The segments of chains of nblk blocks (cut alike in both directions; Kpad
 // each): the candidate with the least expected time (as k_plan).  Returns L.
 uint32_t choose_segments(const std::vector<uint32_t> &nblk, const std::vector<uint32_t> &Kpad, uint32_t par,
-                         uint64_t cap_words, uint32_t max_segs) {
+                         uint64_t cap_words, uint32_t max_segs, uint32_t ncu, bool *latency_bound) {
     uint64_t t_none = 0, t_best = 0;
     uint32_t best = 0;
     for (int c = kSegCands; c >= 0; c--) {
@@ -310,9 +330,11 @@ uint32_t choose_segments(const std::vector<uint32_t> &nblk, const std::vector<ui
         const uint64_t t = seg_time(path, work, par);
         if (c == kSegCands) {
             t_none = t_best = t;
+            *latency_bound = seg_latency_bound(path, work, ncu);
         } else if (words <= cap_words && segs <= max_segs && t < t_best && t < t_none - t_none / 4) {
             t_best = t;
             best = L;
+            *latency_bound = seg_latency_bound(path, work, ncu);
         }
     }
     return best;
@@ -545,14 +567,7 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
     if (!chains.empty()) {
         v = e->choose_pbwt_variant(Kmax_pad);
         if (v < 0) return v;
-        lds = pbwt_lds_bytes(v, Kmax_pad);
-        if (lds > 160 * 1024)
-            return fail(EIMP_ERR_UNSUPPORTED, "K beyond the PBWT kernel's slots or 160 KiB of LDS");
-        if (e->pbwt_prepared_variant != v || e->pbwt_prepared_lds < lds) {
-            HIPCHK(pbwt_prepare(v, lds, &e->pbwt_prepared_occ));
-            e->pbwt_prepared_variant = v;
-            e->pbwt_prepared_lds = lds;
-        }
+        CHK(e->prepare_pbwt(v, Kmax_pad, &lds));
     }
     // chains longest first, cut into segments where that shortens the batch
     std::stable_sort(chains.begin(), chains.end(), [&](uint32_t a, uint32_t b) { return tg[a].Mp > tg[b].Mp; });
@@ -565,7 +580,13 @@ int run_build(eimp_engine *e, uint32_t n, bool digest, uint32_t layout, BatchMem
             nb.push_back((tg[t].Mp + 15) / 16);
             kp.push_back(tg[t].Kpad);
         }
-        const uint32_t L = choose_segments(nb, kp, seg_par(e, e->pbwt_prepared_occ), mem.seg_room() / 2, ~0u);
+        bool latency = false;
+        const uint32_t L = choose_segments(nb, kp, seg_par(e, e->pbwt_occ[v]), mem.seg_room() / 2, ~0u, e->ncu,
+                                           &latency);
+        if (latency && e->pbwt_variant < 0 && latency_variant(v) != v) {
+            v = latency_variant(v);
+            CHK(e->prepare_pbwt(v, Kmax_pad, &lds));
+        }
         for (size_t i = 0; i < chains.size(); i++) {
             TgtDev &T = tg[chains[i]];
             T.nseg = seg_split(nb[i], L, T.seglen);
@@ -960,9 +981,10 @@ struct eimp_stream {
     uint64_t tab_off = 0, gt_off = 0, gt_cap_words = 0;
     HostBuf h_in, h_out;  // h_out = stats | digests | TgtDev table
     // launch configuration
-    int pbwt_v = -1;
-    size_t pbwt_lds = 0;
-    uint32_t cref_grid[2] = {0, 0}, pbwt_grid = 0, seg_par = 0;
+    // chain shapes: the throughput one, and the latency one or -1
+    int pbwt_v[2] = {-1, -1};
+    size_t pbwt_lds[2] = {0, 0};
+    uint32_t cref_grid[2] = {0, 0}, pbwt_grid[2] = {0, 0}, seg_par = 0;
     uint64_t seg_bytes = 0;
     hipGraph_t graph_prep = nullptr, graph_build = nullptr;
     hipGraphExec_t exec_prep = nullptr, exec_build = nullptr;
@@ -1018,6 +1040,8 @@ int stream_launch_build(eimp_stream *s) {
     A.seg_cap = s->seg_bytes / 2;
     A.seg_par = s->seg_par;
     A.cref_want = cref_want(e);
+    A.ncu = e->ncu;
+    A.shapes = s->pbwt_v[1] >= 0 ? 2u : 1u;
     A.rowpref = s->d_rowpref.as<uint32_t>();
     A.layout = batch_layout(s->flags);
     A.digest = (s->flags & EIMP_BATCH_DIGEST) ? 1u : 0u;
@@ -1034,12 +1058,15 @@ int stream_launch_build(eimp_stream *s) {
     CHK(mark(EIMP_KCLASS_PBWT));
     const uint32_t Kpad = (uint32_t)round_up(s->Kmax, 64);
     BatchDev *B = s->d_batch();
-    HIPCHK(launch_order(s->pbwt_v, s->d_tg(), A.rank_items, false, s->pbwt_grid, &B->nrank, &B->rank_ctr,
-                        nullptr, s->pbwt_lds, s->stream));
-    HIPCHK(launch_order(s->pbwt_v, s->d_tg(), A.comb_items, false, s->pbwt_grid, &B->ncomb, &B->comb_ctr,
-                        nullptr, s->pbwt_lds, s->stream));
-    HIPCHK(launch_order(s->pbwt_v, s->d_tg(), A.rows_items, true, s->pbwt_grid, &B->npbwt, &B->pbwt_ctr,
-                        nullptr, s->pbwt_lds, s->stream));
+    for (int v = 0; v < (int)A.shapes; v++) {
+        auto run = [&](const OrderItem *items, bool rows, const uint32_t *count, uint32_t *ctr) {
+            return launch_order(s->pbwt_v[v], s->d_tg(), items, rows, s->pbwt_grid[v], count, ctr, nullptr,
+                                s->pbwt_lds[v], s->stream);
+        };
+        HIPCHK(run(A.rank_items, false, &B->nrank[v], &B->rank_ctr[v]));
+        HIPCHK(run(A.comb_items, false, &B->ncomb[v], &B->comb_ctr[v]));
+        HIPCHK(run(A.rows_items, true, &B->npbwt[v], &B->pbwt_ctr[v]));
+    }
     HIPCHK(launch_rows(s->d_tg(), d_n, 0, A.rowpref + kRowsCounters, s->d_rowlist.as<RowItem>(),
                        A.rowpref, Kpad, (uint64_t)s->nmax * pbwt_blocks(2 * s->Wmax + 1), e->ncu,
                        s->stream));
@@ -1147,17 +1174,17 @@ int stream_setup(eimp_stream *s, size_t pool_bytes, const std::shared_ptr<Stream
     if (s->Kmax > cref_max_k()) return fail(EIMP_ERR_UNSUPPORTED, "K beyond the cref kernel limit");
     if (cref_lds_bytes(e->pd, s->Kmax) > 160 * 1024)
         return fail(EIMP_ERR_UNSUPPORTED, "panel too wide for the cref kernel's LDS staging");
-    int v = e->choose_pbwt_variant(Kpad);
+    const int v = e->choose_pbwt_variant(Kpad);
     if (v < 0) return v;
-    const size_t lds = pbwt_lds_bytes(v, Kpad);
-    if (lds > 160 * 1024)
-        return fail(EIMP_ERR_UNSUPPORTED, "K beyond the PBWT kernel's slots or 160 KiB of LDS");
-    s->pbwt_v = v;
-    s->pbwt_lds = lds;
+    s->pbwt_v[0] = v;
+    CHK(e->prepare_pbwt(v, Kpad, &s->pbwt_lds[0]));
+    if (e->pbwt_variant < 0 && latency_variant(v) != v) {
+        s->pbwt_v[1] = latency_variant(v);
+        CHK(e->prepare_pbwt(s->pbwt_v[1], Kpad, &s->pbwt_lds[1]));
+    }
     const int ncu = (int)e->ncu;
-    int occ_c[2] = {0, 0}, occ_p = 0;
+    int occ_c[2] = {0, 0};
     HIPCHK(cref_persist_prepare(e->pd, s->Kmax, occ_c));
-    HIPCHK(pbwt_prepare(v, lds, &occ_p));
     s->cref_grid[0] = (uint32_t)(std::max(ncu, 1) * std::max(occ_c[0], 1));
     // identity targets need K == N_ad
     const bool ident_possible = cref_ident_ok(e->pd) && s->Kmax == e->Nad && e->Ncorr == e->Nad;
@@ -1165,9 +1192,11 @@ int stream_setup(eimp_stream *s, size_t pool_bytes, const std::shared_ptr<Stream
     // one workgroup per CU, or per chain where there are more: workgroups beyond
     // the items take them first where they share a CU (192 targets on 768
     // workgroups 11.8 ms, on 384 8.7 ms)
-    s->pbwt_grid = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(2 * nmax, (uint64_t)ncu),
-                                                (uint64_t)ncu * (uint64_t)std::max(occ_p, 1));
-    s->seg_par = seg_par(e, occ_p);
+    for (int i = 0; i < 2 && s->pbwt_v[i] >= 0; i++)
+        s->pbwt_grid[i] = (uint32_t)std::min<uint64_t>(
+            std::max<uint64_t>(2 * nmax, (uint64_t)ncu),
+            (uint64_t)ncu * (uint64_t)std::max(e->pbwt_occ[s->pbwt_v[i]], 1));
+    s->seg_par = seg_par(e, e->pbwt_occ[v]);
     // segments of cut chains: at most sqrt(blocks) per chain
     const uint64_t max_nblk = (2ull * s->Wmax + 1 + 15) / 16;
     s->seg_bytes = std::min<uint64_t>(kSegBytes, nmax * seg_words(seg_isqrt((uint32_t)max_nblk) + 1, Kpad) * 2);
@@ -1529,7 +1558,7 @@ int eimp_engine_ref_pbwt(eimp_engine *e, size_t m0, size_t nsites, uint32_t *row
     const uint64_t N = e->Nad, Kpad = round_up(N, 64);
     // panels up to one workgroup's LDS run the LDS-resident kernels; wider ones
     // the large-K kernel (order in global memory)
-    const int v = auto_pbwt_variant((uint32_t)Kpad);
+    int v = auto_pbwt_variant((uint32_t)Kpad);
     const bool big = v < 0;
     if (big && (N > pbwt_big_max_k() || pbwt_big_lds_bytes((uint32_t)N) > 160 * 1024))
         return fail(EIMP_ERR_UNSUPPORTED, "panel wider than " + std::to_string(pbwt_big_max_k()) +
@@ -1558,11 +1587,15 @@ int eimp_engine_ref_pbwt(eimp_engine *e, size_t m0, size_t nsites, uint32_t *row
         T.out = e->p_rows.as<uint32_t>();
         T.count0 = e->p_c0.as<int32_t>();
         T.hdr = e->p_hdr.as<uint16_t>();
-        lds = pbwt_lds_bytes(v, (uint32_t)Kpad);
-        int occ = 1;
-        HIPCHK(pbwt_prepare(v, lds, &occ));
+        CHK(e->prepare_pbwt(v, (uint32_t)Kpad, &lds));
+        bool latency = false;
         // (the cost model counts two directions of a target: half the device)
-        const uint32_t L = choose_segments({(uint32_t)nblk}, {(uint32_t)Kpad}, 2 * seg_par(e, occ), kSegBytes / 2, ~0u);
+        const uint32_t L = choose_segments({(uint32_t)nblk}, {(uint32_t)Kpad}, 2 * seg_par(e, e->pbwt_occ[v]),
+                                           kSegBytes / 2, ~0u, 2 * e->ncu, &latency);
+        if (latency && !absperm) {  // (the row-by-row blocks fill the device)
+            v = latency_variant(v);
+            CHK(e->prepare_pbwt(v, (uint32_t)Kpad, &lds));
+        }
         T.nseg = seg_split((uint32_t)nblk, L, T.seglen);
         chain_items(0, 0, (uint32_t)nblk, T.nseg, T.seglen, absperm ? CHAIN_STARTS : CHAIN_ROWS, oitems,
                     rank_items, comb_items);

@@ -80,10 +80,10 @@ struct TgtDev {
 struct BatchDev {
     uint32_t n;           // targets in this submission (written by the host)
     uint32_t ncref;       // cref blocks queued by k_plan: subset (gather) targets
-    uint32_t npbwt;       // PBWT chain items queued by k_plan: rows
+    uint32_t npbwt[2];    // PBWT chain items queued by k_plan, by chain shape: rows
     uint32_t nfit;        // targets whose outputs fit the pools
     uint32_t cref_ctr;    // work-queue counters (zeroed by k_plan)
-    uint32_t pbwt_ctr;
+    uint32_t pbwt_ctr[2];
     uint32_t ncref_id;    // cref blocks of whole-panel (identity) targets
     uint32_t cref_id_ctr;
     // cref queue order per kind ([0] subset, [1] identity): 0 target-major
@@ -94,7 +94,7 @@ struct BatchDev {
     // subset cref items: blocks of a group, parts of the haplotypes, passes of a part
     uint32_t cref_grp, cref_parts, cref_per;
     // chain items of cut chains: ranks of the segments, then their combination
-    uint32_t nrank, rank_ctr, ncomb, comb_ctr;
+    uint32_t nrank[2], ncomb[2], rank_ctr[2], comb_ctr[2];
 };
 
 // 16-row blocks per work item of the subset cref kernel in a full batch
@@ -181,6 +181,15 @@ __host__ __device__ inline uint64_t seg_time(uint64_t path, uint64_t work, uint3
     const uint64_t w = 20 * work / par;
     return path > w ? path : w;
 }
+// The longest chain takes longer than all work spread over the CUs, by a
+// quarter: the shape with twice the threads, which moves a chain faster and
+// holds fewer of them on a CU (K = 10,000, 1024 against 512 threads: one target
+// of 45,000 rows 2.87 against 3.25 ms as a call, 192 chains 24.3 against 26.0,
+// 512 of very different lengths 55.5 against 61.0; 384 equal ones 22.6 against
+// 19.2).
+__host__ __device__ inline bool seg_latency_bound(uint64_t path, uint64_t work, uint32_t ncu) {
+    return 4 * path * ncu >= 5 * 2 * work;
+}
 // candidates: segments of 4 << c blocks, c < kSegCands, and none
 constexpr int kSegCands = 14;
 // uint16 words of a target's segments, both directions
@@ -218,6 +227,7 @@ struct PlanArgs {
     uint16_t *seg;           // seg_cap words for the segments of cut chains
     uint64_t seg_cap;
     uint32_t cref_want;      // subset cref items that fill the device
+    uint32_t ncu, shapes;    // compute units; 2: the context has a latency shape too
     uint32_t seg_par;        // chains' worth of parallel work, times 10
     uint32_t *rowpref;       // kRowsCounters, then nmax + 1 prefix sums of pbwt_blocks
     uint32_t layout;         // LAYOUT_*

@@ -1072,13 +1072,12 @@ __global__ __launch_bounds__(PLAN_NT) void k_plan(TgtDev *__restrict__ tg, Batch
         B->nfit = (uint32_t)nfit;
         B->cref_ctr = 0;
         B->cref_id_ctr = 0;
-        B->pbwt_ctr = 0;
     }
     // Chains: cut into segments where that shortens the batch.  Wave w works out
     // the expected time of candidate w (the last one: no cut).
     __shared__ uint32_t s_nb[PLAN_NT], s_kp[PLAN_NT];
-    __shared__ uint64_t s_time[kSegCands + 1];
-    __shared__ uint32_t s_L;
+    __shared__ uint64_t s_time[kSegCands + 1], s_path[kSegCands + 1], s_work[kSegCands + 1];
+    __shared__ uint32_t s_L, s_shape;
     s_nb[t] = fit ? nblk : 0u;
     s_kp[t] = Kpad;
     __syncthreads();
@@ -1106,6 +1105,10 @@ __global__ __launch_bounds__(PLAN_NT) void k_plan(TgtDev *__restrict__ tg, Batch
             work = wave_sum64(work);
             words = wave_sum64(words);
             segs = wave_sum64(segs);
+            if ((t & 63) == 0) {
+                s_path[w] = path;
+                s_work[w] = work;
+            }
             if ((t & 63) == 0)
                 s_time[w] = words > A.seg_cap || segs > kMaxSegments ? ~0ull
                                                                     : seg_time(path, work, A.seg_par);
@@ -1122,6 +1125,7 @@ __global__ __launch_bounds__(PLAN_NT) void k_plan(TgtDev *__restrict__ tg, Batch
                 s_time[c] < s_time[kSegCands] - s_time[kSegCands] / 4)
                 best = c;
         s_L = best < kSegCands ? 4u << best : 0u;
+        s_shape = seg_latency_bound(s_path[best], s_work[best], A.ncu) ? 1u : 0u;
     }
     __syncthreads();
     uint32_t seglen = nblk;
@@ -1188,11 +1192,13 @@ __global__ __launch_bounds__(PLAN_NT) void k_plan(TgtDev *__restrict__ tg, Batch
         if (cs[e] > 1) A.comb_items[c0++] = OrderItem{tt, dir, CHAIN_COMBINE, 0, 0, cs[e]};
     }
     if (t == 0) {
-        B->npbwt = (uint32_t)nr_tot;
-        B->nrank = (uint32_t)nk_tot;
-        B->ncomb = (uint32_t)nc_tot;
-        B->rank_ctr = 0;
-        B->comb_ctr = 0;
+        for (uint32_t v = 0; v < 2; v++) {
+            const bool on = v == (A.shapes > 1 ? s_shape : 0u);
+            B->pbwt_ctr[v] = B->rank_ctr[v] = B->comb_ctr[v] = 0;
+            B->npbwt[v] = on ? (uint32_t)nr_tot : 0u;
+            B->nrank[v] = on ? (uint32_t)nk_tot : 0u;
+            B->ncomb[v] = on ? (uint32_t)nc_tot : 0u;
+        }
     }
 }
 

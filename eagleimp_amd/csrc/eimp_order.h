@@ -297,13 +297,13 @@ __device__ __forceinline__ uint64_t match8(uint32_t v, uint32_t sh, uint64_t val
 }
 
 // One pass of the stable sort of R run entries by the 8-bit digit at bits sh:
-// wave w holds entries [w SL 64, (w + 1) SL 64) in ev, 64 per slot, and writes
+// a wave holds the entries from slot s0 of 64 on in ev, SL slots, and writes
 // them to their places in ent.  A slot's ranks come from match8 and the wave's
 // running digit counts; one wave then turns the counts of all waves into
 // bases.  Every wave holds its entries before the first barrier, so ent may be
 // where they were read from.
 template <int NT, int EH>
-__device__ __forceinline__ void sort_pass(const uint32_t (&ev)[EH], uint32_t SL, uint32_t R,
+__device__ __forceinline__ void sort_pass(const uint32_t (&ev)[EH], uint32_t s0, uint32_t SL, uint32_t R,
                                           uint32_t sh, lds_ptr_t<uint32_t> ent,
                                           lds_ptr_t<uint16_t> hist, lds_ptr_t<uint16_t> base) {
     constexpr int NW = NT / 64;
@@ -311,7 +311,7 @@ __device__ __forceinline__ void sort_pass(const uint32_t (&ev)[EH], uint32_t SL,
     const lds_ptr_t<uint16_t> hw = hist + 256 * wave;
     // the conditions of the slots are worked out anew in each loop over them:
     // kept, they would fill the scalar registers
-    uint32_t sl = opaque_s(SL), i0 = wave * SL * 64 + opaque(ln);
+    uint32_t sl = opaque_s(SL), i0 = s0 * 64 + opaque(ln);
     uint32_t rk[EH];
     begin_life(rk);
     ((lds_ptr_t<uint32_t>)hw)[ln] = 0;
@@ -349,7 +349,7 @@ __device__ __forceinline__ void sort_pass(const uint32_t (&ev)[EH], uint32_t SL,
     }
     __syncthreads();
     sl = opaque_s(SL);
-    i0 = wave * SL * 64 + opaque(ln);
+    i0 = s0 * 64 + opaque(ln);
     static_for<0, EH>([&](auto si) {
         constexpr int s = decltype(si)::value;
         if ((uint32_t)s < sl) {
@@ -524,13 +524,15 @@ __device__ __attribute__((noinline)) void order_chain(const TgtDev *tgt, OrderIt
             }
             __syncthreads();
             // the runs' entries, and the run list for k_rows in the block's rows
-            const uint32_t SL = (R + NT - 1) / NT;  // slots of 64 entries per wave, <= EH
+            // slots of 64 entries, spread evenly over the waves (at most EH each)
+            const uint32_t nslot = (R + 63) / 64;
+            const uint32_t s0 = wave * nslot / NW, SL = (wave + 1) * nslot / NW - s0;
             {
                 uint32_t ev[EH];
                 begin_life(ev);
                 const gptr_t<uint32_t> list =
                     gmem(T.out) + ((rev ? (uint64_t)Mp : 0ull) + geo.s0) * RS;
-                const uint32_t sl = opaque_s(SL), i0 = wave * SL * 64 + opaque(ln);
+                const uint32_t sl = opaque_s(SL), i0 = s0 * 64 + opaque(ln);
                 static_for<0, EH>([&](auto si) {
                     constexpr int s = decltype(si)::value;
                     if ((uint32_t)s < sl) {
@@ -542,25 +544,28 @@ __device__ __attribute__((noinline)) void order_chain(const TgtDev *tgt, OrderIt
                     }
                 });
                 if (ROWS && tid == 0) hdr[q] = (uint16_t)R;
-                sort_pass<NT, EH>(ev, SL, R, 16, ent, hist, base);
+                sort_pass<NT, EH>(ev, s0, SL, R, 16, ent, hist, base);
             }
             {
                 uint32_t ev[EH];
                 begin_life(ev);
-                const uint32_t sl = opaque_s(SL), i0 = wave * SL * 64 + opaque(ln);
+                const uint32_t sl = opaque_s(SL), i0 = s0 * 64 + opaque(ln);
                 static_for<0, EH>([&](auto si) {
                     constexpr int s = decltype(si)::value;
                     if ((uint32_t)s < sl) ev[s] = ent[min(i0 + 64 * s, R - 1)];
                 });
-                sort_pass<NT, EH>(ev, SL, R, 24, ent, hist, base);
+                sort_pass<NT, EH>(ev, s0, SL, R, 24, ent, hist, base);
             }
             // new start of every run: prefix sum of the lengths in key order,
-            // SL consecutive sorted runs per thread
+            // per consecutive sorted runs per thread
+            const uint32_t per = (R + NT - 1) / NT;
             uint32_t ra[EH], rl[EH];
             begin_life(ra);
             begin_life(rl);
             uint32_t sum = 0;
-            uint32_t sl = opaque_s(SL), i0 = opaque(tid) * SL;
+            // (waves past the last run skip)
+            const uint32_t mine = wave * 64 * per < R ? per : 0u;
+            uint32_t sl = opaque_s(mine), i0 = opaque(tid) * per;
             static_for<0, EH>([&](auto si) {
                 constexpr int s = decltype(si)::value;
                 if ((uint32_t)s < sl) {
@@ -574,8 +579,8 @@ __device__ __attribute__((noinline)) void order_chain(const TgtDev *tgt, OrderIt
             });
             uint32_t tot;
             uint32_t at = wg_scan_excl<NT>(sum, red + NW, tot);
-            sl = opaque_s(SL);
-            i0 = opaque(tid) * SL;
+            sl = opaque_s(mine);
+            i0 = opaque(tid) * per;
             static_for<0, EH>([&](auto si) {
                 constexpr int s = decltype(si)::value;
                 if ((uint32_t)s < sl) {

@@ -163,7 +163,7 @@ __device__ __forceinline__ uint32_t rows_step(const uint32_t bm, uint32_t &n, ui
 }
 
 // entries per lane instantiated: odd
-constexpr int kRowEntries[] = {1, 3, 5, 7, 9, 11, 13, 17, 21, 25, 33, 41, 49, 63};
+constexpr int kRowEntries[] = {1, 3, 5, 7, 9, 11, 13, 15, 17, 21, 25, 29, 33, 37, 41, 45, 49, 55, 63};
 constexpr int kNumRowEntries = sizeof(kRowEntries) / sizeof(kRowEntries[0]);
 __device__ __forceinline__ uint32_t row_entries(uint32_t n) {
     const uint32_t need = (n + 63) / 64;
@@ -268,14 +268,17 @@ __device__ __forceinline__ void rows_block(const TgtDev &T, const bool rev, cons
 // entries of a wave, and one kernel for all blocks would have two waves per
 // SIMD.  Kernel k does the blocks of R + 1 <= 64 kRowsEntries[k] entries that
 // the kernel before it does not.
-constexpr int kRowsKernels = 3;
-constexpr int kRowsEntries[kRowsKernels] = {17, 33, 63};
+constexpr int kRowsKernels = 4;
+constexpr int kRowsEntries[kRowsKernels] = {17, 33, 49, 63};
 
 // Sorts the blocks into one list per k_rows kernel (their order within a list
 // does not matter).  pref: per target (of *d_n, or n) its first block, both
 // directions, pref[n] their number; cnt: kRowsKernels list lengths, zero
 // beforehand.  The lists of kernels 0 and 1 share `total` entries from both
-// ends, kernel 2's follows them.
+// ends, those of kernels 2 and 3 the `total` after them.
+__device__ __forceinline__ uint64_t list_at(int kernel, uint32_t total, uint32_t i) {
+    return (kernel >= 2 ? (uint64_t)total : 0ull) + (kernel & 1 ? total - 1 - i : i);
+}
 constexpr uint32_t LIST_NT = 1024;
 __global__ __launch_bounds__(LIST_NT) void k_rows_list(const TgtDev *__restrict__ tg,
                                                    const uint32_t *__restrict__ d_n, uint32_t n,
@@ -325,7 +328,7 @@ __global__ __launch_bounds__(LIST_NT) void k_rows_list(const TgtDev *__restrict_
         __syncthreads();
         if (mine >= 0) {
             const uint32_t at = s_base[mine] + s_cnt[mine][wave] + rank;
-            list[mine == 1 ? total - 1 - at : (mine == 2 ? total + at : at)] = item;
+            list[list_at(mine, total, at)] = item;
         }
         __syncthreads();
     }
@@ -333,7 +336,7 @@ __global__ __launch_bounds__(LIST_NT) void k_rows_list(const TgtDev *__restrict_
 
 template <int KERNEL>
 __global__ __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(KERNEL == 0 ? 6 : (KERNEL == 1 ? 4 : 2)))) void k_rows(
+__attribute__((amdgpu_waves_per_eu(KERNEL == 0 ? 6 : (KERNEL == 1 ? 4 : (KERNEL == 2 ? 3 : 2))))) void k_rows(
     const TgtDev *__restrict__ tg, const uint32_t *__restrict__ d_n, uint32_t n,
     const uint32_t *__restrict__ pref, const RowItem *__restrict__ list,
     const uint32_t *__restrict__ cnt, uint32_t ntog) {
@@ -346,7 +349,7 @@ __attribute__((amdgpu_waves_per_eu(KERNEL == 0 ? 6 : (KERNEL == 1 ? 4 : 2)))) vo
     for (uint32_t i = lane_id(); i < ntog; i += 64) tog[i] = 0;
     wave_order();
     for (uint32_t i = blockIdx.x; i < items; i += gridDim.x) {
-        const RowItem it = list[KERNEL == 1 ? total - 1 - i : (KERNEL == 2 ? total + i : i)];
+        const RowItem it = list[list_at(KERNEL, total, i)];
         const TgtDev &T = tg[it.chain >> 1];
         uint64_t dsum = 0;
         rows_block<EMAX>(T, (it.chain & 1u) != 0, it.q, it.runs, ent, tog, dsum);
@@ -567,7 +570,7 @@ hipError_t launch_rows(const TgtDev *tg, const uint32_t *d_n, uint32_t n, const 
     if (!blocks) return hipSuccess;
     using Fn = void (*)(const TgtDev *, const uint32_t *, uint32_t, const uint32_t *, const RowItem *,
                         const uint32_t *, uint32_t);
-    static const Fn fns[kRowsKernels] = {k_rows<0>, k_rows<1>, k_rows<2>};
+    static const Fn fns[kRowsKernels] = {k_rows<0>, k_rows<1>, k_rows<2>, k_rows<3>};
     hipLaunchKernelGGL(k_rows_list, dim3((uint32_t)std::min<uint64_t>((blocks + LIST_NT - 1) / LIST_NT, 2 * ncu)),
                        dim3(LIST_NT), 0, s, tg, d_n, n, pref, list, cnt);
     for (int k = 0; k < kRowsKernels; k++) {
