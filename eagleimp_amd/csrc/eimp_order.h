@@ -98,10 +98,10 @@ __device__ __forceinline__ uint32_t wg_scan_excl(uint32_t v, lds_ptr_t<uint32_t>
 // amount a slot's store address sits below its destination (order_dense).
 __host__ __device__ constexpr uint32_t dense_bias(int ns) { return 128u * (uint32_t)(ns - 1); }
 
-// Most runs of a block that k_rows takes (62 entries per lane, one of them
+// Most runs of a block that k_rows takes (61 entries per lane, one of them
 // closing the list); with it three 512-thread chains of 10,240 positions fit a
 // CU's LDS.
-constexpr uint32_t kMaxRuns = 64 * 62 - 1;
+constexpr uint32_t kMaxRuns = 64 * 61 - 1;
 // Run starts (uint16) a chain keeps room for: at most one run per two positions
 // goes to k_rows, and the positions past Kpad may count as one more.
 __host__ __device__ constexpr uint32_t order_starts(int nt, int e) {

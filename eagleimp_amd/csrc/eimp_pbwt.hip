@@ -162,16 +162,23 @@ __device__ __forceinline__ uint32_t rows_step(const uint32_t bm, uint32_t &n, ui
     return ztot & 0xFFFFu;
 }
 
-// entries per lane instantiated: odd
-constexpr int kRowEntries[] = {1, 3, 5, 7, 9, 11, 13, 15, 17, 21, 25, 29, 33, 37, 41, 45, 49, 55, 63};
-constexpr int kNumRowEntries = sizeof(kRowEntries) / sizeof(kRowEntries[0]);
-__device__ __forceinline__ uint32_t row_entries(uint32_t n) {
+// Entries per lane instantiated, all odd: 1, 3, .. 17, then 21, 25, .. 61
+__host__ __device__ constexpr int row_entries_at(int i) { return i <= 8 ? 2 * i + 1 : 17 + 4 * (i - 8); }
+// the index of the fewest that hold n entries
+__device__ __forceinline__ uint32_t row_entries_index(uint32_t n) {
     const uint32_t need = (n + 63) / 64;
-    uint32_t r = kRowEntries[kNumRowEntries - 1];
-#pragma unroll
-    for (int i = kNumRowEntries - 2; i >= 0; i--)
-        if (need <= (uint32_t)kRowEntries[i]) r = kRowEntries[i];
-    return r;
+    return need <= 17 ? need / 2 : 8 + (need - 17 + 3) / 4;
+}
+// f(integral_constant i) for run-time i in [B, E): a tree of uniform branches
+template <int B, int E, class F>
+__device__ __forceinline__ void dispatch(uint32_t i, F &&f) {
+    if constexpr (E - B == 1) {
+        f(std::integral_constant<int, B>{});
+    } else {
+        constexpr int M = (B + E) / 2;
+        if (i < (uint32_t)M) dispatch<B, M>(i, f);
+        else dispatch<M, E>(i, f);
+    }
 }
 
 template <int EMAX>
@@ -188,8 +195,8 @@ __device__ __forceinline__ void rows_block(const TgtDev &T, const bool rev, cons
     const uint32_t endv = 0xFFFF0000u | Kpad;
     for (uint32_t i = ln; i < R; i += 64) ent[i] = outrow[i];
     uint32_t n = R + 1;  // entries, the last one included
-    uint32_t Ej = row_entries(n);
-    for (uint32_t i = R + ln; i <= 64u * Ej; i += 64) ent[i] = endv;
+    uint32_t ie = row_entries_index(n);
+    for (uint32_t i = R + ln; i <= 64u * (uint32_t)row_entries_at((int)ie); i += 64) ent[i] = endv;
     const uint32_t pw0 = raw ? 2 * nch : 2 * npairs, tw = (RS - pw0) / 2;  // padding pairs of a row
     const uint32_t fw = raw ? ~0u : 0u;
     uint32_t g0 = (rev ? Mp * KW : 0u) + geo.s0 * KW;
@@ -198,16 +205,15 @@ __device__ __forceinline__ void rows_block(const TgtDev &T, const bool rev, cons
 #pragma unroll 1
     for (uint32_t j = 0; j < 16; j++) {
         uint32_t cnt0 = 0;
-        static_for<0, kNumRowEntries>([&](auto ii) {
-            constexpr int E = kRowEntries[decltype(ii)::value];
-            if constexpr (E <= EMAX) {
-                if (Ej == (uint32_t)E) cnt0 = rows_step<E>(0x10000u << j, n, ent, tog);
-            }
+        // the largest index this kernel reaches
+        constexpr int top = EMAX <= 17 ? EMAX / 2 : 8 + (EMAX - 17) / 4;
+        dispatch<0, top + 1>(ie, [&](auto ii) {
+            cnt0 = rows_step<row_entries_at(decltype(ii)::value)>(0x10000u << j, n, ent, tog);
         });
         c0acc = eimp_llvm_writelane(cnt0, j, c0acc);
-        Ej = row_entries(n);
+        ie = row_entries_index(n);
         // entries past the last one: no length, never kept
-        for (uint32_t i = n + ln; i <= 64u * Ej; i += 64) ent[i] = endv;
+        for (uint32_t i = n + ln; i <= 64u * (uint32_t)row_entries_at((int)ie); i += 64) ent[i] = endv;
         wave_order();
         // the row's words: 64 positions per lane
         const gptr_t<uint32_t> row = outrow + (uint64_t)j * RS;
@@ -269,7 +275,7 @@ __device__ __forceinline__ void rows_block(const TgtDev &T, const bool rev, cons
 // SIMD.  Kernel k does the blocks of R + 1 <= 64 kRowsEntries[k] entries that
 // the kernel before it does not.
 constexpr int kRowsKernels = 4;
-constexpr int kRowsEntries[kRowsKernels] = {17, 33, 49, 63};
+constexpr int kRowsEntries[kRowsKernels] = {17, 33, 49, 61};
 
 // Sorts the blocks into one list per k_rows kernel (their order within a list
 // does not matter).  pref: per target (of *d_n, or n) its first block, both
