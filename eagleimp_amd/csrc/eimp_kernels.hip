@@ -196,11 +196,38 @@ __global__ __launch_bounds__(256) void k_distance(PanelDev P, const TgtDev *__re
 // a4: exact top-K selection / take-all.  grid n, block SEL_NT.  Workgroups of
 // 256 threads fit on CUs beside a PBWT workgroup, so a context's selection can
 // run while another context's PBWT holds the device.
+//
+// One workgroup per target, so its time is what the loops over the N distances
+// wait for: eight loads in flight in the radix passes, and a compaction that
+// takes 2,048 haplotypes between two barriers, each wave counting and placing
+// 512 neighbours by ballots (96 targets on 200,000 haplotypes: 1,735 us with a
+// block scan per 256 and one load in flight, 574 us so; four on 20,000: 121 and
+// 51 us).
 // ---------------------------------------------------------------------------
 constexpr int SEL_NT = 256;
 constexpr int SEL_NW = SEL_NT / 64;
 constexpr int SEL_BINS = 1024;                    // 10-bit digits
 constexpr int SEL_BPT = SEL_BINS / SEL_NT;        // bins per thread in the bin scan
+
+constexpr int SEL_SUB = 8;                        // 64-haplotype words per wave and tile
+constexpr uint32_t SEL_TILE = SEL_NT * SEL_SUB;
+
+// f(distance) for the haplotypes that are not excluded, in any order
+template <class F>
+__device__ __forceinline__ void sel_each(const uint32_t *__restrict__ nerr, uint32_t N, F &&f) {
+    constexpr uint32_t U = 8;
+    for (uint32_t h0 = threadIdx.x; h0 < N; h0 += U * SEL_NT) {
+        uint32_t v[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {
+            const uint32_t h = h0 + u * SEL_NT;
+            v[u] = h < N ? nerr[h] : kExcluded;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++)
+            if (v[u] != kExcluded) f(v[u]);
+    }
+}
 
 // block-wide exclusive scan of one value per thread; also returns the total
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t *s_w, uint32_t &total) {
@@ -234,10 +261,7 @@ __global__ __launch_bounds__(SEL_NT) void k_select(PanelDev P, const TgtDev *__r
     if (select) {
         const uint32_t *__restrict__ nerr = T.nerr;
         uint32_t mx = 0;
-        for (uint32_t h = tid; h < N; h += SEL_NT) {
-            uint32_t v = nerr[h];
-            if (v != kExcluded) mx = max(mx, v);
-        }
+        sel_each(nerr, N, [&](uint32_t v) { mx = max(mx, v); });
         mx = wave_max(mx);
         if (l == 0) s_w[wave] = mx;
         __syncthreads();
@@ -252,11 +276,9 @@ __global__ __launch_bounds__(SEL_NT) void k_select(PanelDev P, const TgtDev *__r
             const uint32_t nb = 1u << (hi - lo);
             for (uint32_t b = tid; b < nb; b += SEL_NT) hist[b] = 0;
             __syncthreads();
-            for (uint32_t h = tid; h < N; h += SEL_NT) {
-                uint32_t v = nerr[h];
-                if (v != kExcluded && ((uint64_t)v >> hi) == (prefix >> hi))
-                    atomicAdd(&hist[(v >> lo) & (nb - 1)], 1u);
-            }
+            sel_each(nerr, N, [&](uint32_t v) {
+                if (((uint64_t)v >> hi) == (prefix >> hi)) atomicAdd(&hist[(v >> lo) & (nb - 1)], 1u);
+            });
             __syncthreads();
             // thread tid scans bins SEL_BPT*tid .. SEL_BPT*tid + SEL_BPT-1
             uint32_t cb[SEL_BPT], c = 0, total;
@@ -285,36 +307,69 @@ __global__ __launch_bounds__(SEL_NT) void k_select(PanelDev P, const TgtDev *__r
         thr = (uint32_t)prefix;
         need = k;
     }
-    // compaction in index order: ties at the threshold value go to the lowest indices
+    // compaction in index order: ties at the threshold value go to the lowest
+    // indices.  Per tile wave w holds 64 SEL_SUB neighbours; the waves' counts
+    // alternate between two halves, so a tile has one barrier.
     const uint32_t nwords = ((N + 511) / 512) * 8;
-    uint32_t ties_before = 0, sel_before = 0;
-    for (uint32_t base = 0; base < nwords * 64; base += SEL_NT) {
-        const uint32_t h = base + tid;
-        bool sel, tie = false;
-        if (h >= N) {
-            sel = false;
-        } else if (select) {
-            uint32_t v = T.nerr[h];
-            tie = (v == thr);
-            sel = v < thr;
-        } else {
-            sel = !excluded_hap(P, T.ignore, h);
+    __shared__ uint32_t s_lt[2][SEL_NW], s_eq[2][SEL_NW];
+    uint32_t ties_before = 0, sel_before = 0, par = 0;
+    auto load = [&](uint32_t base, uint32_t (&v)[SEL_SUB]) {
+#pragma unroll
+        for (int u = 0; u < SEL_SUB; u++) {
+            const uint32_t h = base + (wave * SEL_SUB + (uint32_t)u) * 64 + l;
+            v[u] = select && h < N ? T.nerr[h] : 0u;
         }
-        if (select) {
-            uint32_t tcount;
-            uint32_t trank = ties_before + block_excl_scan(tie ? 1u : 0u, s_w, tcount);
-            if (tie && trank < need) sel = true;
-            ties_before += tcount;
+    };
+    uint32_t nx[SEL_SUB];
+    load(0, nx);
+    for (uint32_t base = 0; base < nwords * 64; base += SEL_TILE, par ^= 1u) {
+        uint32_t cur[SEL_SUB];
+#pragma unroll
+        for (int u = 0; u < SEL_SUB; u++) cur[u] = nx[u];
+        load(base + SEL_TILE, nx);
+        uint64_t ltm[SEL_SUB], eqm[SEL_SUB];
+        uint32_t nlt = 0, neq = 0;
+#pragma unroll
+        for (int u = 0; u < SEL_SUB; u++) {
+            const uint32_t h = base + (wave * SEL_SUB + (uint32_t)u) * 64 + l;
+            const bool in = h < N;
+            ltm[u] = __ballot(in && (select ? cur[u] < thr : !excluded_hap(P, T.ignore, h)));
+            eqm[u] = __ballot(in && select && cur[u] == thr);
+            nlt += (uint32_t)__popcll(ltm[u]);
+            neq += (uint32_t)__popcll(eqm[u]);
         }
-        uint32_t scount;
-        const uint32_t pos = sel_before + block_excl_scan(sel ? 1u : 0u, s_w, scount);
-        // exactly K when Ncorr is consistent; the bitmap always matches bh
-        sel = sel && pos < T.K;
-        if (sel) T.bh[pos] = h;
-        const uint64_t sm = __ballot(sel);
-        const uint32_t word = base / 64 + wave;
-        if (l == 0 && word < nwords) T.bhflags[word] = sm;
-        sel_before += scount;
+        if (l == 0) {
+            s_lt[par][wave] = nlt;
+            s_eq[par][wave] = neq;
+        }
+        __syncthreads();
+        uint32_t tb = ties_before, sb = sel_before;
+#pragma unroll
+        for (int w = 0; w < SEL_NW; w++) {
+            const uint32_t c = s_lt[par][w], q = s_eq[par][w];
+            const uint32_t taken = min(q, need > ties_before ? need - ties_before : 0u);
+            if (w < (int)wave) {
+                tb += q;
+                sb += c + taken;
+            }
+            ties_before += q;
+            sel_before += c + taken;
+        }
+#pragma unroll
+        for (int u = 0; u < SEL_SUB; u++) {
+            const bool tie = (eqm[u] >> l) & 1ull;
+            bool sel = ((ltm[u] >> l) & 1ull) || (tie && tb + mbcnt(eqm[u]) < need);
+            tb += (uint32_t)__popcll(eqm[u]);
+            const uint64_t m = __ballot(sel);
+            const uint32_t pos = sb + mbcnt(m);
+            sb += (uint32_t)__popcll(m);
+            // exactly K when Ncorr is consistent; the bitmap always matches bh
+            sel = sel && pos < T.K;
+            const uint32_t word = base / 64 + wave * SEL_SUB + (uint32_t)u;
+            if (sel) T.bh[pos] = word * 64 + l;
+            const uint64_t sm = __ballot(sel);
+            if (l == 0 && word < nwords) T.bhflags[word] = sm;
+        }
     }
     if (tid == 0) T.stats[3] = sel_before;
     // k_monos starts from these
