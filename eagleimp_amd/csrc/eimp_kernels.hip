@@ -79,48 +79,97 @@ __global__ __launch_bounds__(256) void k_panel_mono(PanelDev P, uint64_t *__rest
 }
 
 // ---------------------------------------------------------------------------
-// a3: distances for groups of DIST_G targets.  grid (ceil(N_ad/16),
-// ceil(n/DIST_G)), block 256: 16 haplotypes (4 per wave) x DIST_G targets per
-// workgroup.  Over the union of the group's windows, 64 panel words at a time,
-// the group's genotype words are staged in LDS shifted to panel alignment
-// (sites outside a target's window zero); each lane then reads one word of its
-// 4 haplotype rows once for all targets of the group, so a panel word is read
-// once per group rather than once per target.  nerr = sum of
+// a3: distances for groups of DIST_G targets.  block 256: DIST_W haplotypes
+// (DIST_H per wave) x DIST_G targets per workgroup.  Over the union of the
+// group's windows, 64 panel words at a time, the group's genotype words are
+// staged in LDS shifted to panel alignment (sites outside a target's window
+// zero); each lane then reads one word of its DIST_H haplotype rows once for all
+// targets of the group whose window reaches these words.  nerr = sum of
 // popcount((is0 & h) | (is2 & ~h)) over the window (compare_withPreInit,
 // src/Datatypes.cpp:107-116).
+//
+// Bound by vector instructions (four per word, haplotype and target) once the
+// loads are out of the way: the next 64 words of haplotypes and genotypes are
+// loaded while these are compared, the LDS words alternate between two halves
+// (one barrier per 64), and the staging, whose cost per wave does not depend on
+// DIST_H, is shared by eight haplotypes.  The grid is (8 target groups, groups
+// of 8 haplotype blocks): workgroups go to the XCDs in turn, so that all target
+// groups of a haplotype block run on one XCD and all but the first find its rows
+// in that L2.
+// 256 targets with 10,000 to 100,000 sites on 20,000 haplotypes: 2,275 us with
+// four haplotypes per wave, loads after the barrier and one reduction per sum,
+// 1,185 us so; 96 targets with 20,000 sites on 200,000 haplotypes: 2,415 and
+// 1,513 us (three waves per SIMD; four spill and take longer).
 // ---------------------------------------------------------------------------
 constexpr int DIST_G = 8;
+constexpr int DIST_H = 8;
+constexpr uint32_t DIST_W = 4 * DIST_H;
 
-// genotype words (is0, is2) of T for panel word p, bits of sites outside
+// genotype words (is0, is2) around panel word p of a target, its window's words
+// q and q + 1, as loaded and shifted to panel alignment, bits of sites outside
 // [s0, s0 + W) zero
-__device__ __forceinline__ void gt_panel_word(const TgtDev &T, uint64_t p, uint64_t &a,
-                                              uint64_t &b) {
-    const uint64_t nq = ((uint64_t)T.W + 63) / 64;  // window words with data
-    const int64_t d = (int64_t)(64 * p) - (int64_t)T.s0;  // window bit of panel bit 0
-    auto at = [&](int64_t q, int k) -> uint64_t {
-        return (q >= 0 && (uint64_t)q < nq) ? T.gt[2 * q + k] : 0ull;
-    };
-    if (d >= 0) {
-        const int64_t q = d >> 6;
-        const uint32_t sh = (uint32_t)(d & 63);
-        a = at(q, 0);
-        b = at(q, 1);
-        if (sh) {
-            a = (a >> sh) | (at(q + 1, 0) << (64 - sh));
-            b = (b >> sh) | (at(q + 1, 1) << (64 - sh));
-        }
-    } else if (d > -64) {
-        const uint32_t sh = (uint32_t)(-d);
-        a = at(0, 0) << sh;
-        b = at(0, 1) << sh;
-    } else {
-        a = b = 0ull;
+struct GtWords {
+    uint64_t a0 = 0, b0 = 0, a1 = 0, b1 = 0;
+};
+__device__ __forceinline__ GtWords gt_load(gptr_t<const uint64_t> gt, uint64_t s0, uint64_t W, uint64_t p) {
+    const int64_t nq = (int64_t)((W + 63) / 64), q = ((int64_t)(64 * p) - (int64_t)s0) >> 6;
+    GtWords r;
+    if (q >= 0 && q < nq) {
+        r.a0 = gt[2 * q];
+        r.b0 = gt[2 * q + 1];
+    }
+    if (q + 1 >= 0 && q + 1 < nq) {
+        r.a1 = gt[2 * q + 2];
+        r.b1 = gt[2 * q + 3];
+    }
+    return r;
+}
+__device__ __forceinline__ void gt_align(const GtWords &r, uint64_t s0, uint64_t W, uint64_t p, uint64_t &a,
+                                         uint64_t &b) {
+    const uint32_t sh = (uint32_t)(0u - (uint32_t)s0) & 63u;  // (64 p - s0) mod 64
+    a = r.a0 >> sh;
+    b = r.b0 >> sh;
+    if (sh) {
+        a |= r.a1 << (64 - sh);
+        b |= r.b1 << (64 - sh);
     }
     // panel bits at or beyond the window end
-    const int64_t end = (int64_t)T.s0 + (int64_t)T.W - (int64_t)(64 * p);
+    const int64_t end = (int64_t)s0 + (int64_t)W - (int64_t)(64 * p);
     const uint64_t keep = end >= 64 ? ~0ull : (end <= 0 ? 0ull : ((1ull << end) - 1));
     a &= keep;
     b &= keep;
+}
+
+// Sums of 64 values over the wave: lane l returns the sum of v[wave_sums_index(l)]
+// over all lanes.  Each stage adds two halves of the lanes and halves the values
+// that a lane carries: 32 and 16 by swapping rows, the rest by DPP.
+__device__ __forceinline__ uint32_t wave_sums_index(uint32_t l) {
+    return (l & 0x38u) | ((l & 1u) << 2) | (l & 2u) | ((l >> 2) & 1u);
+}
+__device__ __forceinline__ uint32_t wave_sums(uint32_t (&v)[64]) {
+    const uint32_t l = lane_id();
+#pragma unroll
+    for (int k = 0; k < 32; k++) {
+        const u32x2 s = __builtin_amdgcn_permlane32_swap(v[k], v[k + 32], false, false);
+        v[k] = s.x + s.y;
+    }
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+        const u32x2 s = __builtin_amdgcn_permlane16_swap(v[k], v[k + 16], false, false);
+        v[k] = s.x + s.y;
+    }
+    auto fold = [&](auto ctrl, uint32_t bit, int k, int half) {
+        const uint32_t keep = l & bit ? v[k + half] : v[k], give = l & bit ? v[k] : v[k + half];
+        v[k] = keep + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, decltype(ctrl)::value, 0xF, 0xF, true);
+    };
+#pragma unroll
+    for (int k = 0; k < 8; k++) fold(std::integral_constant<int, 0x128>{}, 8u, k, 8);  // lane ^ 8
+#pragma unroll
+    for (int k = 0; k < 4; k++) fold(std::integral_constant<int, 0xB1>{}, 1u, k, 4);   // lane ^ 1
+#pragma unroll
+    for (int k = 0; k < 2; k++) fold(std::integral_constant<int, 0x4E>{}, 2u, k, 2);   // lane ^ 2
+    const uint32_t keep = l & 4u ? v[1] : v[0], give = l & 4u ? v[0] : v[1];
+    return keep + (uint32_t)__shfl_xor((int)give, 4);
 }
 
 __global__ __launch_bounds__(256) void k_distance(PanelDev P, const TgtDev *__restrict__ tg,
@@ -128,66 +177,85 @@ __global__ __launch_bounds__(256) void k_distance(PanelDev P, const TgtDev *__re
                                                  const uint32_t *__restrict__ d_n) {
     // tlist: targets that select (nlist of them); without it every target of the
     // batch (size *d_n), those that do not select are skipped
-    __shared__ uint64_t sg[DIST_G][64][2];
+    __shared__ uint64_t sg[2][DIST_G][64][2];
     const uint32_t n = tlist ? nlist : *d_n;
-    const uint32_t j0 = blockIdx.y * DIST_G;
+    const uint32_t j0 = (blockIdx.x >> 3) * DIST_G;
     if (j0 >= n) return;
-    const TgtDev *Tj[DIST_G];
-    bool act[DIST_G];
-    uint64_t plo = ~0ull, phi = 0;
+    // panel words of the targets' windows; empty for those left out
+    uint32_t pb[DIST_G], pe[DIST_G];
+    uint32_t plo = ~0u, phi = 0;
 #pragma unroll
     for (int j = 0; j < DIST_G; j++) {
-        const uint32_t q = j0 + j;
-        act[j] = q < n;
-        Tj[j] = act[j] ? &tg[tlist ? tlist[q] : q] : tg;
-        act[j] = act[j] && (Tj[j]->flags & TF_SELECT);
-        if (act[j]) {
-            plo = min(plo, Tj[j]->s0 / 64);
-            phi = max(phi, (Tj[j]->s0 + Tj[j]->W + 63) / 64);
+        const uint32_t q = min(j0 + (uint32_t)j, n - 1);
+        const TgtDev &T = tg[tlist ? tlist[q] : q];
+        pb[j] = pe[j] = 0;
+        if (j0 + j < n && (T.flags & TF_SELECT)) {
+            pb[j] = (uint32_t)(T.s0 / 64);
+            pe[j] = (uint32_t)((T.s0 + T.W + 63) / 64);
+            plo = min(plo, pb[j]);
+            phi = max(phi, pe[j]);
         }
     }
     if (phi == 0) return;
-    const uint32_t tid = threadIdx.x, wave = tid >> 6, l = lane_id();
-    const uint32_t hb = blockIdx.x * 16 + wave * 4;
-    uint32_t e[4][DIST_G];
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), l = lane_id();
+    // this wave stages the words of targets wave and wave + 4
+    gptr_t<const uint64_t> sgt[2];
+    uint64_t ss0[2], sW[2];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < DIST_G; j++) e[i][j] = 0;
-    for (uint64_t c0 = plo; c0 < phi; c0 += 64) {
-        for (uint32_t q = tid; q < DIST_G * 64; q += 256) {
-            const uint32_t j = q / 64, pi = q % 64;
-            uint64_t a = 0, b = 0;
-#pragma unroll
-            for (int jj = 0; jj < DIST_G; jj++)  // static indexing of Tj / act
-                if (jj == (int)j && act[jj] && c0 + pi < phi) gt_panel_word(*Tj[jj], c0 + pi, a, b);
-            sg[j][pi][0] = a;
-            sg[j][pi][1] = b;
-        }
-        __syncthreads();
-        const uint64_t p = c0 + l;
-        uint64_t hv[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            hv[i] = (hb + i < P.N_ad && p < phi) ? P.hap[(uint64_t)(hb + i) * P.hap_stride + p] : 0ull;
-#pragma unroll
-        for (int j = 0; j < DIST_G; j++) {
-            if (!act[j]) continue;
-            const uint64_t g0 = sg[j][l][0], g2 = sg[j][l][1];
-#pragma unroll
-            for (int i = 0; i < 4; i++) e[i][j] += (uint32_t)__popcll((g0 & hv[i]) | (g2 & ~hv[i]));
-        }
-        __syncthreads();
+    for (int u = 0; u < 2; u++) {
+        const uint32_t q = min(j0 + wave + 4u * (uint32_t)u, n - 1);
+        const TgtDev &T = tg[tlist ? tlist[q] : q];
+        sgt[u] = gmem(T.gt);
+        ss0[u] = T.s0;
+        sW[u] = T.W;
     }
+    for (uint32_t hblk = blockIdx.y * 8 + (blockIdx.x & 7u); hblk * DIST_W < P.N_ad; hblk += gridDim.y * 8) {
+        const uint32_t hb = hblk * DIST_W + wave * DIST_H;
+        uint32_t e[64];
 #pragma unroll
-    for (int j = 0; j < DIST_G; j++) {
-        if (!act[j]) continue;
+        for (int k = 0; k < 64; k++) e[k] = 0;
+        uint64_t hv[DIST_H], hx[DIST_H];
+        GtWords gw[2];
+        const gptr_t<const uint64_t> row0 = gmem(P.hap) + (uint64_t)hb * P.hap_stride;
+        auto load = [&](uint32_t c0) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t h = hb + i;
-            const uint32_t s = wave_sum(e[i][j]);
-            if (l == 0 && h < P.N_ad)
-                Tj[j]->nerr[h] = excluded_hap(P, Tj[j]->ignore, h) ? kExcluded : s;
+            for (int u = 0; u < 2; u++) gw[u] = gt_load(sgt[u], ss0[u], sW[u], c0 + l);
+#pragma unroll
+            for (int i = 0; i < DIST_H; i++)
+                hx[i] = (hb + i < P.N_ad && c0 + l < phi) ? row0[i * P.hap_stride + c0 + l] : 0ull;
+        };
+        auto stage = [&](uint32_t c0, uint32_t half) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                uint64_t a, b;
+                gt_align(gw[u], ss0[u], sW[u], c0 + l, a, b);
+                sg[half][wave + 4 * u][l][0] = a;
+                sg[half][wave + 4 * u][l][1] = b;
+            }
+        };
+        load(plo);
+        stage(plo, 0);
+        uint32_t half = 0;
+        for (uint32_t c0 = plo; c0 < phi; c0 += 64, half ^= 1u) {
+#pragma unroll
+            for (int i = 0; i < DIST_H; i++) hv[i] = hx[i];
+            __syncthreads();  // half is written, and everyone is done with the other
+            if (c0 + 64 < phi) load(c0 + 64);
+#pragma unroll
+            for (int j = 0; j < DIST_G; j++) {
+                if (c0 >= pe[j] || c0 + 64 <= pb[j]) continue;
+                const uint64_t g0 = sg[half][j][l][0], g2 = sg[half][j][l][1];
+#pragma unroll
+                for (int i = 0; i < DIST_H; i++)
+                    e[j * DIST_H + i] += (uint32_t)__popcll((g0 & hv[i]) | (g2 & ~hv[i]));
+            }
+            if (c0 + 64 < phi) stage(c0 + 64, half ^ 1u);
+        }
+        __syncthreads();  // the next block's first words go to either half
+        const uint32_t s = wave_sums(e), k = wave_sums_index(l), h = hb + k % DIST_H, q = j0 + k / DIST_H;
+        if (q < n && h < P.N_ad) {
+            const TgtDev &T = tg[tlist ? tlist[q] : q];
+            if (T.flags & TF_SELECT) T.nerr[h] = excluded_hap(P, T.ignore, h) ? kExcluded : s;
         }
     }
 }
@@ -1416,8 +1484,7 @@ hipError_t launch_panel_mono(const PanelDev &P, uint64_t *pand, uint64_t *por, h
 hipError_t launch_distance(const PanelDev &P, const TgtDev *tg, const uint32_t *tlist,
                            uint32_t nsel, hipStream_t s) {
     if (!nsel) return hipSuccess;
-    hipLaunchKernelGGL(k_distance, dim3((P.N_ad + 15) / 16, (nsel + DIST_G - 1) / DIST_G), dim3(256),
-                       0, s, P, tg, tlist, nsel, (const uint32_t *)nullptr);
+    hipLaunchKernelGGL(k_distance, distance_grid(P, nsel), dim3(256), 0, s, P, tg, tlist, nsel, (const uint32_t *)nullptr);
     return hipGetLastError();
 }
 hipError_t launch_select(const PanelDev &P, const TgtDev *tg, uint32_t n, hipStream_t s) {
@@ -1439,6 +1506,10 @@ hipError_t launch_splits(const PanelDev &P, const TgtDev *tg, uint32_t n, hipStr
     return hipGetLastError();
 }
 hipError_t launch_bits_to_list(const TgtDev *tg, uint32_t n, uint32_t nbits_bh, int which,
+static dim3 distance_grid(const PanelDev &P, uint32_t n) {
+    const uint32_t nhb = (P.N_ad + DIST_W - 1) / DIST_W;
+    return dim3(8 * ((n + DIST_G - 1) / DIST_G), std::min((nhb + 7) / 8, 65535u));
+}
                                hipStream_t s) {
     if (!n) return hipSuccess;
     hipLaunchKernelGGL(k_bits_to_list, dim3(n), dim3(SEL_NT), 0, s, tg, nbits_bh, which);
@@ -1510,8 +1581,7 @@ hipError_t launch_prep_dev(int cls, const PanelDev &P, const TgtDev *tg, const u
                            uint32_t nmax, uint32_t max_ww, uint32_t ncu, hipStream_t s) {
     switch (cls) {
     case 0:
-        hipLaunchKernelGGL(k_distance, dim3((P.N_ad + 15) / 16, (nmax + DIST_G - 1) / DIST_G),
-                           dim3(256), 0, s, P, tg, (const uint32_t *)nullptr, 0u, d_n);
+        hipLaunchKernelGGL(k_distance, distance_grid(P, nmax), dim3(256), 0, s, P, tg, (const uint32_t *)nullptr, 0u, d_n);
         break;
     case 1:
         hipLaunchKernelGGL(k_select, dim3(nmax), dim3(SEL_NT), 0, s, P, tg, d_n);
