@@ -784,9 +784,9 @@ __device__ __forceinline__ void cref_fill(const PanelDev &P, const TgtDev &T, ui
 }
 
 // Blocks [b0, b1) of a subset target from the haplotype-major panel, passes
-// [p0, p1) of CREF_NT haplotypes: thread x takes the chosen haplotypes k = x +
-// CREF_NT p and streams each one's
-// row over the sites of the blocks, 32 window sites per step:
+// [p0, p1) of CREF_NT haplotypes.  A wave takes 64 H chosen haplotypes at a
+// time, H per lane, and streams their rows over the sites of the blocks, 32
+// window sites per step:
 //   inc = (v & HomRef) | (~v & HomAlt)  (HomRef = is0 & ~is2, HomAlt =
 //                                        is2 & ~is0; split sites and sites
 //                                        outside the range masked out)
@@ -801,7 +801,16 @@ __device__ __forceinline__ void cref_fill(const PanelDev &P, const TgtDev &T, ui
 // block's uint16.  Only the K chosen rows are read (the site-major layout
 // would need all N bits of every site).  Haplotypes K..Kpad-1 get all-ones
 // values (the PBWT kernel's padding); count0 comes from the PBWT kernel.
-__device__ __forceinline__ void cref_range_hap(const PanelDev &P, const TgtDev &T, uint32_t b0,
+//
+// Bound by instruction issue: the loop over the splits takes four vector
+// instructions per split and haplotype and six scalar ones per split and wave.
+// Where a part has two passes or more a lane takes two haplotypes, which halves
+// the scalar ones (256 targets, windows of 10,000 to 100,000 sites, K of 2,000
+// to 10,000: 8,784 us with one, 5,803 us with two; 96 targets on the
+// 200,000-haplotype panel: 2,763 and 1,611 us); a part of one pass would leave
+// half of its waves idle.
+template <int H>
+__device__ __forceinline__ void cref_range_h(const PanelDev &P, const TgtDev &T, uint32_t b0,
                                                uint32_t b1, uint32_t p0, uint32_t p1) {
     const uint32_t tid = threadIdx.x;
     const uint32_t K = T.K, S = T.S, Kpad = T.Kpad, W = T.W;
@@ -825,21 +834,30 @@ __device__ __forceinline__ void cref_range_hap(const PanelDev &P, const TgtDev &
     const uint64_t rowlen = 2 * P.hap_stride;  // uint32 words per haplotype row
     const uint64_t q0 = T.s0 >> 5;
     const uint32_t sh = (uint32_t)T.s0 & 31;
-    for (uint32_t kb = p0 * CREF_NT; kb < min(K, p1 * CREF_NT); kb += CREF_NT) {
-        const uint32_t k = kb + tid;
-        const bool act = k < K;
-        const uint32_t h = act ? (ident ? k : bh[k]) : 0u;
-        const gptr_t<const uint32_t> row = gmem((const uint32_t *)P.hap) + (uint64_t)h * rowlen;
-        uint32_t cin = 0, acc = 0, j2 = 0, b = b0;  // j2: bit position of the next pair
+    const uint32_t kend = min(K, p1 * CREF_NT), wave = tid >> 6, l = lane_id();
+    for (uint32_t kb = p0 * CREF_NT + 64 * H * wave; kb < kend; kb += H * CREF_NT) {
+        uint32_t k[H], cin[H], acc[H];
+        gptr_t<const uint32_t> row[H];
+#pragma unroll
+        for (int e = 0; e < H; e++) {
+            k[e] = kb + 64 * e + l;
+            const uint32_t h = k[e] < kend ? (ident ? k[e] : bh[k[e]]) : 0u;
+            row[e] = gmem((const uint32_t *)P.hap) + (uint64_t)h * rowlen;
+            cin[e] = acc[e] = 0;
+        }
+        uint32_t room = 8, b = b0;  // pairs until block b is full
+        auto store = [&](uint32_t shift) {
+#pragma unroll
+            for (int e = 0; e < H; e++)
+                if (k[e] < kend) dst[(uint64_t)b * Kpad + k[e]] = (uint16_t)(acc[e] >> shift);
+        };
         // The row is read in chunks of 16 words (64 bytes) aligned in the row
-        // (rows start on 64-byte boundaries), each as four 16-byte loads, two
-        // chunks ahead of the words being processed: a lane asks for both
-        // halves of a 128-byte line close together, so fewer lines are
-        // fetched again after the cache has dropped them.  Window word i is
-        // bits sh.. of row words q0 + i and q0 + i + 1.
-        auto chunk = [&](uint64_t R, uint32_t (&c)[16]) {
+        // (rows start on 64-byte boundaries), each as four 16-byte loads, one
+        // chunk ahead of the words being processed.  Window word i is bits
+        // sh.. of row words q0 + i and q0 + i + 1.
+        auto chunk = [&](int e, uint64_t R, uint32_t (&c)[16]) {
             if (R + 16 <= rowlen) {
-                const gptr_t<const u32x4> r4 = (gptr_t<const u32x4>)(row + R);
+                const gptr_t<const u32x4> r4 = (gptr_t<const u32x4>)(row[e] + R);
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
                     const u32x4 x = r4[u];
@@ -850,24 +868,21 @@ __device__ __forceinline__ void cref_range_hap(const PanelDev &P, const TgtDev &
                 }
             } else {
 #pragma unroll
-                for (int u = 0; u < 16; u++) c[u] = R + u < rowlen ? row[R + u] : 0u;
+                for (int u = 0; u < 16; u++) c[u] = R + u < rowlen ? row[e][R + u] : 0u;
             }
         };
         const uint64_t R0 = (q0 + i0) & ~15ull;  // the first chunk
-        uint32_t cur[16], nx[16], nx2[16];
-        chunk(R0, nx);
-        chunk(R0 + 16, nx2);
+        uint32_t nx[H][16];
+#pragma unroll
+        for (int e = 0; e < H; e++) chunk(e, R0, nx[e]);
         for (uint64_t R = R0; R < q0 + i1; R += 16) {
+            uint32_t w[H][16];
 #pragma unroll
-            for (int u = 0; u < 16; u++) {
-                cur[u] = nx[u];
-                nx[u] = nx2[u];
+            for (int e = 0; e < H; e++) {
+#pragma unroll
+                for (int u = 0; u < 16; u++) w[e][u] = nx[e][u];
+                chunk(e, R + 16, nx[e]);
             }
-            chunk(R + 32, nx2);
-            uint32_t w[17];
-#pragma unroll
-            for (int u = 0; u < 16; u++) w[u] = cur[u];
-            w[16] = nx[0];
             // window word of the chunk's first word (below i0 for the first
             // chunk: those words are skipped)
             const int64_t ib = (int64_t)R - (int64_t)q0;
@@ -876,7 +891,6 @@ __device__ __forceinline__ void cref_range_hap(const PanelDev &P, const TgtDev &
                 if (ib + u < (int64_t)i0) continue;
                 const uint32_t i = (uint32_t)(ib + u);
                 if (i >= i1) break;
-                const uint32_t v = __builtin_amdgcn_alignbit(w[u + 1], w[u], sh);
                 uint32_t rng = ~0u;
                 if (i == i0) rng &= ~0u << (m0 & 31);
                 if (i == i1 - 1 && (m1 & 31)) rng &= (1u << (m1 & 31)) - 1;
@@ -886,32 +900,50 @@ __device__ __forceinline__ void cref_range_hap(const PanelDev &P, const TgtDev &
                 const uint32_t g0 = gt32[4 * (i >> 1) + (i & 1)], g2 = gt32[4 * (i >> 1) + 2 + (i & 1)];
                 const uint32_t hr = __builtin_amdgcn_readfirstlane(g0 & ~g2 & ~spw & rng);
                 const uint32_t ha = __builtin_amdgcn_readfirstlane(g2 & ~g0 & ~spw & rng);
-                const uint32_t inc = (v & hr) | (~v & ha);
-                const uint32_t pr = ~spw;
-                const uint64_t sum = (uint64_t)pr + inc + cin;
-                const uint32_t C = (uint32_t)sum ^ pr ^ inc;
-                cin = (uint32_t)(sum >> 32);
-                for (uint32_t sl = spw; sl; sl &= sl - 1) {
-                    const uint32_t p = (uint32_t)__builtin_ctz(sl);
-                    // the split's two rows: inconsistency (bit 0), allele (bit 1)
-                    const uint32_t pair = __builtin_amdgcn_ubfe(C, p, 1u) |
-                                          (__builtin_amdgcn_ubfe(v, p, 1u) << 1);
-                    acc |= pair << j2;
-                    j2 += 2;
-                    if (j2 == 16) {
-                        if (act) dst[(uint64_t)b * Kpad + k] = (uint16_t)acc;
-                        acc = 0;
-                        j2 = 0;
+                uint32_t v[H], C[H];
+#pragma unroll
+                for (int e = 0; e < H; e++) {
+                    v[e] = __builtin_amdgcn_alignbit(u < 15 ? w[e][(u + 1) & 15] : nx[e][0], w[e][u], sh);
+                    const uint32_t inc = (v[e] & hr) | (~v[e] & ha), pr = ~spw;
+                    const uint64_t sum = (uint64_t)pr + inc + cin[e];
+                    C[e] = (uint32_t)sum ^ pr ^ inc;
+                    cin[e] = (uint32_t)(sum >> 32);
+                }
+                // the splits up to the end of the word or of the block: their
+                // rows, inconsistency and allele, enter acc from the top
+                for (uint32_t sl = spw; sl;) {
+                    uint32_t m = min((uint32_t)__builtin_popcount(sl), room);
+                    room -= m;
+                    do {
+                        const uint32_t p = (uint32_t)__builtin_ctz(sl);
+                        sl &= sl - 1;
+#pragma unroll
+                        for (int e = 0; e < H; e++) {
+                            acc[e] = __builtin_amdgcn_alignbit(C[e] >> p, acc[e], 1u);
+                            acc[e] = __builtin_amdgcn_alignbit(v[e] >> p, acc[e], 1u);
+                        }
+                    } while (--m);
+                    if (!room) {
+                        store(16u);
+                        room = 8;
                         b++;
                     }
                 }
             }
         }
         if (last) {  // row 2S: an inconsistency after the last split
-            acc |= cin << j2;
-            if (act) dst[(uint64_t)b * Kpad + k] = (uint16_t)acc;
+#pragma unroll
+            for (int e = 0; e < H; e++)  // the pairs come down to bit 0, the row above them
+                acc[e] = room == 8 ? cin[e] : (acc[e] >> (16 + 2 * room)) | (cin[e] << (16 - 2 * room));
+            store(0u);
         }
     }
+}
+
+__device__ __forceinline__ void cref_range_hap(const PanelDev &P, const TgtDev &T, uint32_t b0,
+                                               uint32_t b1, uint32_t p0, uint32_t p1) {
+    if (p1 - p0 > 1) cref_range_h<2>(P, T, b0, b1, p0, p1);
+    else cref_range_h<1>(P, T, b0, b1, p0, p1);
 }
 
 // In-register transpose of two 16x16 bit blocks side by side: on entry bit c
@@ -1481,6 +1513,10 @@ hipError_t launch_panel_mono(const PanelDev &P, uint64_t *pand, uint64_t *por, h
     hipLaunchKernelGGL(k_panel_mono, dim3((P.M + 3) / 4), dim3(256), 0, s, P, pand, por);
     return hipGetLastError();
 }
+static dim3 distance_grid(const PanelDev &P, uint32_t n) {
+    const uint32_t nhb = (P.N_ad + DIST_W - 1) / DIST_W;
+    return dim3(8 * ((n + DIST_G - 1) / DIST_G), std::min((nhb + 7) / 8, 65535u));
+}
 hipError_t launch_distance(const PanelDev &P, const TgtDev *tg, const uint32_t *tlist,
                            uint32_t nsel, hipStream_t s) {
     if (!nsel) return hipSuccess;
@@ -1506,10 +1542,6 @@ hipError_t launch_splits(const PanelDev &P, const TgtDev *tg, uint32_t n, hipStr
     return hipGetLastError();
 }
 hipError_t launch_bits_to_list(const TgtDev *tg, uint32_t n, uint32_t nbits_bh, int which,
-static dim3 distance_grid(const PanelDev &P, uint32_t n) {
-    const uint32_t nhb = (P.N_ad + DIST_W - 1) / DIST_W;
-    return dim3(8 * ((n + DIST_G - 1) / DIST_G), std::min((nhb + 7) / 8, 65535u));
-}
                                hipStream_t s) {
     if (!n) return hipSuccess;
     hipLaunchKernelGGL(k_bits_to_list, dim3(n), dim3(SEL_NT), 0, s, tg, nbits_bh, which);
