@@ -1504,6 +1504,25 @@ hipError_t raise_lds_limit(const void *fn, size_t lds) {
     return e;
 }
 
+// Pieces of device arrays into one pinned host buffer (grid x pieces, block
+// 256).  Bound by the link to the host; 16 bytes a thread keep its writes whole.
+__global__ __launch_bounds__(256) void k_gather(GatherArgs A, char *__restrict__ dst) {
+    const uint32_t i = blockIdx.y, bytes = A.bytes[i], n16 = bytes / 16;
+    const gptr_t<const uint32_t> src = (gptr_t<const uint32_t>)(const uint32_t *)A.src[i];
+    const gptr_t<uint32_t> out = (gptr_t<uint32_t>)(uint32_t *)(dst + A.off[i]);
+    for (uint32_t q = blockIdx.x * 256 + threadIdx.x; q < n16; q += gridDim.x * 256) {
+        // the arrays are aligned to their elements only
+        const u32x4 v = u32x4{src[4 * q], src[4 * q + 1], src[4 * q + 2], src[4 * q + 3]};
+        *(gptr_t<u32x4>)(out + 4 * q) = v;
+    }
+    const uint32_t tail = 4 * n16 + threadIdx.x;
+    if (blockIdx.x == 0 && tail < bytes / 4) out[tail] = src[tail];
+}
+hipError_t launch_gather(const GatherArgs &a, void *dst, size_t bytes, hipStream_t s) {
+    const uint32_t wgs = (uint32_t)std::min<size_t>((bytes + 4095) / 4096, 128);
+    hipLaunchKernelGGL(k_gather, dim3(std::max(wgs, 1u), a.n), dim3(256), 0, s, a, static_cast<char *>(dst));
+    return hipGetLastError();
+}
 hipError_t launch_site_to_hap(const PanelDev &P, uint64_t *hap, hipStream_t s) {
     dim3 grid((unsigned)((P.hap_stride + 3) / 4), (P.N_ad + 63) / 64);
     hipLaunchKernelGGL(k_site_to_hap, grid, dim3(256), 0, s, P, hap);

@@ -8,6 +8,17 @@ namespace eimp {
 // raises a kernel's dynamic-LDS limit (process-wide; never lowered)
 hipError_t raise_lds_limit(const void *fn, size_t lds);
 
+// pieces of device arrays for k_gather: piece i, bytes[i] (a multiple of 4) from
+// src[i], goes to off[i] (a multiple of 16) of the destination
+constexpr uint32_t kGatherPieces = 24;
+struct GatherArgs {
+    const void *src[kGatherPieces];
+    uint32_t off[kGatherPieces], bytes[kGatherPieces];
+    uint32_t n;
+};
+// dst: pinned host memory as the device sees it; bytes: the end of the last piece
+hipError_t launch_gather(const GatherArgs &a, void *dst, size_t bytes, hipStream_t s);
+
 hipError_t launch_site_to_hap(const PanelDev &P, uint64_t *hap, hipStream_t s);
 hipError_t launch_panel_mono(const PanelDev &P, uint64_t *pand, uint64_t *por, hipStream_t s);
 hipError_t launch_distance(const PanelDev &P, const TgtDev *tg, const uint32_t *tlist,
