@@ -183,10 +183,10 @@ def panel_pbwt_bench(args):
         "bit_exact": exact,
         "element_steps_per_s": round(steps / (dev_ms / 1e3), 1),
         "with_copies_sites_per_s": round(M / wall, 1),
-        "roofline": {"bound": "hbm", "kernel": "k_panel_pbwt",
+        "roofline": {"bound": "hbm", "kernel": "k_order + k_dense",
                      "achieved": round((M * (N * 4 + 8 * ((N + 31) // 32)) + M * N / 8) / (dev_ms / 1e3) / 1e9, 2),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "traffic": None,
-                     "note": "one workgroup (one CU): the site loop is sequential"},
+                     "note": "the order chain, cut into segments, then all 16-row blocks in parallel"},
         "cpu_baseline": {"value": round(n / cpu_s, 1), "unit": "sites/s", "cores": 1,
                          "kind": "port", "sample": f"first {n} sites, oracle restatement"},
     }
@@ -299,7 +299,7 @@ def find_traffic(kernel_name, workload, targets_per_step, layout="gpu"):
 
 
 def find_sq(kernel_name, workload, layout="gpu"):
-    """Issue counters (SQ_INSTS_VALU etc. per wave-step) of kernel_name on this
+    """Issue counters (SQ_INSTS_VALU etc. per block) of kernel_name on this
     workload and output layout from a committed counter summary, if one was
     taken."""
     import glob
@@ -657,7 +657,7 @@ def batch_bench(args) -> dict:
     # what the PBWT kernel itself moves: rows written and the condensed
     # reference read by each direction
     kbytes_launch = float(pbwt_alg_bytes(Mp_all, K_all).sum()) / max(pbwt_launches, 1)
-    kernel_name = "k_pbwt" if args.engine == "batch" else "k_pbwt_persist"
+    kernel_name = "k_order + k_rows"
     traffic, traffic_src = find_traffic(kernel_name, cfg["name"], batch, args.layout)
     sq = find_sq(kernel_name, cfg["name"], args.layout)
 
@@ -820,14 +820,8 @@ def batch_bench(args) -> dict:
             "traffic_source": traffic_src,
             "traffic_over_alg": None if traffic is None else round(traffic / balg_launch, 3),
             "traffic_over_kernel_bytes": None if traffic is None else round(traffic / kbytes_launch, 3),
-            "limiter": None if sq is None else (
-                f"vector issue and the step's barrier/LDS latency: "
-                f"{sq['valu_per_wave_step']} VALU + {sq['salu_per_wave_step']} SALU + "
-                f"{sq['lds_per_wave_step']} LDS instructions per wave-step, VALU busy "
-                f"{100 * sq['valu_busy']:.1f}%; a step takes "
-                f"{sq.get('issue_model_ratio', float('nan'))} x issuing all of them one at a "
-                f"time at 4 cycles each"),
-            "sq": None if sq is None else {k: sq[k] for k in sq if k not in ("kernel", "workload")},
+            "limiter": None if sq is None else sq.get("limiter"),
+            "sq": None if sq is None else {k: sq[k] for k in sq if k not in ("kernel", "workload", "limiter")},
         },
         "kernel_ms": {k: round(v[0], 3) for k, v in tim.items()},
         "plain_targets_per_s": None if plain_tps is None else round(plain_tps, 3),

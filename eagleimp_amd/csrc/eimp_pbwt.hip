@@ -19,8 +19,8 @@
 // Carrying every haplotype through every row (two barriers and 5 vector
 // instructions per 64 haplotypes and row, one workgroup per chain for all
 // rows) took 32.3 ms for 192 targets of 15,000 rows at K = 10,000; the chain
-// now takes 8.7 ms and the rows 6.9 ms.  One target of 45,000 rows: 60.1 ms
-// before, 19.0 + 0.3 ms now.
+// now takes 9.0 ms and the rows 6.1 ms.  One target of 45,000 rows:
+// 61.3 and 2.8 ms for the whole call (its chain cut into segments).
 //
 // Blocks with more runs than k_rows takes and the last block of a target when
 // it has fewer than 16 rows are done row by row in k_order (order_dense).
@@ -39,24 +39,28 @@ namespace {
 // ---------------------------------------------------------------------------
 // k_rows: the 16 rows of a block from its run list, one wave per block.
 //
-// An entry is key << 16 | first position; entry i's run ends where entry i+1's
-// begins.  A last entry (all-ones key, position Kpad, no length) stands after
-// them; under the stable partition it stays last.  Per row j, lane x takes
-// entries [x Ej, x Ej + Ej) (Ej odd: no two lanes on one LDS bank):
-//   x = entry ^ previous entry; bit j of x: the row's bits change here, so
-//       position P is marked in the row's bit map: -2^P where ones begin, +2^P
-//       where they end (LDS add on the word)
-//   bits j.. of x all zero: the two runs stay together from here on; the
-//       entry is dropped (its length stays with the previous one)
-//   one packed prefix sum over the wave, {4 x entries kept, length} of the
-//       zeros, and one of 4 x entries kept give every entry's new index and
-//       first position: zeros in order from 0, ones after all zeros
-// then the entries are scattered (read into registers before), and the row's
-// words come from the marks: a word's sum, one less where a run goes on into
-// it (run_states), a scan of the words' zeros for the offsets.
-// Bound by vector instructions: about 18 per 64 entries and row and 40 per 64
+// An entry is key << 16 | length.  Behind the R runs stand empty runs of ones
+// up to 64 E entries, E odd (no two lanes on one LDS bank) and fixed for the
+// block; under the stable partition they stay there.  Per row, lane x takes
+// entries [x E, x E + E):
+//   one packed sum {length, ones} per lane and its prefix sum over the wave give
+//       the position and the ones before a lane's first entry; inside the lane
+//       both run along
+//   where the row's bit differs from the previous entry's, position P is marked
+//       in the row's bit map: -2^P where ones begin, +2^P where they end (LDS
+//       add on the word)
+//   the entry is written to its new place: zeros from entry 0, ones behind all
+//       zeros (every entry is in a register before)
+// then the row's words come from the marks: a word's sum, one less where a run
+// goes on into it (run_states), a scan of the words' zeros for the offsets.
+// Bound by vector instructions: 13 per 64 entries and row and about 40 per 64
 // word pairs and row; one wave per block because two barriers a row cost a
-// workgroup more than the wave's own latency.
+// workgroup more than the wave's own latency.  Entries with their first position
+// instead of the length, neighbours with equal remaining bits merged row by row,
+// took 28: the merging (2,400 entries of a block become 1,700 by its twelfth
+// row) cost more than it saved.  96 targets on the 200,000-haplotype panel
+// (2,750 runs a block): 8,106 us so, 5,232 us now; 192 whole-panel targets at
+// K = 10,000 (1,050 runs): 6,757 and 5,950 us; 256 windows: 12.3 and 10.8 ms.
 // ---------------------------------------------------------------------------
 // Lanes entered inside a run of ones, from what every lane does with that
 // state: f0 / f1 = lanes left inside a run when entered outside / inside one.
@@ -85,81 +89,54 @@ __device__ __forceinline__ uint64_t run_states(uint64_t f0, uint64_t f1, uint32_
     }
 }
 
-// Row of bit bm (in the key's half of an entry) on n entries: returns its zero
-// count, leaves the next row's entries and their number in n.
+// LDS of k_rows: entries from byte kRowsBias on (what a store address may lie
+// below its immediate offset), then the marks.
+constexpr uint32_t kRowsBias = 128;
+
+// Row of key bit `bit` (an entry's bit 16 + bit, bit < 8) on E entries per lane,
+// partitioned in place.
 template <int E>
-__device__ __forceinline__ uint32_t rows_step(const uint32_t bm, uint32_t &n, uint32_t *ent,
-                                              uint32_t *tog) {
+__device__ __forceinline__ void rows_step(const uint32_t bit, const bool halve, const lds_ptr_t<uint32_t> tog) {
     const uint32_t ln = opaque(lane_id());
-    const uint32_t first = ln * E;
-    uint32_t p[E + 1], dst[E];
-    const uint32_t pv = ent[ln ? first - 1 : 0];
+    const lds_ptr_t<uint32_t> mine = lds_at(kRowsBias) + ln * E;
+    uint32_t p[E];
 #pragma unroll
-    for (int e = 0; e <= E; e++) p[e] = ent[first + e];
-    // packed {4 x entries kept, length} prefix sums of my zeros (zacc) and my
-    // ones (oacc); an entry notes the sum of its own kind before it
-    uint32_t zacc = 0, oacc = 0, prev = ln ? pv : 0u;
-    // the conditions fit the scalar registers up to here; beyond, they are
-    // computed again
-    constexpr bool keep = E <= 17;
-    uint64_t kept[E], one[E];
-    uint32_t b = bm;
-    static_for<0, E>([&](auto ei) {
-        constexpr int e = decltype(ei)::value;
-        const uint32_t x = p[e] ^ prev;
-        prev = p[e];
-        one[e] = __ballot((p[e] & b) != 0u);
-        kept[e] = __ballot(x >= b) | (e == 0 ? 1ull : 0ull);
-        const uint64_t changed = e == 0 ? __ballot((x & b) != 0u) : one[e] ^ one[e ? e - 1 : 0];
-        if (__builtin_amdgcn_inverse_ballot_w64(changed)) {
-            const uint32_t P = p[e] & 0xFFFFu;
-            const uint32_t sign = __builtin_amdgcn_inverse_ballot_w64(one[e]) ? ~0u : 1u;
-            __hip_atomic_fetch_add(&tog[P >> 5], sign << (P & 31), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WAVEFRONT);
-        }
-        const uint32_t c = __builtin_amdgcn_inverse_ballot_w64(kept[e]) ? 0x40000u : 0u;
-        const uint32_t w = ((p[e + 1] - p[e]) & 0xFFFFu) | c;
-        const bool o = __builtin_amdgcn_inverse_ballot_w64(one[e]);
-        dst[e] = o ? oacc : zacc;
-        const uint32_t wz = o ? 0u : w;
-        zacc += wz;
-        oacc += w - wz;
-        // four entries at a time: the next ones wait for these sums
-        if constexpr (e % 4 == 3) {
-            asm volatile("" : "+v"(zacc), "+v"(oacc), "+s"(b));
-            static_for<e + 2, (e + 6 < E + 1 ? e + 6 : E + 1)>(
-                [&](auto k) { hold(p[decltype(k)::value]); });
-        }
-    });
-    const uint32_t zx = lane_scan_excl<64>(zacc), ox = lane_scan_excl<64>(oacc);
-    const uint32_t ztot = (uint32_t)__builtin_amdgcn_readlane((int)(zx + zacc), 63);
-    const uint32_t otot = (uint32_t)__builtin_amdgcn_readlane((int)(ox + oacc), 63);
-    wave_order();
-    // zeros from index and position 0, ones behind them all
-    const uint32_t ob = ox + ztot;
-    if constexpr (!keep) {
-        b = bm;
-        asm volatile("" : "+s"(b) : "s"(ztot));
-        prev = ln ? pv : 0u;
+    for (int e = 0; e < E; e++) p[e] = mine[e];
+    if (halve) {  // rows 8..15: their bits come down
+#pragma unroll
+        for (int e = 0; e < E; e++) p[e] = __builtin_amdgcn_perm(p[e], p[e], 0x0C030100u);
     }
+    // {length, ones} of my entries: no more than 61 ones above a length of at
+    // most 32,768
+    uint32_t bm = opaque_s(0x10000u << bit), acc = 0;
+    const uint32_t am = bm | 0xFFFFu;
+    static_for<0, E>([&](auto ei) { acc += p[decltype(ei)::value] & am; });
+    const uint32_t sum = (acc & 0xFFFFu) | (acc >> (16 + bit) << 16);
+    const uint32_t ex = lane_scan_excl<64>(sum);
+    const uint32_t nz = 64u * E - ((uint32_t)__builtin_amdgcn_readlane((int)(ex + sum), 63) >> 16);
+    uint64_t before = __ballot((p[E - 1] & bm) != 0u) << 1;  // the entry before each lane's first
+    wave_order();
+    // y ones before the entry: a one goes to entry nz + y, a zero to (E ln + e) -
+    // y; in bytes less 2 e, the store's immediate offset, that is x and V - x,
+    // and x grows by 2 behind a one and falls by 2 behind a zero
+    uint32_t x = 4u * ((ex >> 16) + nz) + kRowsBias, P = ex & 0xFFFFu;
+    const uint32_t V = 4u * (E * ln + nz) + 2u * kRowsBias;
     static_for<0, E>([&](auto ei) {
         constexpr int e = decltype(ei)::value;
-        if constexpr (!keep) {
-            one[e] = __ballot((p[e] & b) != 0u);
-            kept[e] = __ballot((p[e] ^ prev) >= b) | (e == 0 ? 1ull : 0ull);
-            prev = p[e];
-        }
-        const uint32_t to = dst[e] + (__builtin_amdgcn_inverse_ballot_w64(one[e]) ? ob : zx);
-        if (__builtin_amdgcn_inverse_ballot_w64(kept[e]))
-            *(uint32_t *)((char *)ent + (to >> 16)) = (p[e] & 0xFFFF0000u) | (to & 0xFFFFu);
-        if constexpr (!keep && e % 4 == 3) {
-            asm volatile("" : "+s"(b)::"memory");
-            static_for<e + 1, (e + 5 < E ? e + 5 : E)>(
-                [&](auto k) { hold(p[decltype(k)::value]); });
-        }
+        const uint64_t one = __ballot((p[e] & bm) != 0u);
+        const uint64_t changed = one ^ before;
+        before = one;
+        const bool o = __builtin_amdgcn_inverse_ballot_w64(one);
+        const uint32_t to = o ? x : V - x;
+        *(lds_ptr_t<uint32_t>)(size_t)(to + 2u * e) = p[e];
+        x += o ? 2u : ~1u;
+        if (__builtin_amdgcn_inverse_ballot_w64(changed))
+            __hip_atomic_fetch_add(&tog[P >> 5], (o ? ~0u : 1u) << (P & 31), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WAVEFRONT);
+        P += p[e] & 0xFFFFu;
+        if constexpr (e % 4 == 3) asm volatile("" : "+v"(x), "+v"(P), "+s"(bm));
     });
-    n = (ztot + otot) >> 18;
-    return ztot & 0xFFFFu;
+    wave_order();
 }
 
 // Entries per lane instantiated, all odd: 1, 3, .. 17, then 21, 25, .. 61
@@ -181,10 +158,9 @@ __device__ __forceinline__ void dispatch(uint32_t i, F &&f) {
     }
 }
 
-template <int EMAX>
+template <int E>
 __device__ __forceinline__ void rows_block(const TgtDev &T, const bool rev, const uint32_t q,
-                                           const uint32_t R, uint32_t *ent, uint32_t *tog,
-                                           uint64_t &dsum) {
+                                           const uint32_t R, const lds_ptr_t<uint32_t> tog, uint64_t &dsum) {
     const uint32_t ln = lane_id();
     const uint32_t K = T.K, Mp = T.Mp, Kpad = T.Kpad, RS = T.RS;
     const uint32_t nblk = (Mp + 15) / 16, nch = Kpad / 64, npairs = (K + 31) / 32, KW = 2 * npairs;
@@ -192,11 +168,25 @@ __device__ __forceinline__ void rows_block(const TgtDev &T, const bool rev, cons
     const bool raw = (T.flags & TF_RAW) != 0;
     const bool dig = T.digest != nullptr;
     const gptr_t<uint32_t> outrow = gmem(T.out) + ((rev ? (uint64_t)Mp : 0ull) + geo.s0) * RS;
-    const uint32_t endv = 0xFFFF0000u | Kpad;
-    for (uint32_t i = ln; i < R; i += 64) ent[i] = outrow[i];
-    uint32_t n = R + 1;  // entries, the last one included
-    uint32_t ie = row_entries_index(n);
-    for (uint32_t i = R + ln; i <= 64u * (uint32_t)row_entries_at((int)ie); i += 64) ent[i] = endv;
+    // run list (key, first position) to entries (key, length); behind them
+    // empty runs of ones, which stay there
+    const lds_ptr_t<uint32_t> ent = lds_at(kRowsBias);
+    constexpr int B = 8;  // slots whose loads are in flight together
+    static_for<0, (E + B - 1) / B>([&](auto bi) {
+        constexpr int e0 = decltype(bi)::value * B, e1 = e0 + B < E ? e0 + B : E;
+        uint32_t here[B], next[B];
+#pragma unroll
+        for (int e = e0; e < e1; e++) {
+            const uint32_t i = 64 * e + ln;
+            here[e - e0] = outrow[min(i, R - 1)];
+            next[e - e0] = outrow[min(i + 1, R - 1)];
+        }
+#pragma unroll
+        for (int e = e0; e < e1; e++) {
+            const uint32_t i = 64 * e + ln, h = here[e - e0], len = (i + 1 < R ? next[e - e0] : Kpad) - h;
+            ent[i] = i < R ? (h & 0xFFFF0000u) | (len & 0xFFFFu) : 0xFFFF0000u;
+        }
+    });
     const uint32_t pw0 = raw ? 2 * nch : 2 * npairs, tw = (RS - pw0) / 2;  // padding pairs of a row
     const uint32_t fw = raw ? ~0u : 0u;
     uint32_t g0 = (rev ? Mp * KW : 0u) + geo.s0 * KW;
@@ -204,17 +194,7 @@ __device__ __forceinline__ void rows_block(const TgtDev &T, const bool rev, cons
     wave_order();
 #pragma unroll 1
     for (uint32_t j = 0; j < 16; j++) {
-        uint32_t cnt0 = 0;
-        // the largest index this kernel reaches
-        constexpr int top = EMAX <= 17 ? EMAX / 2 : 8 + (EMAX - 17) / 4;
-        dispatch<0, top + 1>(ie, [&](auto ii) {
-            cnt0 = rows_step<row_entries_at(decltype(ii)::value)>(0x10000u << j, n, ent, tog);
-        });
-        c0acc = eimp_llvm_writelane(cnt0, j, c0acc);
-        ie = row_entries_index(n);
-        // entries past the last one: no length, never kept
-        for (uint32_t i = n + ln; i <= 64u * (uint32_t)row_entries_at((int)ie); i += 64) ent[i] = endv;
-        wave_order();
+        rows_step<E>(j & 7u, j == 8, tog);
         // the row's words: 64 positions per lane
         const gptr_t<uint32_t> row = outrow + (uint64_t)j * RS;
         uint32_t zrun = 0, state = 0;
@@ -223,8 +203,9 @@ __device__ __forceinline__ void rows_block(const TgtDev &T, const bool rev, cons
             const bool in = ch < nch;
             u32x2 t = u32x2{0u, 0u};
             if (in) {
-                t = *(u32x2 *)(tog + 2 * ch);
-                *(u32x2 *)(tog + 2 * ch) = u32x2{0u, 0u};
+                const lds_ptr_t<u32x2> w = (lds_ptr_t<u32x2>)(tog + 2 * ch);
+                t = *w;
+                *w = u32x2{0u, 0u};
             }
             // a word with marks +2^e at the ends and -2^s at the starts of
             // its one-runs is their sum, less one if a run goes on into it;
@@ -235,7 +216,7 @@ __device__ __forceinline__ void rows_block(const TgtDev &T, const bool rev, cons
             const uint32_t lo = t[0] - (__builtin_amdgcn_inverse_ballot_w64(entered) ? 1u : 0u);
             const uint32_t hi = t[1] + (uint32_t)((int32_t)lo >> 31);
             const uint32_t z0 = 32u - (uint32_t)__popc(lo);
-            const uint32_t zl = z0 + 32u - (uint32_t)__popc(hi);
+            const uint32_t zl = in ? z0 + 32u - (uint32_t)__popc(hi) : 0u;
             const uint32_t zex = lane_scan_excl<64>(zl);
             const uint32_t o1 = zrun + zex + z0, o3 = zrun + zex + zl;
             zrun += (uint32_t)__builtin_amdgcn_readlane((int)(zex + zl), 63);
@@ -261,11 +242,12 @@ __device__ __forceinline__ void rows_block(const TgtDev &T, const bool rev, cons
                 }
             }
         }
+        c0acc = eimp_llvm_writelane(zrun, j, c0acc);
         if (ln < tw) *(gptr_t<u32x2>)(row + pw0 + 2 * ln) = u32x2{fw, fw};
         g0 += KW;
+        if (ln == 0) tog[Kpad / 32] = 0;  // the end of ones before the empty runs
         wave_order();
     }
-    if (ln == 0) tog[Kpad / 32] = 0;  // the last entry's toggle
     if (!rev && ln < 16) gmem(T.count0)[geo.s0 + ln] = (int32_t)c0acc;
     wave_order();
 }
@@ -346,9 +328,11 @@ __attribute__((amdgpu_waves_per_eu(KERNEL == 0 ? 6 : (KERNEL == 1 ? 4 : (KERNEL 
     const TgtDev *__restrict__ tg, const uint32_t *__restrict__ d_n, uint32_t n,
     const uint32_t *__restrict__ pref, const RowItem *__restrict__ list,
     const uint32_t *__restrict__ cnt, uint32_t ntog) {
-    extern __shared__ uint32_t smem[];
     constexpr int EMAX = kRowsEntries[KERNEL];
-    uint32_t *ent = smem, *tog = smem + 64 * EMAX + 2;
+    // the indexes of the sizes of this kernel
+    constexpr int top = EMAX <= 17 ? EMAX / 2 : 8 + (EMAX - 17) / 4;
+    constexpr int low = KERNEL == 0 ? 0 : 8 + (kRowsEntries[KERNEL ? KERNEL - 1 : 0] - 17) / 4 + 1;
+    const lds_ptr_t<uint32_t> tog = lds_at(kRowsBias) + 64 * EMAX;
     const uint32_t items = cnt[KERNEL];
     if (blockIdx.x >= items) return;
     const uint32_t total = pref[d_n ? *d_n : n];
@@ -358,7 +342,9 @@ __attribute__((amdgpu_waves_per_eu(KERNEL == 0 ? 6 : (KERNEL == 1 ? 4 : (KERNEL 
         const RowItem it = list[list_at(KERNEL, total, i)];
         const TgtDev &T = tg[it.chain >> 1];
         uint64_t dsum = 0;
-        rows_block<EMAX>(T, (it.chain & 1u) != 0, it.q, it.runs, ent, tog, dsum);
+        dispatch<low, top + 1>(row_entries_index(it.runs + 1), [&](auto ii) {
+            rows_block<row_entries_at(decltype(ii)::value)>(T, (it.chain & 1u) != 0, it.q, it.runs, tog, dsum);
+        });
         if (T.digest) {
             dsum = wave_sum64(dsum);
             if (lane_id() == 0)
@@ -582,7 +568,7 @@ hipError_t launch_rows(const TgtDev *tg, const uint32_t *d_n, uint32_t n, const 
     for (int k = 0; k < kRowsKernels; k++) {
         if (k && Kpad / 2 + 1 <= 64u * (uint32_t)kRowsEntries[k - 1]) break;
         const uint32_t ntog = Kpad / 32 + 2;
-        const size_t lds = (64 * (size_t)kRowsEntries[k] + 2 + ntog) * 4;
+        const size_t lds = kRowsBias + (64 * (size_t)kRowsEntries[k] + ntog) * 4;
         int occ = 0;
         hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void *)fns[k], 64, lds);
         if (e != hipSuccess) return e;
