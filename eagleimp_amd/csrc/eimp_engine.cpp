@@ -171,7 +171,6 @@ struct HostCopier {
         size_t bytes;
     };
     std::mutex mu;
-    hipStream_t own = nullptr;
     hipEvent_t ev[kBufs] = {};
     HostBuf buf;
     std::vector<Chunk> chunks;
@@ -196,13 +195,10 @@ struct HostCopier {
     // device resources (the device is current)
     void release() {
         std::lock_guard<std::mutex> lk(mu);
-        if (own) (void)hipStreamSynchronize(own);
         for (auto &e : ev) {
             if (e) (void)hipEventDestroy(e);
             e = nullptr;
         }
-        if (own) (void)hipStreamDestroy(own);
-        own = nullptr;
         buf.release();
     }
     void slice(uint32_t t) {
@@ -239,14 +235,9 @@ struct HostCopier {
     void quiesce() {
         while (active.load(std::memory_order_acquire)) std::this_thread::yield();
     }
-    // Copies the jobs; the sources are complete, or written by work on s.
-    // s: the stream to copy on, or null for one of its own.
+    // Copies the jobs on s; the sources are complete, or written by work on s.
     int run(const std::vector<Job> &jobs, hipStream_t s) {
         std::lock_guard<std::mutex> lk(mu);
-        if (!s) {
-            if (!own) HIPCHK(hipStreamCreateWithFlags(&own, hipStreamNonBlocking));
-            s = own;
-        }
         chunks.clear();
         for (const Job &j : jobs) {
             if (!j.bytes) continue;
@@ -278,7 +269,7 @@ struct HostCopier {
             HIPCHK(hipStreamSynchronize(s));
             return EIMP_OK;
         }
-        CHK(buf.ensure(nc == 1 ? std::min(kChunk, std::max<size_t>(chunks[0].bytes, 256u << 10)) : kBufs * kChunk));
+        CHK(buf.ensure(nc == 1 ? std::min(kChunk, std::max<size_t>(chunks[0].bytes, 64u << 10)) : kBufs * kChunk));
         for (auto &d : done) d.store(0, std::memory_order_relaxed);
         ready.store(0, std::memory_order_relaxed);
         auto launch = [&](uint32_t c) {
@@ -956,7 +947,7 @@ int copy_target_out(const TgtDev &T, const TgtDev *d_tg, uint32_t t, uint64_t Na
         HIPCHK(hipStreamSynchronize(s));
         jobs.push_back({cref_rows, tmp.p, (size_t)T.Mp * rw * 8});
     }
-    return copier.run(jobs, nullptr);
+    return copier.run(jobs, s);
 }
 
 // Mono bits of a target (Target::findMonos, src/Target.cpp:878-897: site m
@@ -1871,7 +1862,7 @@ int eimp_engine_ref_pbwt(eimp_engine *e, size_t m0, size_t nsites, uint32_t *row
     if (b) e->event_pool.push_back(b);
     std::vector<HostCopier::Job> jobs{{rows, e->p_rows.p, nsites * RS * 4}, {count0, e->p_c0.p, nsites * 4}};
     if (absperm) jobs.push_back({absperm, e->p_abs.p, (nsites + 1) * N * 4});
-    return e->copier.run(jobs, nullptr);
+    return e->copier.run(jobs, e->stream);
 }
 
 int eimp_engine_set_timing(eimp_engine *e, int enable) {

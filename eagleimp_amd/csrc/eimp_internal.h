@@ -111,7 +111,7 @@ struct CrefItem {
 // haplotypes) into at least `want` items where it can be: first the
 // haplotypes into parts, then groups of 32 blocks.  A batch with that many
 // groups stays whole: smaller groups read more of each row's cache lines
-// twice (96 targets on the 200,000-haplotype panel: 3.5 ms whole).
+// twice (96 targets on the 200,000-haplotype panel are 1.6 ms whole).
 __host__ __device__ inline void cref_cut(uint32_t n128, uint32_t K, uint32_t want, uint32_t &grp,
                                          uint32_t &parts) {
     const uint32_t passes = (K + kCrefThreads - 1) / kCrefThreads;

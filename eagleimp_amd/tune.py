@@ -1,5 +1,5 @@
 """Autotuner for the stream-context path: picks the PBWT kernel variant
-(threads per workgroup x chunks per wave, which fixes the workgroup's LDS and
+(threads per workgroup x positions per thread, which fixes the workgroup's LDS and
 so the resident workgroups per CU) and the targets per submission, by timing
 a sample batch of the actual workload through timed contexts (HIP events
 between the kernel classes).  Results are cached per panel shape, K range,

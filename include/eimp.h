@@ -151,9 +151,10 @@ int eimp_engine_run_batch(eimp_engine *engine, size_t n, const eimp_target *targ
  * rows[t] to 2*Mp*rowstride uint32 and count0[t] to Mp int32 of device
  * memory (rowstride as the layout flag chooses; Mp <= max_Mp, which the
  * caller sizes the buffers by).  Everything else (distances, best haps,
- * split data, condensed reference, tables) lives in a fixed 64 MiB device
- * scratch array that every device running the library holds until the
- * process ends; a batch needing more, more than 256 targets, or an Mp above
+ * split data, condensed reference, tables) lives in a fixed device scratch
+ * array, 64 MiB and as much again for the PBWT's tables, that every device
+ * running the library holds until the process ends; a batch needing more than
+ * either part, more than 256 targets, or an Mp above
  * max_Mp fails with EIMP_ERR_UNSUPPORTED.  The panel parts a batch reads must
  * be resident already: the mono bits are built by
  * eimp_engine_set_panel_extras, the hap-major rows (targets with K < Ncorr or
@@ -301,7 +302,8 @@ int eimp_engine_get_timing(eimp_engine *engine, double *ms, uint64_t *launches);
 int eimp_engine_reset_timing(eimp_engine *engine);
 
 /* PBWT kernel variant: -1 automatic, otherwise an index into the engine's
- * variant table (threads per workgroup x chunks per wave); the autotuner in
+ * variant table (threads per workgroup x positions per thread, which is chunks of
+ * 64 positions per wave); the autotuner in
  * the Python package sweeps these. */
 int eimp_engine_set_pbwt_variant(eimp_engine *engine, int variant);
 int eimp_pbwt_variant_count(void);
