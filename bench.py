@@ -630,7 +630,9 @@ def batch_bench(args) -> dict:
         pbwt_launches = len(results)
         pbwt_ms = kms.get("pbwt", 0.0)
         tim["pbwt"] = (pbwt_ms, pbwt_launches)
-        if args.graph_steps > 0:
+        # with one context, as in the timed passes' other mode; a shared pool's
+        # contexts are timed only
+        if args.graph_steps > 0 and not share:
             gsts = contexts(timed=False)
             pipeline(gsts, 1, 0)
             t = time.perf_counter()
