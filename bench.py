@@ -372,7 +372,8 @@ def main():
                     help="stream engine: pick the PBWT variant and targets per submission with "
                          "the autotuner on a sample of the workload first")
     ap.add_argument("--graph-steps", type=int, default=2,
-                    help="steps replayed through captured hipGraphs after the timed region")
+                    help="steps replayed through captured hipGraphs after the timed region (not "
+                         "with a shared pool)")
     ap.add_argument("--phase", action="store_true",
                     help="phasing (beam search) over device-built cPBWTs on host threads, "
                          "beside the reference's beam")
@@ -612,29 +613,36 @@ def batch_bench(args) -> dict:
         for ci, st in enumerate(sts):
             if ci in last:
                 b, res = last[ci]
+                log(f"context {ci}: digests of the stored outputs")
                 try:
                     dp, dc = st.digest_outputs()
                 except EimpError:
                     # a context sharing the pool has built over these outputs
+                    log(f"context {ci}: built over, close")
                     st.close()
                     continue
                 for j, t in enumerate(b):
                     if int(res.Mp[j]) > 0:
                         if not post and not args.no_cpu:
                             # the first of them is also compared byte for byte
+                            log(f"context {ci}: copy of target {t}")
                             stored = (t, st.copy_target(j))
                         post[t] = (int(res.Mp[j]), int(dp[j]), int(dc[j]))
+            log(f"context {ci}: close")
             st.close()
         tim = {k: (v, 0) for k, v in kms.items()}
         # one PBWT launch per submission
         pbwt_launches = len(results)
         pbwt_ms = kms.get("pbwt", 0.0)
         tim["pbwt"] = (pbwt_ms, pbwt_launches)
-        # with one context, as in the timed passes' other mode; a shared pool's
-        # contexts are timed only
+        # contexts on a shared pool replay no graphs (a run that did, on the
+        # 20,000 x 200,000 workload, did not return; cause not known)
         if args.graph_steps > 0 and not share:
+            log("graph contexts")
             gsts = contexts(timed=False)
+            log("graph replay: warmup")
             pipeline(gsts, 1, 0)
+            log("graph replay: timed steps")
             t = time.perf_counter()
             gres, _, _ = pipeline(gsts, args.graph_steps, args.warmup)
             gwall = time.perf_counter() - t

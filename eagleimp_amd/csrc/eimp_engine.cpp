@@ -1149,10 +1149,14 @@ int run_batch_impl(eimp_engine *e, size_t n, const eimp_target *targets, float c
 // build then waits for the pool's previous build, whichever context ran it,
 // while the preparation of a submission runs beside the other context's
 // build.  A context's pool outputs stay valid until a context sharing the
-// pool submits again.
+// pool submits again.  Such contexts launch their kernels one by one: a run of
+// two contexts of 1,024 targets on one pool of 274 GiB did not come back from
+// the steps after its timed passes, the last of which replayed both contexts'
+// graphs.  Whether the replay held it up was not shown; the timed passes, which
+// launch one by one, ended as they should.
 // ---------------------------------------------------------------------------
 // Contexts sharing a pool may be driven from different host threads: `mu`
-// guards seq and last_build, and is held from the wait on the previous build
+// guards seq, shared and last_build, and is held from the wait on the previous build
 // to the record of the new one, and across every synchronous read of pool
 // rows, so a build is never enqueued while another context reads them.
 struct StreamPool {
@@ -1160,6 +1164,7 @@ struct StreamPool {
     uint64_t cap = 0;
     std::mutex mu;
     uint64_t seq = 0;                 // builds submitted into the pool
+    bool shared = false;              // more than one context has used it: no graph replay
     hipEvent_t last_build = nullptr;  // the last submitted build's event (its context owns it)
 };
 
@@ -1361,6 +1366,8 @@ int stream_setup(eimp_stream *s, size_t pool_bytes, const std::shared_ptr<Stream
     CHK(s->d_rowlist.ensure(2 * nmax * hdr_n * sizeof(RowItem), "row items"));
     if (pool) {
         s->pool = pool;
+        std::lock_guard<std::mutex> lk(pool->mu);
+        pool->shared = true;
     } else {
         s->pool = std::make_shared<StreamPool>();
         CHK(s->pool->buf.ensure(pool_bytes, "output pool", false));
@@ -1414,7 +1421,7 @@ int stream_setup(eimp_stream *s, size_t pool_bytes, const std::shared_ptr<Stream
         T.stats = s->d_stats.as<uint32_t>() + 4 * t;
         T.hdr = s->d_hdr.as<uint16_t>() + t * hdr_n;
     }
-    if (!(s->flags & (EIMP_STREAM_NO_GRAPH | EIMP_STREAM_TIMED))) {
+    if (!pool && !(s->flags & (EIMP_STREAM_NO_GRAPH | EIMP_STREAM_TIMED))) {
         CHK(stream_capture(s, stream_launch_prep, &s->graph_prep, &s->exec_prep));
         CHK(stream_capture(s, stream_launch_build, &s->graph_build, &s->exec_build));
     }
@@ -1978,12 +1985,17 @@ int eimp_stream_submit(eimp_stream *s, size_t n, const eimp_target *targets, flo
     if (gw) HIPCHK(hipMemcpyAsync(gtdev, gtst, gw * 8, hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipEventRecord(s->ev[1], s->stream));
     if (nt) {
-        if (s->exec_prep) HIPCHK(hipGraphLaunch(s->exec_prep, s->stream));
+        bool replay = s->exec_prep && s->exec_build;
+        if (replay) {
+            std::lock_guard<std::mutex> lk(s->pool->mu);
+            replay = !s->pool->shared;
+        }
+        if (replay) HIPCHK(hipGraphLaunch(s->exec_prep, s->stream));
         else CHK(stream_launch_prep(s));
         // the pool's previous build (this context's or another's) ends first
         std::lock_guard<std::mutex> lk(s->pool->mu);
         if (s->pool->last_build) HIPCHK(hipStreamWaitEvent(s->stream, s->pool->last_build, 0));
-        if (s->exec_build) HIPCHK(hipGraphLaunch(s->exec_build, s->stream));
+        if (replay) HIPCHK(hipGraphLaunch(s->exec_build, s->stream));
         else CHK(stream_launch_build(s));
         HIPCHK(hipEventRecord(s->build_done, s->stream));
         s->pool->last_build = s->build_done;

@@ -227,7 +227,9 @@ int eimp_stream_create(eimp_engine *engine, size_t max_targets, size_t max_windo
  * (distances, top-K, monos, call locations) runs beside that build.  A
  * context's outputs in the pool (count0, rows, cref) stay valid until any
  * context sharing the pool submits again; copying them afterwards returns
- * EIMP_ERR_STATE.  The pool lives until its last context is destroyed. */
+ * EIMP_ERR_STATE.  The contexts of a shared pool, `other` included, launch their
+ * kernels one by one (as with EIMP_STREAM_NO_GRAPH).  The pool lives until its
+ * last context is destroyed. */
 int eimp_stream_create_shared(eimp_stream *other, size_t max_targets, size_t max_window,
                               size_t max_K, uint32_t flags, eimp_stream **stream);
 
