@@ -236,8 +236,15 @@ struct HostCopier {
         while (active.load(std::memory_order_acquire)) std::this_thread::yield();
     }
     // Copies the jobs on s; the sources are complete, or written by work on s.
+    // After an error too, nothing writes to a destination or a chunk any more
+    // when this returns.
     int run(const std::vector<Job> &jobs, hipStream_t s) {
         std::lock_guard<std::mutex> lk(mu);
+        const int rc = copy(jobs, s);
+        if (rc != EIMP_OK) (void)hipStreamSynchronize(s);
+        return rc;
+    }
+    int copy(const std::vector<Job> &jobs, hipStream_t s) {
         chunks.clear();
         for (const Job &j : jobs) {
             if (!j.bytes) continue;
@@ -300,10 +307,7 @@ struct HostCopier {
         }
         cv.notify_all();
         const int rc = pump(nc, s, launch);
-        if (rc != EIMP_OK) {
-            abort.store(true, std::memory_order_relaxed);
-            (void)hipStreamSynchronize(s);
-        }
+        if (rc != EIMP_OK) abort.store(true, std::memory_order_relaxed);
         quiesce();
         return rc;
     }

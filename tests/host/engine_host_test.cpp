@@ -161,6 +161,37 @@ void shared_pool_without_graphs(int) {
     eimp_engine_destroy(e);
 }
 
+// A copy that fails returns only when nothing writes to the caller's memory any
+// more: the rows go straight to pinned memory, then the chunks' buffer cannot be
+// had, or the gather of the other array does not start.
+void failed_copy_leaves_nothing_in_flight(int) {
+    eimp_engine *e = engine();
+    const Batch b({{20000, 512}});
+    auto s = shared_contexts(e, 1, 0);
+    submit(s[0], b);
+    wait(s[0], b);
+    const size_t Mp = 2 * (20000 / 4) + 1, words = 2 * Mp * row_stride(512, LAYOUT_GPU);
+    void *rows = nullptr;
+    REQUIRE(hipHostMalloc(&rows, words * 4, 0) == hipSuccess);
+    std::vector<int32_t> c0(Mp);
+    stub.copy_us = 30000;
+    for (int way = 0; way < 2; way++) {
+        stub.copies = stub.copies_done = stub.gathers = 0;
+        stub.fail_host_malloc = way == 0;
+        stub.fail_gather = way == 1 ? 0 : -1;
+        REQUIRE(eimp_stream_copy_target(s[0], 0, nullptr, nullptr, nullptr, nullptr, nullptr, c0.data(),
+                                        static_cast<uint32_t *>(rows), nullptr) != EIMP_OK);
+        REQUIRE(stub.copies == 1 && stub.copies_done == 1);
+    }
+    stub.fail_host_malloc = false;
+    stub.fail_gather = -1;
+    stub.copy_us = 0;
+    check_copy(s[0], b, 0);
+    (void)hipHostFree(rows);
+    eimp_stream_destroy(s[0]);
+    eimp_engine_destroy(e);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -169,6 +200,7 @@ int main(int argc, char **argv) {
     if (name == "shared_pool_sequence") shared_pool_sequence(rounds);
     else if (name == "shared_pool_threads") shared_pool_threads(rounds);
     else if (name == "shared_pool_without_graphs") shared_pool_without_graphs(rounds);
+    else if (name == "failed_copy_leaves_nothing_in_flight") failed_copy_leaves_nothing_in_flight(rounds);
     else return 2;
     std::printf("ok %s\n", name.c_str());
     return 0;

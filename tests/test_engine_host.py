@@ -41,3 +41,7 @@ def test_shared_pool_on_two_threads(host):
 
 def test_shared_pool_without_graphs(host):
     host("shared_pool_without_graphs")
+
+
+def test_failed_copy_leaves_nothing_in_flight(host):
+    host("failed_copy_leaves_nothing_in_flight")
