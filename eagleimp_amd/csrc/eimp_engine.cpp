@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <cstdio>
 #include <cstring>
@@ -17,7 +18,6 @@
 #include <memory>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -150,7 +150,10 @@ struct HostBuf {
 // Here the arrays are one byte stream, cut into chunks that a kernel gathers
 // into pinned buffers (k_gather: one launch per chunk, however many arrays it
 // holds), several chunks ahead of the host, and from two chunks on a small team
-// of threads copies the slices of the chunks that have arrived.  Whole calls,
+// of threads copies the slices of the chunks that have arrived.  The team is
+// woken when the first chunk has arrived, and a thread that waits for a later one
+// for more than kSpin sleeps: the work before the copy, or another context's
+// kernels beside it, can take far longer than the copy.  Whole calls,
 // before and now: three targets of 256 haplotypes with all their arrays 692 and
 // 444 us; one target with 15 MB of rows 3,069 and 1,843 us; 12 targets with
 // 92 MB 6,003 and 2,671 us; 30 MB of panel orders 2,650 and 1,672 us.
@@ -160,6 +163,8 @@ struct HostCopier {
     static constexpr size_t kChunk = 2u << 20, kBufs = 4, kAlign = 16;
     static constexpr uint32_t kSlices = 8;   // per chunk
     static constexpr uint32_t kThreads = 3;  // beside the caller
+    // a 2 MiB chunk arrives about every 40 us where nothing holds it up
+    static constexpr std::chrono::microseconds kSpin{100};
     struct Job {
         void *dst;
         const void *src;
@@ -177,7 +182,8 @@ struct HostCopier {
     // the team: woken by gen, takes slices by ticket, leaves when none is left
     std::vector<std::thread> team;
     std::mutex tm;
-    std::condition_variable cv;
+    std::condition_variable cv, arrived;
+    std::atomic<uint32_t> asleep{0};  // team threads waiting on `arrived`
     uint64_t gen = 0;
     bool quit = false, no_team = false;
     std::atomic<uint32_t> active{0}, next{0}, ready{0}, total{0};
@@ -223,14 +229,52 @@ struct HostCopier {
             }
             for (;;) {
                 const uint32_t t = next.fetch_add(1, std::memory_order_relaxed);
-                if (t >= total.load(std::memory_order_acquire)) break;
-                while (ready.load(std::memory_order_acquire) <= t / kSlices && !abort.load(std::memory_order_relaxed))
-                    std::this_thread::yield();
-                if (ready.load(std::memory_order_acquire) <= t / kSlices) break;
+                if (t >= total.load(std::memory_order_acquire) || !await(t / kSlices)) break;
                 slice(t);
             }
             active.fetch_sub(1, std::memory_order_release);
         }
+    }
+    // team threads: until chunk c has arrived; false: the copy has failed
+    bool await(uint32_t c) {
+        const auto until = std::chrono::steady_clock::now() + kSpin;
+        while (ready.load() <= c) {
+            if (abort.load()) return false;
+            if (std::chrono::steady_clock::now() < until) {
+                std::this_thread::yield();
+                continue;
+            }
+            std::unique_lock<std::mutex> lk(tm);
+            asleep++;
+            arrived.wait(lk, [&] { return ready.load() > c || abort.load(); });
+            asleep--;
+        }
+        return true;
+    }
+    // after `ready` or `abort` was set (all sequentially consistent: a thread that
+    // is not counted yet sees the new value)
+    void tell() {
+        if (!asleep.load()) return;
+        { std::lock_guard<std::mutex> lk(tm); }
+        arrived.notify_all();
+    }
+    // the team as it is (device work under way meanwhile), then its start
+    void gather_team() {
+        while (team.size() < kThreads && !no_team) {
+            try {
+                team.emplace_back([this] { work(); });
+            } catch (const std::exception &) {
+                no_team = true;  // the caller alone, with the threads there are
+            }
+        }
+    }
+    void start_team() {
+        active.store((uint32_t)team.size(), std::memory_order_relaxed);
+        {
+            std::lock_guard<std::mutex> lk(tm);
+            gen++;
+        }
+        cv.notify_all();
     }
     void quiesce() {
         while (active.load(std::memory_order_acquire)) std::this_thread::yield();
@@ -278,7 +322,7 @@ struct HostCopier {
         }
         CHK(buf.ensure(nc == 1 ? std::min(kChunk, std::max<size_t>(chunks[0].bytes, 64u << 10)) : kBufs * kChunk));
         for (auto &d : done) d.store(0, std::memory_order_relaxed);
-        ready.store(0, std::memory_order_relaxed);
+        ready.store(0);
         auto launch = [&](uint32_t c) {
             return launch_gather(chunks[c].args, buf.as<char>() + (c % kBufs) * kChunk, chunks[c].bytes, s);
         };
@@ -290,24 +334,14 @@ struct HostCopier {
         }
         for (auto &e : ev)
             if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        while (team.size() < kThreads && !no_team) {
-            try {
-                team.emplace_back([this] { work(); });
-            } catch (const std::system_error &) {
-                no_team = true;  // the caller alone, with the threads there are
-            }
-        }
-        abort.store(false, std::memory_order_relaxed);
+        abort.store(false);
         next.store(0, std::memory_order_relaxed);
         total.store(nc * kSlices, std::memory_order_release);
-        active.store((uint32_t)team.size(), std::memory_order_relaxed);
-        {
-            std::lock_guard<std::mutex> tl(tm);
-            gen++;
-        }
-        cv.notify_all();
         const int rc = pump(nc, s, launch);
-        if (rc != EIMP_OK) abort.store(true, std::memory_order_relaxed);
+        if (rc != EIMP_OK) {
+            abort.store(true);
+            tell();
+        }
         quiesce();
         return rc;
     }
@@ -319,10 +353,13 @@ struct HostCopier {
             return (int)EIMP_OK;
         };
         for (uint32_t c = 0; c < std::min<uint32_t>(nc, kBufs); c++) CHK(go(c));
+        gather_team();
         uint32_t mine = ~0u;  // a ticket of a chunk that has not arrived
         for (uint32_t c = 0; c < nc; c++) {
             HIPCHK(hipEventSynchronize(ev[c % kBufs]));
-            ready.store(c + 1, std::memory_order_release);
+            ready.store(c + 1);
+            if (c == 0) start_team();
+            else tell();
             for (;;) {
                 if (mine == ~0u) {
                     if (next.load(std::memory_order_relaxed) >= (c + 1) * kSlices) break;

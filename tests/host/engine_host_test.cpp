@@ -18,7 +18,7 @@ namespace {
         }                                                                                   \
     } while (0)
 
-constexpr size_t kN = 512, kM = 40000;
+constexpr size_t kN = 512, kM = 80000;
 
 eimp_engine *engine() {
     static std::vector<uint64_t> site(kM * kN / 64, 0x5555555555555555ull);
@@ -192,6 +192,39 @@ void failed_copy_leaves_nothing_in_flight(int) {
     eimp_engine_destroy(e);
 }
 
+// The threads that move chunks on do not run while the device has not filled
+// them: five chunks, 60 ms each, are copied with far less processor time than
+// they take.
+void waiting_for_the_device_is_idle(int) {
+    eimp_engine *e = engine();
+    const Batch b({{80000, 512}});  // 10.2 MB of rows
+    auto s = shared_contexts(e, 1, 0);
+    submit(s[0], b);
+    wait(s[0], b);
+    const size_t Mp = 2 * (80000 / 4) + 1;
+    std::vector<uint32_t> rows(2 * Mp * row_stride(512, LAYOUT_GPU));
+    auto copy = [&] {
+        REQUIRE(eimp_stream_copy_target(s[0], 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, rows.data(),
+                                        nullptr) == EIMP_OK);
+    };
+    copy();  // makes the buffers and the threads, touches the rows
+    auto cpu_ms = [] { return 1e3 * (double)std::clock() / CLOCKS_PER_SEC; };
+    stub.gathers = 0;
+    stub.gather_us = 60000;
+    const auto t0 = std::chrono::steady_clock::now();
+    const double c0 = cpu_ms();
+    copy();
+    const double cpu = cpu_ms() - c0;
+    const double wall = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    std::fprintf(stderr, "%d chunks: %.1f ms, %.1f ms of processor time\n", stub.gathers.load(), wall, cpu);
+    REQUIRE(stub.gathers >= 4 && wall > 200);
+    REQUIRE(cpu < wall / 4);
+    stub.gather_us = 0;
+    check_copy(s[0], b, 0);
+    eimp_stream_destroy(s[0]);
+    eimp_engine_destroy(e);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -201,6 +234,7 @@ int main(int argc, char **argv) {
     else if (name == "shared_pool_threads") shared_pool_threads(rounds);
     else if (name == "shared_pool_without_graphs") shared_pool_without_graphs(rounds);
     else if (name == "failed_copy_leaves_nothing_in_flight") failed_copy_leaves_nothing_in_flight(rounds);
+    else if (name == "waiting_for_the_device_is_idle") waiting_for_the_device_is_idle(rounds);
     else return 2;
     std::printf("ok %s\n", name.c_str());
     return 0;

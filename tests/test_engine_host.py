@@ -45,3 +45,7 @@ def test_shared_pool_without_graphs(host):
 
 def test_failed_copy_leaves_nothing_in_flight(host):
     host("failed_copy_leaves_nothing_in_flight")
+
+
+def test_waiting_for_the_device_is_idle(host):
+    host("waiting_for_the_device_is_idle")
