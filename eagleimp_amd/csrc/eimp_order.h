@@ -644,10 +644,18 @@ __device__ __attribute__((noinline)) void order_chain(const TgtDev *tgt, OrderIt
 // Waves per SIMD that one workgroup's LDS allows at the variant's capacity: the
 // register budget is capped so that VGPRs do not lower it (512 x 20: three
 // workgroups, 80 registers; 8.65 ms for 384 chains of 941 blocks at K = 10,000
-// against 9.36 ms with two workgroups and 128 registers).
+// against 9.36 ms with two workgroups and 128 registers).  No fewer than five
+// waves, 96 registers: 1024 x 24 and 512 x 32 hold four waves per SIMD, which at
+// 128 registers are all there are, and nothing else then runs on a CU until its
+// chains end, not even the copies and the selection of another context (380 KB
+// copied beside 256 chains of 1,024 threads: up to 30 ms so, 2 ms with 96
+// registers; their build takes 66.6 ms either way.  The sizes above 12 positions
+// per thread spill a few registers more: two targets at K = 16,000 in 512 x 32
+// 3.27 and 3.42 ms, in 1024 x 24, which the automatic choice takes there, 2.66
+// and 2.64).
 constexpr int order_waves_hint(int NT, int CPW) {
     const int w = (163840 / (int)order_lds(NT, CPW)) * (NT / 256);
-    return w < 1 ? 1 : (w > 6 ? 6 : w);
+    return w < 5 ? 5 : (w > 6 ? 6 : w);
 }
 
 // positions per thread instantiated; a target uses the smallest that holds Kpad
