@@ -1504,13 +1504,16 @@ hipError_t raise_lds_limit(const void *fn, size_t lds) {
     return e;
 }
 
-// Pieces of device arrays into one pinned host buffer (grid x pieces, block
-// 256).  Bound by the link to the host; 16 bytes a thread keep its writes whole.
-__global__ __launch_bounds__(256) void k_gather(GatherArgs A, char *__restrict__ dst) {
+// Pieces of device arrays into one pinned host buffer (grid x pieces).  Bound by
+// the link to the host; 16 bytes a thread keep its writes whole.  One wave per
+// workgroup: it finds a place beside other contexts' kernels where four at once
+// would not.
+constexpr uint32_t GATHER_NT = 64;
+__global__ __launch_bounds__(GATHER_NT) void k_gather(GatherArgs A, char *__restrict__ dst) {
     const uint32_t i = blockIdx.y, bytes = A.bytes[i], n16 = bytes / 16;
     const gptr_t<const uint32_t> src = (gptr_t<const uint32_t>)(const uint32_t *)A.src[i];
     const gptr_t<uint32_t> out = (gptr_t<uint32_t>)(uint32_t *)(dst + A.off[i]);
-    for (uint32_t q = blockIdx.x * 256 + threadIdx.x; q < n16; q += gridDim.x * 256) {
+    for (uint32_t q = blockIdx.x * GATHER_NT + threadIdx.x; q < n16; q += gridDim.x * GATHER_NT) {
         // the arrays are aligned to their elements only
         const u32x4 v = u32x4{src[4 * q], src[4 * q + 1], src[4 * q + 2], src[4 * q + 3]};
         *(gptr_t<u32x4>)(out + 4 * q) = v;
@@ -1519,8 +1522,8 @@ __global__ __launch_bounds__(256) void k_gather(GatherArgs A, char *__restrict__
     if (blockIdx.x == 0 && tail < bytes / 4) out[tail] = src[tail];
 }
 hipError_t launch_gather(const GatherArgs &a, void *dst, size_t bytes, hipStream_t s) {
-    const uint32_t wgs = (uint32_t)std::min<size_t>((bytes + 4095) / 4096, 128);
-    hipLaunchKernelGGL(k_gather, dim3(std::max(wgs, 1u), a.n), dim3(256), 0, s, a, static_cast<char *>(dst));
+    const uint32_t wgs = (uint32_t)std::min<size_t>((bytes + 1023) / 1024, 512);
+    hipLaunchKernelGGL(k_gather, dim3(std::max(wgs, 1u), a.n), dim3(GATHER_NT), 0, s, a, static_cast<char *>(dst));
     return hipGetLastError();
 }
 hipError_t launch_site_to_hap(const PanelDev &P, uint64_t *hap, hipStream_t s) {

@@ -59,3 +59,10 @@ def test_beside_chains_on_every_cu(built):
     """Chains of 1,024 threads, one on every compute unit, few runs per block."""
     copy, build = longest_copy(60, 4)
     assert copy < 0.2 * build
+
+
+def test_beside_the_rows_of_all_blocks(built):
+    """Chains that leave room, and blocks of more than 1,087 runs (the rows
+    kernel for them fills the registers)."""
+    copy, build = longest_copy(400, 2)
+    assert copy < 0.1 * build
