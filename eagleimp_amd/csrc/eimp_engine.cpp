@@ -33,10 +33,12 @@ using namespace eimp;
 // code the name is only a stand-in: the device address of the current
 // device's copy comes from hipGetSymbolAddress (scratch_for_device) and only
 // that address is passed to kernels and copies.
-// kScratchBytes is what a batch's buffers may take; the PBWT's own tables come
-// from the extra part behind it: 26 bytes per block and direction (a block has
-// at least 128 bytes of condensed reference in the first part), the segments of
-// cut chains (at most kScratchSegs; their items are fewer bytes than they).
+// kScratchBytes is what a batch's data may take; tables, whose size follows from
+// it, come from the extra part behind it, which never fills first: per block of
+// the condensed reference (at least 128 bytes of the first part, so no more than
+// 524,288) 52 bytes of the PBWT's tables and a cref item, 36 MiB, the segments of
+// cut chains (kScratchSegs) and their items (a fifth of that), and the target
+// table twice.
 static constexpr size_t kScratchBytes = 64ull << 20;
 static constexpr size_t kScratchSegs = 16ull << 20;
 static constexpr size_t kScratchExtra = 64ull << 20;
@@ -585,9 +587,9 @@ uint32_t choose_segments(const std::vector<uint32_t> &nblk, const std::vector<ui
 // file-scope scratch array with caller-provided outputs
 // (eimp_engine_run_batch_noalloc).
 enum MemSlot : int {
-    MS_TG, MS_NERR, MS_BH, MS_BHF, MS_MONO, MS_SS, MS_SPL, MS_CMD, MS_STATS, MS_TLIST,
-    MS_CREF, MS_DIG, MS_CITEMS, MS_CROWS, MS_ORD, MS_BIG,
-    MS_OITEMS, MS_HDR, MS_RPREF, MS_RLIST, MS_SEG  // tables of the PBWT
+    MS_NERR, MS_BH, MS_BHF, MS_MONO, MS_SS, MS_SPL, MS_CMD, MS_STATS, MS_TLIST,
+    MS_CREF, MS_DIG, MS_CROWS, MS_ORD, MS_BIG,
+    MS_TG, MS_CITEMS, MS_OITEMS, MS_HDR, MS_RPREF, MS_RLIST, MS_SEG  // tables
 };
 struct BatchMem {
     virtual ~BatchMem() = default;
@@ -666,7 +668,7 @@ struct ScratchMem final : BatchMem {
         : base(reinterpret_cast<char *>(scr)), rows(rows_), c0(c0_), max_Mp(max_Mp_) {}
     int get(MemSlot s, size_t bytes, const char *what, void **p) override {
         const size_t b = round_up(std::max<size_t>(bytes, 1), 256);
-        if (s >= MS_OITEMS) {
+        if (s >= MS_TG) {
             if (used_extra + b > kScratchExtra)
                 return fail(EIMP_ERR_UNSUPPORTED, std::string("no-allocation scratch full (at ") + what + ")");
             *p = base + kScratchBytes + used_extra;

@@ -152,9 +152,9 @@ int eimp_engine_run_batch(eimp_engine *engine, size_t n, const eimp_target *targ
  * memory (rowstride as the layout flag chooses; Mp <= max_Mp, which the
  * caller sizes the buffers by).  Everything else (distances, best haps,
  * split data, condensed reference, tables) lives in a fixed device scratch
- * array, 64 MiB and as much again for the PBWT's tables, that every device
+ * array, 64 MiB and as much again for tables, that every device
  * running the library holds until the process ends; a batch needing more than
- * either part, more than 256 targets, or an Mp above
+ * 64 MiB for its data, more than 256 targets, or an Mp above
  * max_Mp fails with EIMP_ERR_UNSUPPORTED.  The panel parts a batch reads must
  * be resident already: the mono bits are built by
  * eimp_engine_set_panel_extras, the hap-major rows (targets with K < Ncorr or
