@@ -2,8 +2,8 @@
 (threads per workgroup x positions per thread, which fixes the workgroup's LDS and
 so the resident workgroups per CU) and the targets per submission, by timing
 a sample batch of the actual workload through timed contexts (HIP events
-between the kernel classes).  Results are cached per panel shape, K range,
-window range and candidate set.
+between the kernel classes).  Results are cached per build of the library,
+panel shape, K range, window range and candidate set.
 
     from eagleimp_amd.tune import tune
     best = tune(eng, targets, sample_idx)   # sets eng's PBWT variant
@@ -17,14 +17,16 @@ import time
 
 import numpy as np
 
-from .engine import Engine, pbwt_variants
+from .engine import LIB_PATH, Engine, pbwt_variants
 
 CACHE = os.environ.get("EIMP_TUNE_CACHE",
                        os.path.join(os.path.expanduser("~"), ".cache", "eagleimp_amd", "tune.json"))
 
 
 def _key(eng: Engine, Kmax: int, Wmax: int, batches, variants) -> str:
-    sig = json.dumps([eng.Nad, eng.Ncorr, eng.M, Kmax, Wmax, list(batches),
+    with open(LIB_PATH, "rb") as f:  # the timings are those of its kernels
+        build = hashlib.sha1(f.read()).hexdigest()
+    sig = json.dumps([build, eng.Nad, eng.Ncorr, eng.M, Kmax, Wmax, list(batches),
                       [(v["threads"], v["chunks_per_wave"]) for v in variants]])
     return hashlib.sha1(sig.encode()).hexdigest()[:16]
 
