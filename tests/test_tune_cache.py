@@ -27,3 +27,18 @@ def test_choice_of_other_kernels_is_not_taken(tmp_path, monkeypatch):
     other.write_bytes(b"another build")
     monkeypatch.setattr(tune, "LIB_PATH", str(other))
     assert not tune.tune(_Engine(), tg, range(300), batches=batches)["cached"]
+
+
+def test_automatic_stays_on_where_it_starts_from_the_choice(tmp_path, monkeypatch):
+    """The automatic choice starts from the smallest shape that holds K (2 at
+    K = 10,000) and takes one with more threads for few targets: a tuned engine
+    keeps that where the tuner picks the same shape, from the cache too."""
+    monkeypatch.setattr(tune, "CACHE", str(tmp_path / "tune.json"))
+    tg = _Targets(300, 10000)
+    for per, variant, on in (({2: 1.0, 3: 2.0}, 2, -1), ({2: 2.0, 4: 1.0}, 4, 4)):
+        for use_cache in (False, True, True):
+            eng = _Engine(per=per)
+            best = tune.tune(eng, tg, range(300), batches=(128, 256) if on < 0 else (256,),
+                             use_cache=use_cache)
+            assert best["variant"] == variant and eng.variant == on
+        assert best["cached"]
