@@ -225,6 +225,25 @@ void waiting_for_the_device_is_idle(int) {
     eimp_engine_destroy(e);
 }
 
+// The chains of targets with these row counts at this K are all cut, from one
+// workgroup on a compute unit to eight.
+void cut(int argc, char **argv) {
+    std::vector<uint32_t> nblk, Kpad;
+    for (int i = 3; i < argc; i++) {
+        nblk.push_back(((uint32_t)std::atoi(argv[i]) + 15) / 16);
+        Kpad.push_back((uint32_t)round_up(std::atoi(argv[2]), 64));
+    }
+    REQUIRE(!nblk.empty());
+    for (uint32_t occ = 1; occ <= 8; occ++) {
+        bool latency = false;
+        const uint32_t L = choose_segments(nblk, Kpad, 256 * (10 + 2 * (occ - 1)), kSegBytes / 2, ~0u, 256, &latency);
+        for (uint32_t nb : nblk) {
+            uint32_t len = 0;
+            REQUIRE(seg_split(nb, L, len) >= 3);
+        }
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -235,6 +254,7 @@ int main(int argc, char **argv) {
     else if (name == "shared_pool_without_graphs") shared_pool_without_graphs(rounds);
     else if (name == "failed_copy_leaves_nothing_in_flight") failed_copy_leaves_nothing_in_flight(rounds);
     else if (name == "waiting_for_the_device_is_idle") waiting_for_the_device_is_idle(rounds);
+    else if (name == "cut") cut(argc, argv);
     else return 2;
     std::printf("ok %s\n", name.c_str());
     return 0;
