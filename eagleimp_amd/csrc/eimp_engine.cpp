@@ -326,7 +326,7 @@ struct HostCopier {
         for (auto &d : done) d.store(0, std::memory_order_relaxed);
         ready.store(0);
         auto launch = [&](uint32_t c) {
-            return launch_gather(chunks[c].args, buf.as<char>() + (c % kBufs) * kChunk, chunks[c].bytes, s);
+            return launch_gather(chunks[c].args, buf.as<char>() + (c % kBufs) * kChunk, s);
         };
         if (nc == 1) {
             HIPCHK(launch(0));

@@ -1521,8 +1521,10 @@ __global__ __launch_bounds__(GATHER_NT) void k_gather(GatherArgs A, char *__rest
     const uint32_t tail = 4 * n16 + threadIdx.x;
     if (blockIdx.x == 0 && tail < bytes / 4) out[tail] = src[tail];
 }
-hipError_t launch_gather(const GatherArgs &a, void *dst, size_t bytes, hipStream_t s) {
-    const uint32_t wgs = (uint32_t)std::min<size_t>((bytes + 1023) / 1024, 512);
+hipError_t launch_gather(const GatherArgs &a, void *dst, hipStream_t s) {
+    uint32_t most = 0;
+    for (uint32_t i = 0; i < a.n; i++) most = std::max(most, a.bytes[i]);
+    const uint32_t wgs = std::min((most + 1023) / 1024, 512u);
     hipLaunchKernelGGL(k_gather, dim3(std::max(wgs, 1u), a.n), dim3(GATHER_NT), 0, s, a, static_cast<char *>(dst));
     return hipGetLastError();
 }

@@ -16,8 +16,8 @@ struct GatherArgs {
     uint32_t off[kGatherPieces], bytes[kGatherPieces];
     uint32_t n;
 };
-// dst: pinned host memory as the device sees it; bytes: the end of the last piece
-hipError_t launch_gather(const GatherArgs &a, void *dst, size_t bytes, hipStream_t s);
+// dst: pinned host memory as the device sees it
+hipError_t launch_gather(const GatherArgs &a, void *dst, hipStream_t s);
 
 hipError_t launch_site_to_hap(const PanelDev &P, uint64_t *hap, hipStream_t s);
 hipError_t launch_panel_mono(const PanelDev &P, uint64_t *pand, uint64_t *por, hipStream_t s);

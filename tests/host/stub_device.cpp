@@ -282,7 +282,7 @@ void fill(const TgtDev &T) {
     for (uint32_t r = 0; r < T.Mp; r++) T.count0[r] = (int32_t)(r ^ T.W);
 }
 }  // namespace
-hipError_t launch_gather(const GatherArgs &a, void *dst, size_t, hipStream_t s) {
+hipError_t launch_gather(const GatherArgs &a, void *dst, hipStream_t s) {
     if (stub.fail_gather >= 0 && stub.gathers == stub.fail_gather) return hipErrorLaunchFailure;
     stub.gathers++;
     st(s)->push([=] {
