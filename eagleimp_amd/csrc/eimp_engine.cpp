@@ -152,10 +152,9 @@ struct HostBuf {
 // Here the arrays are one byte stream, cut into chunks that a kernel gathers
 // into pinned buffers (k_gather: one launch per chunk, however many arrays it
 // holds), several chunks ahead of the host, and from two chunks on a small team
-// of threads copies the slices of the chunks that have arrived.  The team is
-// woken when the first chunk has arrived, and a thread that waits for a later one
-// for more than kSpin sleeps: the work before the copy, or another context's
-// kernels beside it, can take far longer than the copy.  Whole calls,
+// of threads copies the slices of the chunks that have arrived.  One that waits
+// for a chunk for more than kSpin sleeps: the work before the copy, or another
+// context's kernels beside it, can take far longer than the copy.  Whole calls,
 // before and now: three targets of 256 haplotypes with all their arrays 692 and
 // 444 us; one target with 15 MB of rows 3,069 and 1,843 us; 12 targets with
 // 92 MB 6,003 and 2,671 us; 30 MB of panel orders 2,650 and 1,672 us.
@@ -260,8 +259,8 @@ struct HostCopier {
         { std::lock_guard<std::mutex> lk(tm); }
         arrived.notify_all();
     }
-    // the team as it is (device work under way meanwhile), then its start
-    void gather_team() {
+    // (made, the first time, while the device works on the first chunks)
+    void start_team() {
         while (team.size() < kThreads && !no_team) {
             try {
                 team.emplace_back([this] { work(); });
@@ -269,8 +268,6 @@ struct HostCopier {
                 no_team = true;  // the caller alone, with the threads there are
             }
         }
-    }
-    void start_team() {
         active.store((uint32_t)team.size(), std::memory_order_relaxed);
         {
             std::lock_guard<std::mutex> lk(tm);
@@ -355,13 +352,12 @@ struct HostCopier {
             return (int)EIMP_OK;
         };
         for (uint32_t c = 0; c < std::min<uint32_t>(nc, kBufs); c++) CHK(go(c));
-        gather_team();
+        start_team();
         uint32_t mine = ~0u;  // a ticket of a chunk that has not arrived
         for (uint32_t c = 0; c < nc; c++) {
             HIPCHK(hipEventSynchronize(ev[c % kBufs]));
             ready.store(c + 1);
-            if (c == 0) start_team();
-            else tell();
+            tell();
             for (;;) {
                 if (mine == ~0u) {
                     if (next.load(std::memory_order_relaxed) >= (c + 1) * kSlices) break;
