@@ -19,7 +19,7 @@
 // Carrying every haplotype through every row (two barriers and 5 vector
 // instructions per 64 haplotypes and row, one workgroup per chain for all
 // rows) took 32.3 ms for 192 targets of 15,000 rows at K = 10,000; the chain
-// now takes 9.0 ms and the rows 6.1 ms.  One target of 45,000 rows:
+// now takes 9.1 ms and the rows 5.6 ms.  One target of 45,000 rows:
 // 61.3 and 2.8 ms for the whole call (its chain cut into segments).
 //
 // Blocks with more runs than k_rows takes and the last block of a target when
@@ -59,8 +59,8 @@ namespace {
 // instead of the length, neighbours with equal remaining bits merged row by row,
 // took 28: the merging (2,400 entries of a block become 1,700 by its twelfth
 // row) cost more than it saved.  96 targets on the 200,000-haplotype panel
-// (2,750 runs a block): 8,106 us so, 5,232 us now; 192 whole-panel targets at
-// K = 10,000 (1,050 runs): 6,757 and 5,950 us; 256 windows: 12.3 and 10.8 ms.
+// (2,750 runs a block): 8,106 us so, 5,021 us now; 192 whole-panel targets at
+// K = 10,000 (1,050 runs): 6,757 and 5,630 us; 256 windows: 12.3 and 9.8 ms.
 // ---------------------------------------------------------------------------
 // Lanes entered inside a run of ones, from what every lane does with that
 // state: f0 / f1 = lanes left inside a run when entered outside / inside one.
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(BIG_NT) void k_pbwt_big(const BigItem *__restrict__
         if (I.absperm && q < K) gmem(I.absperm)[q] = (int32_t)q;
     }
     {
-        // the padding words of every row, stored once (as pbwt_steps)
+        // the padding words of every row, stored once
         const uint32_t pw0 = I.raw ? 2 * nch : 2 * npairs;
         const uint32_t fw = I.raw ? ~0u : 0u;
         for (uint32_t rr = tid; rr < Mp; rr += BIG_NT) {

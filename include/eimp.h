@@ -191,7 +191,7 @@ int eimp_engine_copy_monos(eimp_engine *engine, size_t t, uint64_t *monos);
  * (data / cumulative zero pairs, 1-padding), count0 nsites int32, and absperm,
  * if not NULL, (nsites+1) x N int32 absolute orders (row m = order before site
  * m0+m; getSortOrder, src/PBWT.h:78).  device_ms (NULL or 1 double): device
- * time.  N up to 24,576 (one workgroup carries the order). */
+ * time.  N up to 524,288 (above 24,576 the order is carried in global memory). */
 int eimp_engine_ref_pbwt(eimp_engine *engine, size_t m0, size_t nsites, uint32_t *rows,
                          int32_t *count0, int32_t *absperm, double *device_ms);
 
