@@ -369,8 +369,8 @@ class Stream:
     def __init__(self, eng: Engine, max_targets, max_window, max_K, pool_bytes, digest=True,
                  compact=False, graph=True, timed=False, raw=False, share=None):
         """share: another Stream whose output pool this one uses (pool_bytes
-        is then ignored, and both launch their kernels one by one); their builds take turns, each preparation runs
-        beside the other's build."""
+        is then ignored, and both launch their kernels one by one); their
+        builds take turns, each preparation runs beside the other's build."""
         self.eng = eng
         self._h = _P()
         self.layout = layout_name(compact, raw)

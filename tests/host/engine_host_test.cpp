@@ -244,6 +244,36 @@ void cut(int argc, char **argv) {
     }
 }
 
+// Several arrays in one copy, as the drop-in call has: ends on, before and behind
+// the edges of chunks, of the four buffers and of the pieces that a chunk holds.
+void arrays_at_chunk_edges(int) {
+    HostCopier c;
+    hipStream_t s = nullptr;
+    REQUIRE(hipStreamCreateWithFlags(&s, 0) == hipSuccess);
+    constexpr size_t C = HostCopier::kChunk;
+    const std::vector<std::vector<size_t>> sets = {
+        {C}, {C - 4}, {C + 4}, {C, C}, {C - 16, 16, C}, {C - 16, 4, 4}, {C - 4, 4, 4}, {4 * C, 4}, {4 * C - 8, C + 8, 12},
+        {8 * C + 4, 0, C - 4}, std::vector<size_t>(kGatherPieces, 20), std::vector<size_t>(kGatherPieces + 1, 20),
+        std::vector<size_t>(3 * kGatherPieces + 2, C / kGatherPieces / 4 * 4)};
+    for (const auto &set : sets) {
+        std::vector<std::vector<uint32_t>> src, dst;
+        std::vector<HostCopier::Job> jobs;
+        for (size_t b : set) {
+            src.emplace_back(b / 4 + 1);
+            for (size_t i = 0; i < src.back().size(); i++) src.back()[i] = (uint32_t)((i + b) * 2654435761u + src.size());
+            dst.emplace_back(b / 4 + 1, 7u);
+        }
+        for (size_t i = 0; i < set.size(); i++) jobs.push_back({dst[i].data(), src[i].data(), set[i]});
+        REQUIRE(c.run(jobs, s) == EIMP_OK);
+        for (size_t i = 0; i < set.size(); i++) {
+            REQUIRE(std::equal(dst[i].begin(), dst[i].end() - 1, src[i].begin()));
+            REQUIRE(dst[i].back() == 7u);
+        }
+    }
+    c.release();
+    (void)hipStreamDestroy(s);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -255,6 +285,7 @@ int main(int argc, char **argv) {
     else if (name == "failed_copy_leaves_nothing_in_flight") failed_copy_leaves_nothing_in_flight(rounds);
     else if (name == "waiting_for_the_device_is_idle") waiting_for_the_device_is_idle(rounds);
     else if (name == "cut") cut(argc, argv);
+    else if (name == "arrays_at_chunk_edges") arrays_at_chunk_edges(rounds);
     else return 2;
     std::printf("ok %s\n", name.c_str());
     return 0;

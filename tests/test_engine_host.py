@@ -49,3 +49,7 @@ def test_failed_copy_leaves_nothing_in_flight(host):
 
 def test_waiting_for_the_device_is_idle(host):
     host("waiting_for_the_device_is_idle")
+
+
+def test_arrays_at_chunk_edges(host):
+    host("arrays_at_chunk_edges")
