@@ -653,7 +653,7 @@ __device__ __attribute__((noinline)) void order_chain(const TgtDev *tgt, OrderIt
 // per thread spill a few registers more: two targets at K = 16,000 in 512 x 32
 // 3.27 and 3.42 ms, in 1024 x 24, which the automatic choice takes there, 2.66
 // and 2.64; one target of 45,000 rows at K = 10,000, 10 positions per thread,
-// 2.77 and 2.79.
+// 2.77 and 2.79).
 constexpr int order_waves_hint(int NT, int CPW) {
     const int w = (163840 / (int)order_lds(NT, CPW)) * (NT / 256);
     return w < 5 ? 5 : (w > 6 ? 6 : w);
